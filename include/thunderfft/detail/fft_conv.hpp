@@ -1118,236 +1118,3 @@ __global__ __launch_bounds__(256) void conv1d_real_kernel(
 }
 
 }  // namespace thff
-
-namespace thff {
-
-// ---------------------------------------------------------------------------
-// Tiled valid 1-D correlation with 64-point FFTs (overlap-save), the
-// reference's conv1d_direct_fft_kernel (sample/conv1d/main.cu:38-128):
-//   y[b][i] = sum_{k < F} x[b][i + k] * f[k],   i < L - F + 1,  1 <= F <= 64,
-// complex x, f, no conjugation.  Window w of a signal is x[w*V .. w*V + 63]
-// with V = 65 - F; its circular convolution with g[m] = f[(64 - m) mod 64] / 64
-// (the reversed filter, main.cu:145-154) equals y[w*V + j] for j < V, since
-// those outputs never wrap.  Each wave owns 16 consecutive windows: it stages
-// their input span (15 V + 64 <= 1024 values) in its own LDS region, gathers
-// every window into its transform slot's registers, runs FFT * G * IFFT and
-// writes the V valid outputs of each window back contiguously.  Nothing
-// crosses waves, so the kernel has no workgroup barrier after its set-up:
-// every workgroup transforms the filter once (fp32 taps) into a 64-value LDS
-// table G, then walks groups of 64 windows (one per transform slot) with
-// tile_walk: groups_per_block consecutive groups, or 0 for grid-stride over a
-// device-sized grid.
-// Inputs past the end of a signal read as zero; no valid output uses them.
-// Spans and output runs start at multiples of 16 values of their signal, so
-// signals that start on a 16-byte boundary move as whole 16-byte vectors
-// (one partial vector at a signal's end); others value by value.
-// float2: the next group's span is loaded into registers while the current
-// one is transformed (when every signal starts on a 16-byte boundary), at 2
-// waves per SIMD: 2^26 values, 9 taps, 232 us against 261 us without.  The
-// library runs half2 on conv1d_valid_mfma_kernel (fft_conv_mfma.hpp:
-// 256-point windows on MFMA, 112 us against 162 us for this kernel in half2,
-// which keeps 3 waves per SIMD and no prefetch).
-// ---------------------------------------------------------------------------
-template <class IO>
-inline constexpr bool kValidPrefetch = std::is_same_v<IO, float2>;
-template <class IO>
-inline constexpr int kValidMinWavesPerEU = kValidPrefetch<IO> ? 2 : 3;
-
-// kExact: the 64-point passes use exact per-lane twiddles (LaneTwiddles64Exact,
-// 610 instead of 666 VALU instructions per window group, 243 VGPRs): float2
-// only, which already runs at 2 waves per SIMD; 227 vs 233 us at 2^26 values.
-template <class IO, bool kExact = kValidPrefetch<IO>>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kValidMinWavesPerEU<IO>))) void conv1d_valid_kernel(
-    const IO* __restrict__ x, const float2* __restrict__ taps, IO* __restrict__ y,
-    long long len, int ntaps, int batch, const float2* __restrict__ tw, int groups_per_block) {
-    using P = C2CPlan<64>;
-    using I = Io<IO>;
-    using W1 = typename I::W1;
-    using W4 = typename I::W4;
-    constexpr int kVec = I::kVec;      // complex values per 16-byte vector
-    constexpr int kWindowsPerWave = 16;
-    constexpr int kSpan = 1024;        // values staged per wave, >= 15 V + 64 and >= 16 V
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int t = tid & 3;             // lane within its window's transform
-    const int fl = (tid >> 2) & 15;    // window within the wave
-    __shared__ __align__(16) cpx lds[P::kLdsSlots];
-    __shared__ cpx spectrum[64];  // G, natural order
-    cpx* const region = lds + wave * kWindowsPerWave * P::kSlot;  // 16 slots = 1088 >= kSpan
-    cpx* const slot = region + fl * P::kSlot;
-
-    std::conditional_t<kExact, LaneTwiddles64Exact, LaneTwiddles<64>> w;
-    w.load(t, tw);
-
-    const int V = 65 - ntaps;                            // valid outputs per window
-    const unsigned rcpV = (65536u + V - 1) / V;          // e / V == (e * rcpV) >> 16 for e < 1024
-    const long long out_len = len - ntaps + 1;
-    const long long windows = (out_len + V - 1) / V;     // per signal
-    const long long groups_per_signal = (windows + P::kFPB - 1) / P::kFPB;
-    const long long groups = groups_per_signal * batch;
-    const bool x16 = (reinterpret_cast<unsigned long long>(x) & 15) == 0;
-    const bool y16 = (reinterpret_cast<unsigned long long>(y) & 15) == 0;
-
-    // G = FFT(g), g[m] = f[(64 - m) mod 64] / 64, m = t + 4 j, computed by
-    // every slot and published once by the first slot.
-    {
-        cpx G[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int m = t + 4 * j;
-            const int k = m == 0 ? 0 : 64 - m;
-            const float2 c = k < ntaps ? taps[k] : make_float2(0.f, 0.f);
-            G[j] = {c.x * (1.0f / 64), c.y * (1.0f / 64)};
-        }
-        fft_registers<64, true>(G, slot, t, w);
-        if (tid < 4)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) spectrum[t + 4 * j] = G[j];
-        __syncthreads();
-    }
-
-    long long g, g_end, step;
-    tile_walk(groups, groups_per_block, g, g_end, step);
-    // A wave's 16 windows read 15 V + 64 values of its span; nothing past
-    // that is loaded (it is the next wave's, which may run on another XCD).
-    const int need = 15 * V + 64;
-    // The span of group gg (this wave's windows) as 16-byte vectors, zero past
-    // the signal's end; for signals that start on a 16-byte boundary.
-    constexpr int kLoads = kSpan / (64 * kVec);
-    // Signal and group within it of the walk's groups, advanced per step.
-    const DivWalk walk(step, groups_per_signal);
-    DivPos pos = walk.at(g);
-    auto span_load = [&](DivPos gp, W4 (&r)[kLoads]) {
-        const long long bb = gp.q;
-        const long long s0 = (gp.r * P::kFPB + wave * kWindowsPerWave) * V;
-        const long long av = len - s0 < need ? len - s0 : need;
-        const IO* sp = x + bb * len + s0;
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int e = kVec * (lane + 64 * i);
-            if (s0 < out_len && e + kVec <= av) {
-                r[i] = ld_nt(reinterpret_cast<const W4*>(sp + e));
-            } else {
-                W4 z{};
-                if (s0 < out_len)
-#pragma unroll
-                    for (int c = 0; c < kVec; ++c)
-                        if (e + c < av)
-                            reinterpret_cast<W1*>(&z)[c] = *reinterpret_cast<const W1*>(sp + e + c);
-                r[i] = z;
-            }
-        }
-    };
-    // Prefetch only when every signal starts on a 16-byte boundary.
-    const bool prefetch = kValidPrefetch<IO> && x16 && len % kVec == 0;
-    W4 next[kLoads];
-    if (prefetch && g < g_end) span_load(pos, next);
-    // A wave's issue priority falls as its workgroup gets ahead of the others
-    // (ProgressPriority): 223.5 against 227.3-227.5 us for 2^26 values (the
-    // fp16 MFMA valid kernel measured 1.5% slower with it and does not use it).
-    long long left = (g_end - g + step - 1) / step;
-    const ProgressPriority priority(left);
-    for (; g < g_end; g += step, --left) {
-        priority.set(left);
-        const long long b = pos.q;
-        // This wave's first window, and where its input span and its outputs
-        // start in signal b (both w0 * V, a multiple of 16 values).
-        const long long w0 = pos.r * P::kFPB + wave * kWindowsPerWave;
-        const long long span0 = w0 * V;
-        pos = walk.advance(pos);
-        W4 cur[kLoads];
-        if (prefetch) {
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i) cur[i] = next[i];
-            if (g + step < g_end) span_load(pos, next);
-        }
-        if (span0 >= out_len) continue;  // no window of this wave has an output
-        const long long avail = len - span0 < need ? len - span0 : need;  // > 0
-        const IO* src = x + b * len + span0;
-        // Whole 16-byte vectors when the signal starts on one (always for b = 0).
-        const bool in_vec = x16 && (b * len) % kVec == 0;
-        const bool out_vec = y16 && (b * out_len) % kVec == 0;
-
-        wave_lds_sync();  // the previous group's reads of the region are done
-        if (prefetch) {
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i) {
-                const int e = kVec * (lane + 64 * i);
-                cpx q[kVec];
-                I::decode4(cur[i], q);
-#pragma unroll
-                for (int c = 0; c < kVec; ++c) region[e + c] = q[c];
-            }
-        } else if (in_vec) {
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i) {
-                const int e = kVec * (lane + 64 * i);
-                cpx q[kVec];
-                if (e + kVec <= avail) {
-                    I::decode4(*reinterpret_cast<const W4*>(src + e), q);
-                } else {
-#pragma unroll
-                    for (int c = 0; c < kVec; ++c)
-                        q[c] = e + c < avail ? I::decode1(*reinterpret_cast<const W1*>(src + e + c))
-                                             : cpx{0.f, 0.f};
-                }
-#pragma unroll
-                for (int c = 0; c < kVec; ++c) region[e + c] = q[c];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < kSpan / 64; ++i) {
-                const int e = lane + 64 * i;
-                region[e] = e < avail ? I::decode1(*reinterpret_cast<const W1*>(src + e))
-                                      : cpx{0.f, 0.f};
-            }
-        }
-        wave_lds_sync();
-        cpx v[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) v[j] = region[fl * V + t + 4 * j];
-        wave_lds_sync();  // the gather is done before the transform reuses the region
-
-        fft_registers<64, true>(v, slot, t, w);
-#pragma unroll
-        for (int j = 0; j < 16; ++j) v[j] = cmul(v[j], spectrum[t + 4 * j]);
-        fft_registers<64, false>(v, slot, t, w);
-
-        wave_lds_sync();
-#pragma unroll
-        for (int j = 0; j < 16; ++j) slot[lds_pad(t + 4 * j)] = v[j];
-        wave_lds_sync();
-        // Output e of the wave (e < 16 V) is element e mod V of window e / V.
-        const long long left = out_len - span0;
-        const int count = left < kWindowsPerWave * V ? static_cast<int>(left) : kWindowsPerWave * V;
-        IO* dst = y + b * out_len + span0;
-        auto value = [&](int e) {
-            const int q = static_cast<int>((static_cast<unsigned>(e) * rcpV) >> 16);
-            return region[q * P::kSlot + lds_pad(e - q * V)];
-        };
-        if (out_vec) {
-#pragma unroll 1
-            for (int i = 0; i < kSpan / (64 * kVec); ++i) {
-                const int e = kVec * (lane + 64 * i);
-                if (e + kVec <= count) {
-                    cpx q[kVec];
-#pragma unroll
-                    for (int c = 0; c < kVec; ++c) q[c] = value(e + c);
-                    st_nt(reinterpret_cast<W4*>(dst + e), I::encode4(q));
-                } else {
-#pragma unroll
-                    for (int c = 0; c < kVec; ++c)
-                        if (e + c < count)
-                            *reinterpret_cast<W1*>(dst + e + c) = I::encode1(value(e + c));
-                }
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < kSpan / 64; ++i) {
-                const int e = lane + 64 * i;
-                if (e < count) *reinterpret_cast<W1*>(dst + e) = I::encode1(value(e));
-            }
-        }
-    }
-}
-
-}  // namespace thff

@@ -206,56 +206,6 @@ __device__ __forceinline__ void fft_registers(cpx (&v)[16], Slot slot, int t,
         for (int m = 0; m < kRL; ++m) v[q + m * (16 / kRL)] = o[q * kRL + m];
 }
 
-// N = 64 with exact per-lane twiddles: the radix-4 pass multiplies input j of
-// butterfly t + 4q by W_64^(j (t + 4 q)), all 12 of them kept in registers
-// (24 VGPRs), instead of a base factor W_64^(j t) times a compile-time W_16^(j q)
-// rotation: 32 fewer VALU instructions per transform.  Same LDS exchange and
-// register order as fft_registers<64>.
-struct LaneTwiddles64Exact {
-    cpx e[4][3];  // e[q][j - 1] = W_64^(j (t + 4 q)), positive angle
-    __device__ __forceinline__ void load(int t, const float2* __restrict__ tw) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int j = 1; j < 4; ++j) {
-                const float2 x = tw[(j * (t + 4 * q)) & 63];
-                e[q][j - 1] = cpx{x.x, x.y};
-            }
-    }
-};
-
-template <int N, bool FWD>
-__device__ __forceinline__ void fft_registers(cpx (&v)[16], cpx* slot, int t,
-                                              const LaneTwiddles64Exact& w) {
-    static_assert(N == 64, "exact lane twiddles: N = 64");
-    using P = C2CPlan<64>;
-    Dft<16, FWD>::run(v);
-    // the radix-16 outputs of butterfly t go to 16 t + m
-    region_sync<P::kWaveLocal>();
-#pragma unroll
-    for (int m = 0; m < 16; ++m) slot[lds_pad(16 * t + m)] = v[m];
-    region_sync<P::kWaveLocal>();
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int b = t + 4 * q;
-        v[4 * q] = slot[lds_pad(b)];
-#pragma unroll
-        for (int j = 1; j < 4; ++j) {
-            const cpx x = slot[lds_pad(b + 16 * j)];
-            v[4 * q + j] = FWD ? cmulc(x, w.e[q][j - 1]) : cmul(x, w.e[q][j - 1]);
-        }
-        Dft<4, FWD>::run(v + 4 * q);
-    }
-    // output m of butterfly t + 4q is X[t + 4 (q + 4 m)]
-    cpx o[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[i] = v[i];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int m = 0; m < 4; ++m) v[q + 4 * m] = o[4 * q + m];
-}
-
 // Raw per-lane data of one tile as loaded from global memory: 16/kVec
 // 16-byte vectors of kVec consecutive complex values.  Lane l of wave w
 // holds tile elements 1024*w + kVec*l + 64*kVec*i, i < 16/kVec.

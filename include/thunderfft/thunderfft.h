@@ -143,9 +143,10 @@ int thff_conv1d_real(int precision, int n, const void* d_x, const void* d_spectr
 int thff_conv1d_real_async(int precision, int n, const void* d_x, const void* d_spectrum,
                            void* d_y, int batch, int channels, void* stream);
 
-/* Tiled valid 1-D correlation with 64-point FFT windows (overlap-save), the
- * reference's conv1d_direct_fft_kernel (sample/conv1d/main.cu:38-128, driven
- * by main :207-336 with the definition of :156-174):
+/* Valid 1-D correlation with a short filter, the result of the reference's
+ * conv1d_direct_fft_kernel (sample/conv1d/main.cu:38-128, driven by main
+ * :207-336 with the definition of :156-174), which tiles it in 64-point FFT
+ * windows; here the sum itself, on the matrix cores:
  *   y[b][i] = sum_{k < filter_len} x[b][i + k] * taps[k],  i < input_len - filter_len + 1,
  * complex, no conjugation.  x holds batch signals of input_len values and y
  * batch outputs of input_len - filter_len + 1 values, both in `precision`
@@ -153,8 +154,8 @@ int thff_conv1d_real_async(int precision, int n, const void* d_x, const void* d_
  * precisions.  1 <= filter_len <= 64 and input_len >= filter_len (the
  * sample's checks, main.cu:223-230), THFF_EINVAL otherwise; batch < 0, null,
  * aliased or misaligned pointers are THFF_EINVAL, batch = 0 is a no-op.
- * Requires thff_initialize(precision, 64) (the windows are 64-point
- * transforms).  Synchronises `stream` before returning. */
+ * Requires thff_initialize(precision, 64), as the reference's windows do.
+ * Synchronises `stream` before returning. */
 int thff_conv1d_valid(int precision, const void* d_x, long long input_len, const void* d_taps,
                       int filter_len, void* d_y, int batch, void* stream);
 

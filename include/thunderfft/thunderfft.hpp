@@ -138,9 +138,9 @@ inline void ThunderFFT_conv1d_real(const T* d_x, const float2* d_spectrum, T* d_
                                    channels, static_cast<void*>(stream)));
 }
 
-// Tiled valid 1-D correlation y[b][i] = sum_k x[b][i + k] * taps[k] of `batch`
-// signals of input_len values with 1 <= filter_len <= 64 fp32 complex taps,
-// through 64-point FFT windows (the reference's sample/conv1d/main.cu:38-174).
+// Valid 1-D correlation y[b][i] = sum_k x[b][i + k] * taps[k] of `batch`
+// signals of input_len values with 1 <= filter_len <= 64 fp32 complex taps
+// (the reference's sample/conv1d/main.cu:38-174).
 // y holds batch * (input_len - filter_len + 1) values; Initialize<T>(64) first.
 template <typename T>
 inline void ThunderFFT_conv1d_valid(const vec2_t<T>* d_x, long long input_len,

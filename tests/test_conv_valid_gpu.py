@@ -187,3 +187,34 @@ def test_signal_beyond_2e31_values(T):
         assert ok, (T, lo, hi)
     del d_x, d_y
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("T", ["float", "half"])
+def test_span_edges_and_tap_scales(T):
+    """Outputs one below, at and above whole spans (512 float, 1024 half, four
+    waves each) and filters one below, at and above a step of the matrix, with
+    taps of any size.  Per output, S = sum |x||taps|:
+      float: 4 chains of F/2 products and their sum, (F/2 + 4) 2^-23 S;
+      half: taps to 2^-21 of the largest, the same sums, one rounding to f16
+      (2^-11 of the result, 2^-24 at least)."""
+    rng = np.random.default_rng(512)
+    span = 512 if T == "float" else 1024
+    for ntaps in (1, 2, 8, 9, 10, 17, 18, 41, 42, 49, 50, 57, 58, 64):
+        for out, batch in ((1, 5), (span - 1, 2), (span, 1), (span + 1, 3), (4 * span + 1, 1)):
+            for scale in (1.0, 2.0 ** -12, 2.0 ** 9):
+                length = out + ntaps - 1
+                x = rng.uniform(-1, 1, (batch, length)) + 1j * rng.uniform(-1, 1, (batch, length))
+                f = rng.normal(size=ntaps) + 1j * rng.normal(size=ntaps)
+                f = (f * scale * 2.0 ** rng.integers(-6, 1, ntaps)).astype(np.complex64)
+                xr = oracle.represent(x.astype(np.complex64), T)
+                y, guards = run(T, xr, f, batch)
+                want = np.asarray(oracle.conv1d_valid(xr, f)).reshape(batch, out)
+                size = np.stack([np.convolve(np.abs(r.astype(np.complex128)), np.abs(f)[::-1], "valid")
+                                 for r in xr])
+                if T == "float":
+                    bound = (ntaps / 2 + 4) * 2.0 ** -23 * size
+                else:
+                    bound = ((ntaps / 2 + 4) * 2.0 ** -23 * size + 2.0 ** -11 * np.abs(want) + 2.0 ** -24
+                             + 2.0 ** -21 * np.abs(f).max() * np.abs(xr).max() * ntaps)
+                worst = float(np.max(np.abs(y - want) / bound))
+                assert guards == 0 and worst <= 1.0, (T, ntaps, out, batch, scale, worst)

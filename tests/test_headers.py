@@ -11,7 +11,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADERS = ["thunderfft/thunderfft.h", "thunderfft/thunderfft.hpp", "thunderfft/thunderfft.cuh",
            "thunderfft/thunderfft_device.hpp"] + [
     f"thunderfft/detail/{h}" for h in ("fft_core.hpp", "fft_tile.hpp", "fft_c2c.hpp",
-                                      "fft_conv.hpp", "fft_mfma.hpp", "fft_conv_mfma.hpp")]
+                                      "fft_conv.hpp", "fft_mfma.hpp", "fft_conv_mfma.hpp",
+                                      "fft_fir.hpp")]
 
 
 def hipcc():

@@ -196,8 +196,8 @@ def ThunderFFT_conv1d_real_async(T, N: int, d_x, d_spectrum, d_y, batch: int, ch
 
 def ThunderFFT_conv1d_valid(T, d_x, input_len: int, d_taps, filter_len: int, d_y, batch: int = 1,
                             stream=0) -> None:
-    """Tiled valid correlation y[b][i] = sum_k x[b][i + k] * taps[k] (complex, type T;
-    taps complex64, 1 <= filter_len <= 64) through 64-point FFT windows; synchronous."""
+    """Valid correlation y[b][i] = sum_k x[b][i + k] * taps[k] (complex, type T; taps
+    complex64, 1 <= filter_len <= 64); needs the table of N = 64; synchronous."""
     _raise(lib().thff_conv1d_valid(_precision(T), _ptr(d_x), int(input_len), _ptr(d_taps),
                                    int(filter_len), _ptr(d_y), int(batch), _stream(stream)))
 

@@ -4,6 +4,7 @@
 #include "thunderfft/detail/fft_c2c.hpp"
 #include "thunderfft/detail/fft_conv.hpp"
 #include "thunderfft/detail/fft_conv_mfma.hpp"
+#include "thunderfft/detail/fft_fir.hpp"
 #include "thunderfft/detail/fft_mfma.hpp"
 #include "launch.hpp"
 
@@ -405,33 +406,31 @@ hipError_t launch_conv1d_real(int precision, const void* x, const float2* spectr
 }
 
 #if THFF_N == 64
-hipError_t launch_conv1d_valid(int precision, const void* x, long long len, const float2* taps,
-                               int ntaps, void* y, int batch, const float2* tw, int num_cus,
-                               hipStream_t stream) {
-    // fp32: a group is the 64 windows (one per transform slot) of one
-    // workgroup pass; each workgroup transforms the filter once and walks
-    // many groups, 2 workgroups per CU (the occupancy, with its span
-    // prefetch).  2^26 values, 9 taps: 232 us, against 294 us for runs of 4
-    // groups.
-    // half2: 256-point windows on MFMA (conv1d_valid_mfma_kernel), 16 windows
-    // per workgroup tile, a device grid of 4 workgroups per CU.
-    if (precision != 0) {
-        const long long valid = 257 - ntaps;
-        const long long windows = (len - ntaps + 1 + valid - 1) / valid;
-        const long long groups = (windows + 15) / 16 * batch;
-        const Grid g = make_grid(groups, 4, num_cus);
-        conv1d_valid_mfma_kernel<256><<<g.blocks, 256, 0, stream>>>(
-            static_cast<const __half2*>(x), taps, static_cast<__half2*>(y), len, ntaps, batch,
-            g.tiles_per_block);
-        return hipGetLastError();
+template <class IO, int A = 1>
+void enqueue_conv1d_fir(int steps, const IO* x, const float2* taps, IO* y, long long len, int ntaps,
+                        int batch, int num_cus, hipStream_t stream) {
+    using P = FirPlan<IO, A>;
+    if constexpr (A < P::kMaxSteps) {
+        if (steps > A) {
+            enqueue_conv1d_fir<IO, A + 1>(steps, x, taps, y, len, ntaps, batch, num_cus, stream);
+            return;
+        }
     }
-    const long long valid = 65 - ntaps;
-    const long long windows = (len - ntaps + 1 + valid - 1) / valid;
-    const long long groups = (windows + 63) / 64 * batch;
-    const Grid g = make_grid(groups, 2, num_cus);
-    conv1d_valid_kernel<float2><<<g.blocks, 256, 0, stream>>>(
-        static_cast<const float2*>(x), taps, static_cast<float2*>(y), len, ntaps, batch, tw,
-        g.tiles_per_block);
+    const long long spans = (len - ntaps + P::kSpan) / P::kSpan * batch;
+    const Grid g = make_grid((spans + 3) / 4, kFirPerCu<IO, A>, num_cus);
+    conv1d_fir_kernel<IO, A><<<g.blocks, 256, 0, stream>>>(x, taps, y, len, ntaps, batch);
+}
+
+hipError_t launch_conv1d_valid(int precision, const void* x, long long len, const float2* taps,
+                               int ntaps, void* y, int batch, int num_cus, hipStream_t stream) {
+    if (precision == 0)
+        enqueue_conv1d_fir<float2>(FirPlan<float2, 1>::steps(ntaps), static_cast<const float2*>(x),
+                                   taps, static_cast<float2*>(y), len, ntaps, batch, num_cus,
+                                   stream);
+    else
+        enqueue_conv1d_fir<__half2>(FirPlan<__half2, 1>::steps(ntaps),
+                                    static_cast<const __half2*>(x), taps, static_cast<__half2*>(y),
+                                    len, ntaps, batch, num_cus, stream);
     return hipGetLastError();
 }
 

@@ -334,9 +334,8 @@ int conv1d_valid_impl(int precision, const void* x, long long input_len, const v
     if ((reinterpret_cast<std::uintptr_t>(x) | reinterpret_cast<std::uintptr_t>(y)) % elem ||
         reinterpret_cast<std::uintptr_t>(taps) % 8)
         return fail(THFF_EINVAL, "ThunderFFT_conv1d_valid: misaligned pointer");
-    // Window groups of one launch (fp32: 64 windows of 64 points per group;
-    // fp16: 16 windows of 256 points), counted in 32 bits by the kernels'
-    // grid walk.
+    // The most that one call takes, counted in groups of 64 windows of 64
+    // points (fp32) or 16 of 256 (fp16): at least 2^30 outputs.
     const long long window = precision == THFF_FLOAT ? 64 : 256;
     const long long per_group = precision == THFF_FLOAT ? 64 : 16;
     const long long valid = window + 1 - filter_len;
@@ -350,7 +349,7 @@ int conv1d_valid_impl(int precision, const void* x, long long input_len, const v
     auto s = static_cast<hipStream_t>(stream);
     const hipError_t err = thff::launch_conv1d_valid(precision, x, input_len,
                                                      static_cast<const float2*>(taps), filter_len,
-                                                     y, batch, table, cus, s);
+                                                     y, batch, cus, s);
     if (err != hipSuccess) return fail_hip(err, "ThunderFFT_conv1d_valid launch");
     return finish(s, synchronize, "ThunderFFT_conv1d_valid synchronize");
 }
