@@ -585,195 +585,6 @@ __global__ __launch_bounds__(1024) void conv2d128_lanes_kernel(const float2* __r
 }
 
 // ---------------------------------------------------------------------------
-// Column pass of the multi-pass 2-D convolution of images too large for one
-// workgroup (R x C = 1024 x 1024 here; the reference's built 2-D convolution
-// is the same split, sample/conv2d/thunder.cu:70-207: row FFT kernel, a
-// column kernel that runs FFT x H x IFFT, an inverse row kernel).  The row
-// passes are the library's C2C kernels; this kernel does the columns.
-// A workgroup of 512 lanes takes 8 adjacent columns of one image (a unit):
-// it loads the R x 8 block in 16-byte pieces of whole rows (64 bytes per row
-// fp32, 32 half), stages it column by column into LDS slots, and wave w
-// transforms column c0 + w (R / 16 = 64 lanes, 16 values each) in its slot:
-//   kConv:  out = IFFT_col(FFT_col(in) * H[., c0 + w])  (H fp32, R x C)
-//   !kConv: out = scale * FFT_col(in)                   (a filter's spectrum)
-// then stages the results back and stores them the way they came.  In and
-// out may be the same buffer (each unit reads its block before writing it).
-// Units are walked grid-stride; with a grid that is a multiple of the column
-// blocks per image, a workgroup keeps one column block for every image, so
-// its H column is loaded once and held in registers.  Slots are kSlotStride
-// apart (2 kSlotStride = 8 mod 64 banks), so the staging accesses of a
-// half-wave (4 columns x 8 rows) fall on distinct banks.  The next unit's
-// pieces are loaded before the current unit is transformed: held to 2 waves
-// per SIMD (one workgroup per CU), the kernel keeps its block, the next
-// block and the H column in registers without spilling (at 4 per SIMD the
-// forward and inverse column transforms alone spill).
-// ---------------------------------------------------------------------------
-namespace conv2dcols {
-template <int R>
-inline constexpr int kSlotStride = C2CPlan<R>::kSlot + 4;
-
-// Cols columns per unit, moved by kLanes lanes in 16-byte row pieces.
-template <class IO, int R, int Cols, int kLanes = 64 * Cols>
-struct Block {
-    static constexpr int kVec = Io<IO>::kVec;
-    static constexpr int kPer = Cols / kVec;                 // pieces per row
-    static constexpr int kRowsPerStep = kLanes / kPer;       // rows per lane step
-    static constexpr int kCount = R / kRowsPerStep;     // pieces per lane
-    typename Io<IO>::W4 w[kCount];
-};
-
-template <int First, int Last, int C, class IO, int R, int Cols, int L>
-__device__ __forceinline__ void load(Block<IO, R, Cols, L>& b, const IO* in, long long base, int tid) {
-    constexpr long long cols = C;
-    using B = Block<IO, R, Cols, L>;
-    const int p = tid % B::kPer, r0 = tid / B::kPer;
-#pragma unroll
-    for (int i = First; i < Last; ++i) {
-        const long long e = base + static_cast<long long>(r0 + B::kRowsPerStep * i) * cols + B::kVec * p;
-        b.w[i] = ld_nt(reinterpret_cast<const typename Io<IO>::W4*>(in + e));
-    }
-}
-
-template <class IO, int R, int Cols, int L>
-__device__ __forceinline__ void stage(const Block<IO, R, Cols, L>& b, cpx* lds, int tid) {
-    using B = Block<IO, R, Cols, L>;
-    const int p = tid % B::kPer, r0 = tid / B::kPer;
-#pragma unroll
-    for (int i = 0; i < B::kCount; ++i) {
-        cpx q[B::kVec];
-        Io<IO>::decode4(b.w[i], q);
-#pragma unroll
-        for (int c = 0; c < B::kVec; ++c)
-            lds[(B::kVec * p + c) * kSlotStride<R> + lds_pad(r0 + B::kRowsPerStep * i)] = q[c];
-    }
-}
-
-template <int C, class IO, int R, int Cols, int L = 64 * Cols>
-__device__ __forceinline__ void store(IO* out, long long base, const cpx* lds, int tid) {
-    constexpr long long cols = C;
-    using B = Block<IO, R, Cols, L>;
-    const int p = tid % B::kPer, r0 = tid / B::kPer;
-#pragma unroll
-    for (int i = 0; i < B::kCount; ++i) {
-        cpx q[B::kVec];
-#pragma unroll
-        for (int c = 0; c < B::kVec; ++c)
-            q[c] = lds[(B::kVec * p + c) * kSlotStride<R> + lds_pad(r0 + B::kRowsPerStep * i)];
-        const long long e = base + static_cast<long long>(r0 + B::kRowsPerStep * i) * cols + B::kVec * p;
-        st_nt(reinterpret_cast<typename Io<IO>::W4*>(out + e), Io<IO>::encode4(q));
-    }
-}
-}  // namespace conv2dcols
-
-// Waves per SIMD: 8 columns per unit (512 lanes, one wave per column) hold
-// two, with the next unit's block prefetched; 16 columns (512 lanes, two
-// columns per wave) two, loading each block when its unit starts (the
-// prefetch would spill there); 4 columns (256 lanes) three, likewise.
-template <int Cols>
-inline constexpr int kColsWavesPerEU = Cols == 8 || Cols == 16 ? 2 : 3;
-template <int Cols>
-inline constexpr bool kColsPrefetch = Cols == 8;
-// Lanes per workgroup: one wave per column up to 8 columns; 16 columns are
-// 8 waves of two columns each.
-template <int Cols>
-inline constexpr int kColsLanes = Cols <= 8 ? 64 * Cols : 512;
-
-template <class In, class Out, int R, int C, bool kConv, int Cols>
-__global__ __launch_bounds__(kColsLanes<Cols>) __attribute__((amdgpu_waves_per_eu(kColsWavesPerEU<Cols>))) void
-conv2d_cols_kernel(const In* in, Out* out, const float2* __restrict__ H, long long units,
-                   float scale, const float2* __restrict__ tw) {
-    using P = C2CPlan<R>;
-    static_assert(P::kTPF == 64, "one wave per column");
-    using namespace conv2dcols;
-    constexpr int kL = kColsLanes<Cols>;
-    constexpr int kWaves = kL / 64;
-    constexpr int kCPW = Cols / kWaves;  // columns per wave
-    __shared__ __align__(16) cpx lds[Cols * kSlotStride<R>];
-    const int tid = threadIdx.x, wave = tid >> 6, t = tid & 63;
-    LaneTwiddles<R> w;
-    w.load(t, tw);
-    constexpr long long cols = C;
-    constexpr long long blocks_per_image = C / Cols;
-    constexpr int kAll = Block<In, R, Cols, kL>::kCount;
-
-    // A 128-byte line of a row holds kShare adjacent column blocks.  Work
-    // items u = b + k G are renamed within aligned groups of 8 kShare so that
-    // workgroups b, b + 8, b + 16, ... -- dispatched to the same XCD -- take
-    // the kShare blocks of one line: the line is then fetched into one XCD's
-    // L2 once instead of once per XCD (with consecutive blocks on consecutive
-    // XCDs, FETCH_SIZE read 2x the data for fp32, 4x for half).
-    constexpr int kShare = 128 / (Cols * static_cast<int>(sizeof(In))) > 1
-                               ? 128 / (Cols * static_cast<int>(sizeof(In))) : 1;
-    constexpr int kGroup = 8 * kShare;
-    static_assert(blocks_per_image % kGroup == 0, "column blocks per image: whole groups");
-    auto where = [&](long long u0, long long& base, int& c0) {
-        const int i = static_cast<int>(u0 % kGroup);
-        const long long u = u0 - i + kShare * (i % 8) + i / 8;
-        const long long img = u / blocks_per_image;
-        c0 = static_cast<int>(u - img * blocks_per_image) * Cols;
-        base = img * R * static_cast<long long>(cols) + c0;
-    };
-    long long u = blockIdx.x;
-    if (u >= units) return;  // uniform over the workgroup
-    long long base;
-    int c0;
-    where(u, base, c0);
-    Block<In, R, Cols, kL> raw;
-    if constexpr (kColsPrefetch<Cols>) load<0, kAll, C>(raw, in, base, tid);
-    int h_c0 = -1;
-    cpx hs[kCPW][kConv ? 16 : 1];
-    for (; u < units; u += gridDim.x) {
-        const long long next_u = u + gridDim.x;
-        long long next_base = 0;
-        int next_c0 = 0;
-        if (next_u < units) where(next_u, next_base, next_c0);
-        if constexpr (!kColsPrefetch<Cols>) load<0, kAll, C>(raw, in, base, tid);
-        __syncthreads();  // the previous unit's reads of the slots are done
-        stage(raw, lds, tid);
-        if constexpr (kColsPrefetch<Cols>)
-            if (next_u < units) load<0, kAll, C>(raw, in, next_base, tid);
-        if constexpr (kConv) {
-            if (c0 != h_c0) {  // uniform: this workgroup's column block changed
-#pragma unroll
-                for (int v = 0; v < kCPW; ++v) {
-                    const float2* hc = H + c0 + wave + kWaves * v;
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) {
-                        const float2 hk = hc[static_cast<long long>(t + 64 * j) * cols];
-                        hs[v][j] = {hk.x, hk.y};
-                    }
-                }
-                h_c0 = c0;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int cv = 0; cv < kCPW; ++cv) {
-            cpx* const slot = lds + (wave + kWaves * cv) * kSlotStride<R>;
-            cpx v[16];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) v[j] = slot[lds_pad(t + 64 * j)];
-            fft_registers<R, true>(v, slot, t, w);
-            if constexpr (kConv) {
-#pragma unroll
-                for (int j = 0; j < 16; ++j) v[j] = cmul(v[j], hs[cv][j]);
-                fft_registers<R, false>(v, slot, t, w);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 16; ++j) v[j] = {v[j].re * scale, v[j].im * scale};
-            }
-            wave_lds_sync();
-#pragma unroll
-            for (int j = 0; j < 16; ++j) slot[lds_pad(t + 64 * j)] = v[j];
-        }
-        __syncthreads();
-        store<C, Out, R, Cols, kL>(out, base, lds, tid);
-        base = next_base;
-        c0 = next_c0;
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Real-input, real-output fused convolution with one real filter per channel
 // (the reference's thunder_convN_block_kernel_realin_realout,
 // sample/conv1d/conv1d_fullfft_l4096_thunder.cu:280-331, generalised to all

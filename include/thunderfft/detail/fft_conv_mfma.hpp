@@ -1487,181 +1487,3 @@ conv2d128_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__
 }
 
 }  // namespace thff
-
-namespace thff {
-
-// ---------------------------------------------------------------------------
-// The fused column pass of the 1024 x 1024 half2 convolution on MFMA: for
-// each of a unit's 16 adjacent columns, IFFT_col(FFT_col(y) * H) with the
-// two-stage N = 1024 transform of c2c_mfma_kernel (conv2d_cols_kernel's
-// contract with conv = true; H is the fp32 filter spectrum, 1/2^20 folded
-// in, read once per workgroup).  One 512-lane workgroup per CU, 8 waves of
-// two columns each:
-//   load:  the unit's 1024 rows as 64-byte row pieces (16 rows per wave
-//          instruction; lane l of half h takes piece 2h + ((l & 31) >> 4) of
-//          row 16 (8 i + w) + (l & 15));
-//   stage: each piece's four half2 go to the four columns' slots at the
-//          transform's input positions (MfmaPlan<4>::in_pad).  Slots are
-//          kSlot = 1284 dwords apart (4 mod 32): the pieces 2h and 2h + 1 of
-//          16 consecutive rows that one half-wave writes fall on 32 banks;
-//   per column: stage 1 from the slot, steps 2-6 (their wave-local
-//          transposes in a 256-byte-aligned window of the slot), the product
-//          with H's column (fp32 registers, the forward's output layout),
-//          the inverse as conj(DFT(conj(P))) from the registers, and the
-//          result into the slot at the output positions (out_pad);
-//   store: the four columns of each row piece back together, 16 bytes.
-// The workgroups walk the units grid-stride with the grid a multiple of the
-// image's 64 column blocks, so each keeps one block (and its H columns) for
-// every image; blocks that share a 128-byte line are renamed onto one XCD
-// as in conv2d_cols_kernel.  The next unit's pieces are loaded while the
-// current unit is transformed (250 VGPRs, 96.5 KB of LDS).  Measured on
-// MI355X, 32 images end to end: 214.8 us against 249.7 us with the VALU
-// column pass; without the prefetch 224.6 us; 16 waves of one column each
-// (4 per SIMD, 128 VGPRs, no room for the prefetch) 224.4 us.  The f16
-// roundings of the two transforms take the convolution's rel L2 against the
-// fp64 direct convolution from 5.3e-4 to 7.0e-4.
-// ---------------------------------------------------------------------------
-namespace conv2dcolsm {
-inline constexpr int kCols = 16;
-inline constexpr int kRows = 1024;
-inline constexpr int kImgCols = 1024;
-inline constexpr int kSlot = 1284;
-static_assert(MfmaPlan<4>::kRegion <= kSlot, "a slot holds the transform's staging region");
-static_assert(1024 + 60 <= kSlot, "a slot holds a 256-byte-aligned transpose window");
-}  // namespace conv2dcolsm
-
-template <int kUnused = 0>  // a template: the header is compiled into several objects
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void
-conv2d_cols_mfma_kernel(const __half2* in, __half2* out, const float2* __restrict__ H,
-                        long long units, const float2* __restrict__ tw) {
-    using namespace conv2dcolsm;
-    using P = MfmaPlan<4>;
-    constexpr int kWaves = 8;
-    constexpr int kLanes = 64 * kWaves;
-    constexpr int kSteps = kRows * (kCols / 4) / kLanes;  // 16-byte pieces per lane
-    constexpr int kRowStep = 16 * kWaves;                 // rows between a lane's pieces
-    constexpr int kCPW = kCols / kWaves;                  // columns per wave
-    __shared__ __align__(256) unsigned blk[kCols * kSlot];
-    __shared__ cpx w1[P::kTw1];
-    __shared__ u32x4 a3[P::kA3];
-    const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int n = lane & 15, q = lane >> 4;
-
-    f16x8 a[2], a_regs[2];
-    mfma_setup<4, true, kLanes>(a, w1, a3, nullptr, tw);
-    dft16_operands<true, true>(a_regs, lane);
-    const Stage3Folded s3{a, a3, lane};
-
-    // This lane's row pieces: piece p of rows row0 + kRowStep i.
-    const int p = 2 * (lane >> 5) + ((lane & 31) >> 4);
-    const int row0 = 16 * wave + (lane & 15);
-
-    constexpr long long blocks_per_image = kImgCols / kCols;
-    constexpr int kShare = 2;  // 64-byte pieces: two column blocks per 128-byte line
-    constexpr int kGroup = 8 * kShare;
-    static_assert(blocks_per_image % kGroup == 0, "column blocks per image: whole groups");
-    auto where = [&](long long u0, long long& base, int& c0) {
-        const int i = static_cast<int>(u0 % kGroup);
-        const long long u = u0 - i + kShare * (i % 8) + i / 8;
-        const long long img = u / blocks_per_image;
-        c0 = static_cast<int>(u - img * blocks_per_image) * kCols;
-        base = img * kRows * static_cast<long long>(kImgCols) + c0;
-    };
-    long long u = blockIdx.x;
-    if (u >= units) return;  // uniform over the workgroup
-
-    int h_c0 = -1;
-    cpx hs[kCPW][4][4];  // H of the wave's columns, bin n + 16 m + 64 (q + 4 r)
-    auto load = [&](long long b, u32x4 (&raw)[kSteps]) {
-#pragma unroll
-        for (int i = 0; i < kSteps; ++i)
-            raw[i] = ld_nt(reinterpret_cast<const u32x4*>(
-                in + b + static_cast<long long>(row0 + kRowStep * i) * kImgCols + 4 * p));
-    };
-    long long base;
-    int c0;
-    where(u, base, c0);
-    u32x4 raw[kSteps];
-    load(base, raw);  // the next unit's pieces are loaded during the current unit
-    {
-        // kSteps stores to a resource of no bytes (dropped by the range
-        // check): the loop is then entered, like every later pass, with the
-        // pieces followed by kSteps stores in flight, so the compiler's count
-        // at the staging waits for the pieces only, not for the previous
-        // unit's stores.  (The size is a run-time value, units >= 0 always,
-        // so the stores are not deleted.)
-        const __amdgpu_buffer_rsrc_t none =
-            __builtin_amdgcn_make_buffer_rsrc(out, 0, units < 0 ? 16 : 0, 0x00020000);
-        __builtin_amdgcn_sched_barrier(0);  // after the loads, as in the loop
-#pragma unroll
-        for (int i = 0; i < kSteps; ++i)
-            __builtin_amdgcn_raw_buffer_store_b128(u32x4{}, none, 16 * i, 0, 2);
-    }
-    for (; u < units; u += gridDim.x) {
-        if (c0 != h_c0) {  // uniform: this workgroup's column block changed
-#pragma unroll
-            for (int cv = 0; cv < kCPW; ++cv)
-#pragma unroll
-                for (int m = 0; m < 4; ++m)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int k = n + 16 * m + 64 * (q + 4 * r);
-                        const float2 hk = H[static_cast<long long>(k) * kImgCols + c0 + wave + kWaves * cv];
-                        hs[cv][m][r] = cpx{hk.x, hk.y};
-                    }
-            wait_vmem_all();  // here, on this rarely taken path (not after the branch)
-            h_c0 = c0;
-        }
-        __syncthreads();  // the previous unit's store reads of the slots are done
-#pragma unroll
-        for (int i = 0; i < kSteps; ++i) {
-            const int pos = P::in_pad(row0 + kRowStep * i);
-            const unsigned w[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
-#pragma unroll
-            for (int c = 0; c < 4; ++c) blk[(4 * p + c) * kSlot + pos] = w[c];
-        }
-        const long long cur = base;
-        if (u + gridDim.x < units) {
-            where(u + gridDim.x, base, c0);
-            load(base, raw);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int cv = 0; cv < kCPW; ++cv) {
-            const int col = wave + kWaves * cv;
-            unsigned* const slot = blk + col * kSlot;
-            // the transposes' window: the slot's first 256-byte boundary
-            unsigned* const win = slot + ((64 - (col * kSlot) % 64) % 64);
-            cpx v[4][4];
-            mfma_stage1_lds<4>(slot, a, lane, v);
-            mfma_steps2to6<4, true>(win, w1, s3, lane, v);
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[m][r] = cmul(v[m][r], hs[cv][m][r]);
-            mfma_stage1_regs<4, true>(a_regs, v);
-            mfma_steps2to6<4, true>(win, w1, s3, lane, v);
-            wave_lds_sync();
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    slot[P::out_pad(n + 16 * m + 64 * (q + 4 * r))] =
-                        pack_half2({v[m][r].re, -v[m][r].im});
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < kSteps; ++i) {
-            const int pos = P::out_pad(row0 + kRowStep * i);
-            u32x4 w;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) w[c] = blk[(4 * p + c) * kSlot + pos];
-            st_nt(reinterpret_cast<u32x4*>(out + cur + static_cast<long long>(row0 + kRowStep * i) * kImgCols +
-                                           4 * p),
-                  w);
-        }
-    }
-}
-
-}  // namespace thff

@@ -53,15 +53,8 @@ struct C2CPlan {
 
 __device__ __forceinline__ int lds_pad(int i) { return i + (i >> 4); }
 
-// A transform's LDS slot: element i of a contiguous slot sits at lds_pad(i);
-// a strided slot holds element i at base[i * stride] (a column of an image
-// kept row-major in LDS, transformed where it lies).
+// A transform's LDS slot: element i of a contiguous slot sits at lds_pad(i).
 __device__ __forceinline__ cpx& slot_at(cpx* slot, int i) { return slot[lds_pad(i)]; }
-struct StridedSlot {
-    cpx* base;
-    int stride;
-};
-__device__ __forceinline__ cpx& slot_at(StridedSlot s, int i) { return s.base[i * s.stride]; }
 
 template <bool WaveLocal>
 __device__ __forceinline__ void region_sync() {
@@ -69,6 +62,18 @@ __device__ __forceinline__ void region_sync() {
         wave_lds_sync();
     else
         __syncthreads();
+}
+
+// A contiguous slot whose transform's lanes are spread over the waves of the
+// workgroup, at any N: its passes synchronise the workgroup.
+struct SharedSlot {
+    cpx* base;
+};
+__device__ __forceinline__ cpx& slot_at(SharedSlot s, int i) { return s.base[lds_pad(i)]; }
+
+template <bool WaveLocal, class Slot>
+__device__ __forceinline__ void slot_sync(Slot) {
+    region_sync<WaveLocal && !std::is_same_v<Slot, SharedSlot>>();
 }
 
 // Twiddles of the pass of radix R that follows sub-transforms of length L.
@@ -160,7 +165,7 @@ __device__ __forceinline__ void stockham_pass(cpx (&v)[16], Slot slot, int t,
                                               const PassTwiddles<N, R, L>& tw) {
     using P = C2CPlan<N>;
     // previous outputs: butterfly b = t + TPF*q, output m -> (b/LPrev)*LPrev*RPrev + b%LPrev + m*LPrev
-    region_sync<P::kWaveLocal>();
+    slot_sync<P::kWaveLocal>(slot);
 #pragma unroll
     for (int q = 0; q < 16 / RPrev; ++q) {
         const int b = t + P::kTPF * q;
@@ -168,7 +173,7 @@ __device__ __forceinline__ void stockham_pass(cpx (&v)[16], Slot slot, int t,
 #pragma unroll
         for (int m = 0; m < RPrev; ++m) slot_at(slot, base + m * LPrev) = v[q * RPrev + m];
     }
-    region_sync<P::kWaveLocal>();
+    slot_sync<P::kWaveLocal>(slot);
     cpx w[R - 1];
     tw.expand(w);
     static_for<0, 16 / R>([&](auto qc) {
@@ -186,7 +191,7 @@ __device__ __forceinline__ void stockham_pass(cpx (&v)[16], Slot slot, int t,
 
 // The whole transform of the lane's transform slot: v[j] = x[t + TPF*j] in,
 // v[j] = X[t + TPF*j] out.  `slot` is the transform's LDS slot (cpx* or
-// StridedSlot).
+// SharedSlot).
 template <int N, bool FWD, class Slot>
 __device__ __forceinline__ void fft_registers(cpx (&v)[16], Slot slot, int t,
                                               const LaneTwiddles<N>& w) {

@@ -456,3 +456,36 @@ def test_conv2d_beyond_2e31_values(T):
     assert err <= TIGHT[T]
     del x, y
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("T", ["float", "half"])
+@pytest.mark.parametrize("batch", [1, 2, 3, 4, 5, 7])
+def test_conv2d_1024_image_counts_and_range(T, batch):
+    """Image counts around the images that a column pass has in flight (3 on
+    256 CUs, then a second round of some or all), each image rolled by a
+    one-tap filter; and constant images of 60, whose row sums (61440) are just
+    below the largest half.  Bound of a result in half: one rounding of it
+    (2^-11) and two of the spectra on the way, at most 2^-11 of the largest
+    spectrum each, spread evenly; gated as the other convolutions here."""
+    import torch
+
+    import thunderfft_amd as thff
+
+    size = 1024
+    thff.ThunderFFTInitialize(T, size)
+    dt = torch.float32 if T == "float" else torch.float16
+    x = torch.empty(2 * size * size * batch, dtype=dt, device="cuda")
+    thff.fill_uniform(T, x, size * size * batch, 31 + batch)
+    flat = torch.zeros(batch, size, size, 2, dtype=dt, device="cuda")
+    flat[..., 0] = 60.0
+    dr, dc = 129, 31
+    imp = np.zeros((size, size), dtype=np.complex64)
+    imp[dr, dc] = 1
+    h = to_device(imp, T)
+    for image in (x, flat):
+        y = torch.full_like(image, float("nan"))
+        thff.ThunderFFT_conv2d(T, size, size, image, h, y, batch)
+        want = torch.roll(image.view(batch, size, size, 2).float(), shifts=(dr, dc), dims=(1, 2))
+        err = (y.view(batch, size, size, 2).float() - want).flatten(1)
+        rel = torch.linalg.vector_norm(err, dim=1) / torch.linalg.vector_norm(want.flatten(1), dim=1)
+        assert bool(torch.isfinite(rel).all()) and float(rel.max()) <= TIGHT[T], (T, batch, rel)

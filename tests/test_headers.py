@@ -12,7 +12,7 @@ HEADERS = ["thunderfft/thunderfft.h", "thunderfft/thunderfft.hpp", "thunderfft/t
            "thunderfft/thunderfft_device.hpp"] + [
     f"thunderfft/detail/{h}" for h in ("fft_core.hpp", "fft_tile.hpp", "fft_c2c.hpp",
                                       "fft_conv.hpp", "fft_mfma.hpp", "fft_conv_mfma.hpp",
-                                      "fft_fir.hpp")]
+                                      "fft_fir.hpp", "fft_image.hpp")]
 
 
 def hipcc():

@@ -5,6 +5,7 @@
 #include "thunderfft/detail/fft_conv.hpp"
 #include "thunderfft/detail/fft_conv_mfma.hpp"
 #include "thunderfft/detail/fft_fir.hpp"
+#include "thunderfft/detail/fft_image.hpp"
 #include "thunderfft/detail/fft_mfma.hpp"
 #include "launch.hpp"
 
@@ -477,69 +478,32 @@ hipError_t launch_conv2d128(int precision, const void* x, const void* h, void* y
 #endif
 
 #if THFF_N == 1024
-hipError_t launch_conv2d_cols(int precision, bool conv, const void* in, void* out,
-                              const float2* H, int cols, long long images, float scale,
-                              const float2* tw, int num_cus, hipStream_t stream) {
-    if (cols != 1024) return hipErrorInvalidValue;  // the kernels are built for 1024 columns
-    // kCols columns per unit (one wave per column for fp32, two per wave for
-    // half); workgroups walk the units grid-stride, and the grid is a multiple
-    // of the image's column blocks, so every workgroup keeps one column block
-    // (and its H columns).  The unit's rows move as 16-byte pieces, 64 bytes
-    // of each row (fp32: 8 columns; half: 16), through one 512-lane workgroup
-    // per CU.  Measured on MI355X, 32 images of 1024 x 1024 end to end: fp32
-    // 8 columns with the next block prefetched 359 us (16 columns, two per
-    // wave, no prefetch: 358 us, 124 bytes of spill); half 16 columns 253 us
-    // against 277 us with 8 columns (32-byte pieces: a wave's loads then touch
-    // twice the rows); one column per wave on MFMA with 16-byte pieces (4
-    // columns per 256-lane workgroup) 545 us.  A pass over fewer units than
-    // two per CU (one or a few images, and the filter's column pass of every
-    // call) runs 4-column units instead, 256-lane workgroups of one column
-    // per wave, so that more CUs share the columns: one image end to end
-    // (filter spectrum included) fp16 43.5 against 60.8 us, fp32 48.6 against
-    // 52.4 us (2-column fp32 units: 57.5 us); 32 images fp16 248.5 against
-    // 253.1 us (the filter's pass).
-    auto launch = [&](auto cols_tag, const void* src, void* dst) {
-        constexpr int kCols = decltype(cols_tag)::value;
-        constexpr int kPerCu = kColsWavesPerEU<kCols> * 4 / (kColsLanes<kCols> / 64);
-        const long long blocks_per_image = cols / kCols;
-        const long long units = blocks_per_image * images;
-        long long grid = static_cast<long long>(kPerCu) * (num_cus > 0 ? num_cus : 256);
-        if (grid >= blocks_per_image) grid -= grid % blocks_per_image;
-        const dim3 blocks(static_cast<unsigned>(units < grid ? units : grid));
-        const dim3 lanes(kColsLanes<kCols>);
-        if (precision == 0) {
-            if (conv)
-                conv2d_cols_kernel<float2, float2, 1024, 1024, true, kCols><<<blocks, lanes, 0, stream>>>(
-                    static_cast<const float2*>(src), static_cast<float2*>(dst), H, units, scale, tw);
-            else
-                conv2d_cols_kernel<float2, float2, 1024, 1024, false, kCols><<<blocks, lanes, 0, stream>>>(
-                    static_cast<const float2*>(src), static_cast<float2*>(dst), H, units, scale, tw);
-        } else {
-            if (conv)
-                conv2d_cols_kernel<__half2, __half2, 1024, 1024, true, kCols><<<blocks, lanes, 0, stream>>>(
-                    static_cast<const __half2*>(src), static_cast<__half2*>(dst), H, units, scale, tw);
-            else
-                conv2d_cols_kernel<__half2, float2, 1024, 1024, false, kCols><<<blocks, lanes, 0, stream>>>(
-                    static_cast<const __half2*>(src), static_cast<float2*>(dst), H, units, scale, tw);
-        }
-    };
-    const long long wide = precision == 0 ? 8 : 16;
-    const long long cus = num_cus > 0 ? num_cus : 256;
-    if (images * (cols / wide) < 2LL * cus) {
-        launch(std::integral_constant<int, 4>{}, in, out);
-    } else if (precision != 0 && conv) {
-        // half2 with the product: 16 columns per unit on MFMA, one 512-lane
-        // workgroup per CU (conv2d_cols_mfma_kernel): 32 images end to end
-        // 214.8 against 249.7 us with the VALU pass below.
-        const long long units = images * (cols / 16);
-        long long grid = cus;
-        if (grid >= cols / 16) grid -= grid % (cols / 16);
-        conv2d_cols_mfma_kernel<><<<static_cast<unsigned>(units < grid ? units : grid), 512, 0, stream>>>(
-            static_cast<const __half2*>(in), static_cast<__half2*>(out), H, units, tw);
-    } else if (precision == 0)
-        launch(std::integral_constant<int, 8>{}, in, out);
+namespace {
+template <class IO>
+void enqueue_conv2d1024(const IO* x, const IO* h, IO* y, float2* workspace, int batch,
+                        const float2* tw, int num_cus, hipStream_t stream) {
+    using P = ImagePlan<IO>;
+    const unsigned groups = static_cast<unsigned>(batch) * P::kLen;
+    image_rows_kernel<IO, true><<<groups + P::kLen, P::kRowLanes, 0, stream>>>(
+        x, y, h, workspace, groups, tw);
+    const int wanted = kImageColsPerCu * num_cus / P::kBlocks;  // images in flight
+    const int images = wanted < 1 ? 1 : wanted < batch ? wanted : batch;
+    image_cols_kernel<IO><<<P::kBlocks * images, 256, 0, stream>>>(
+        y, workspace, batch, P::kScale / (1024.0f * 1024.0f), tw);
+    image_rows_kernel<IO, false><<<groups, P::kRowLanes, 0, stream>>>(y, y, nullptr, nullptr, groups,
+                                                                      tw);
+}
+}  // namespace
+
+hipError_t launch_conv2d1024(int precision, const void* x, const void* h, void* y,
+                             float2* workspace, int batch, const float2* tw, int num_cus,
+                             hipStream_t stream) {
+    if (precision == 0)
+        enqueue_conv2d1024(static_cast<const float2*>(x), static_cast<const float2*>(h),
+                           static_cast<float2*>(y), workspace, batch, tw, num_cus, stream);
     else
-        launch(std::integral_constant<int, 16>{}, in, out);
+        enqueue_conv2d1024(static_cast<const __half2*>(x), static_cast<const __half2*>(h),
+                           static_cast<__half2*>(y), workspace, batch, tw, num_cus, stream);
     return hipGetLastError();
 }
 #endif

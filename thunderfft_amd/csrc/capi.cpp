@@ -355,10 +355,8 @@ int conv1d_valid_impl(int precision, const void* x, long long input_len, const v
 }
 
 // 2-D convolution sizes: rows = cols = 64 and 128 run one fused kernel per
-// image (the image stays on chip); 1024 runs the multi-pass form of the
-// reference's built sample (sample/conv2d/thunder.cu:70-207): the filter's
-// spectrum into a stream-ordered workspace, then row FFTs (the C2C kernel),
-// a column pass doing FFT x H x IFFT, and inverse row FFTs, in place in y.
+// image (the image stays on chip); 1024 runs the three passes of
+// fft_image.hpp, with a stream-ordered workspace for the filter's row spectra.
 int conv2d_impl(int precision, int rows, int cols, const void* x, const void* h, void* y,
                 int batch, void* stream, bool synchronize, bool allocate = true) {
     if (!supported_precision(precision))
@@ -406,20 +404,8 @@ int conv2d_impl(int precision, int rows, int cols, const void* x, const void* h,
             if (src != THFF_OK) return src;
             spectrum = p;
         }
-        auto* H = static_cast<float2*>(spectrum);
-        const int row_signals = batch * kN;
-        // H = FFT2(h) / (rows * cols): columns (scaled, into fp32), then rows in place
-        err = thff::launch_conv2d_cols(precision, false, h, H, nullptr, kN, 1,
-                                       1.0f / (static_cast<float>(kN) * kN), table, cus, s);
-        if (err == hipSuccess)
-            err = thff::launch_c2c<kN>(THFF_FLOAT, true, true, H, H, kN, table, cus, s);
-        if (err == hipSuccess)
-            err = thff::launch_c2c<kN>(precision, true, true, x, y, row_signals, table, cus, s);
-        if (err == hipSuccess)
-            err = thff::launch_conv2d_cols(precision, true, y, y, H, kN, batch, 0.0f, table,
-                                           cus, s);
-        if (err == hipSuccess)
-            err = thff::launch_c2c<kN>(precision, false, true, y, y, row_signals, table, cus, s);
+        err = thff::launch_conv2d1024(precision, x, h, y, static_cast<float2*>(spectrum), batch,
+                                      table, cus, s);
         if (allocate) {
             const hipError_t ferr = hipFreeAsync(spectrum, s);
             if (err == hipSuccess) err = ferr;

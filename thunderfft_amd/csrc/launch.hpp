@@ -49,16 +49,14 @@ hipError_t launch_conv2d64(int precision, const void* x, const void* h, void* y,
 hipError_t launch_conv2d128(int precision, const void* x, const void* h, void* y, int batch,
                             const float2* tw, int num_cus, hipStream_t stream);
 
-// Enqueue the column pass of the multi-pass 2-D convolution over `images`
-// 1024-row images with `cols` columns (tw: the N = 1024 table).  conv:
-// out = IFFT_col(FFT_col(in) * H) (in, out: the precision's storage, may be
-// the same buffer; H fp32 rows x cols); otherwise out = scale * FFT_col(in)
-// with out fp32 complex.
-hipError_t launch_conv2d_cols(int precision, bool conv, const void* in, void* out,
-                              const float2* H, int cols, long long images, float scale,
-                              const float2* tw, int num_cus, hipStream_t stream);
+// Enqueue the fused 2-D circular convolution of `batch` 1024 x 1024 images
+// with one shared 1024 x 1024 filter h (tw: the N = 1024 table); workspace: one
+// image of fp32 complex values.
+hipError_t launch_conv2d1024(int precision, const void* x, const void* h, void* y,
+                             float2* workspace, int batch, const float2* tw, int num_cus,
+                             hipStream_t stream);
 
-// Transforms per tile (4096 complex values, one workgroup pass) for length N.// Transforms per tile (4096 complex values, one workgroup pass) for length N.
+// Transforms per tile (4096 complex values, one workgroup pass) for length N.
 int c2c_transforms_per_block(int n);
 
 
