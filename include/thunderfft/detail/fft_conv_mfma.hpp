@@ -112,7 +112,7 @@ template <int C, bool kBufferIO = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kConvMfmaMinWavesPerEU<C>))) void
 conv1d_real_mfma_kernel(const __half* __restrict__ x, const float2* __restrict__ spectrum,
                         __half* __restrict__ y, int batch, int channels,
-                        const float2* __restrict__ tw, int tiles_per_block) {
+                        int tiles_per_block) {
     using P = MfmaPlan<C>;
     constexpr int N = P::N;
     constexpr int kB = P::kBlocks;
@@ -128,7 +128,7 @@ conv1d_real_mfma_kernel(const __half* __restrict__ x, const float2* __restrict__
     unsigned* region = lds + wave * P::kRegion;
 
     f16x8 a[2], a_regs[2];
-    mfma_setup<C, true>(a, w1, a3, nullptr, tw);  // forward operands and twiddles
+    mfma_setup<C, true>(a, w1, a3, nullptr);  // forward operands and twiddles
     dft16_operands<true, true>(a_regs, lane);
     const Stage3Folded s3{a, a3, lane};
 
@@ -300,8 +300,7 @@ inline constexpr int kConv1dMfmaMinWavesPerEU = C <= 4 ? 3 : 2;
 template <int C, bool kPerSignal>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kConv1dMfmaMinWavesPerEU<C>))) void
 conv1d_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__ h,
-                   __half2* __restrict__ y, int batch, const float2* __restrict__ tw,
-                   int tiles_per_block) {
+                   __half2* __restrict__ y, int batch, int tiles_per_block) {
     using P = MfmaPlan<C>;
     constexpr int N = P::N;
     constexpr int kB = P::kBlocks;
@@ -317,7 +316,7 @@ conv1d_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__ h,
     unsigned* region = lds + wave * P::kRegion;
 
     f16x8 a[2], a_regs[2];
-    mfma_setup<C, true>(a, w1, a3, nullptr, tw);
+    mfma_setup<C, true>(a, w1, a3, nullptr);
     // The inverse's stage-1 operands carry the 1/N of the convolution: a
     // power of two, exact in f16 for every coefficient here (|c| >= 0.38).
     dft16_operands<true, true>(a_regs, lane);
@@ -565,7 +564,7 @@ template <int N, bool kBufferIO = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
 conv1d_real_mfma4096_kernel(const __half* __restrict__ x, const float2* __restrict__ spectrum,
                             __half* __restrict__ y, int batch, int channels,
-                            const float2* __restrict__ tw, int tiles_per_block) {
+                            int tiles_per_block) {
     using P = Mfma4096;
     static_assert(N == P::N, "the three-stage transform is N = 4096");
     __shared__ __align__(16) unsigned xbuf[P::kExchange];
@@ -594,12 +593,9 @@ conv1d_real_mfma4096_kernel(const __half* __restrict__ x, const float2* __restri
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) a2[b][h] = dft16_operand_twiddled<true>(lane, h, 4 * wave + b, 16, tw);
+        for (int h = 0; h < 2; ++h) a2[b][h] = dft16_operand_twiddled<true>(lane, h, 4 * wave + b, 16);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float2 g = tw[(n * (4 * wave + b + 16 * (q + 4 * r))) & (N - 1)];
-            w2[b][r] = cpx{g.x, g.y};
-        }
+        for (int r = 0; r < 4; ++r) w2[b][r] = cis_rev(n * (4 * wave + b + 16 * (q + 4 * r)), N);
     }
 
     // tiles_per_block = 0: the grid is sized to the device and walks the
@@ -842,7 +838,7 @@ inline constexpr int kConv4096MinWavesPerEU = kPerSignal ? 3 : 2;
 template <int N, bool kPerSignal>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kConv4096MinWavesPerEU<kPerSignal>))) void
 conv1d_mfma4096_kernel(const __half2* __restrict__ x, const __half2* __restrict__ h,
-                       __half2* __restrict__ y, int batch, const float2* __restrict__ tw) {
+                       __half2* __restrict__ y, int batch) {
     using P = Mfma4096;
     static_assert(N == P::N, "the three-stage transform is N = 4096");
     __shared__ __align__(16) unsigned xbuf[P::kExchange];
@@ -864,12 +860,9 @@ conv1d_mfma4096_kernel(const __half2* __restrict__ x, const __half2* __restrict_
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) a2[b][hh] = dft16_operand_twiddled<true>(lane, hh, 4 * wave + b, 16, tw);
+        for (int hh = 0; hh < 2; ++hh) a2[b][hh] = dft16_operand_twiddled<true>(lane, hh, 4 * wave + b, 16);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float2 g = tw[(n * (4 * wave + b + 16 * (q + 4 * r))) & (N - 1)];
-            w2[b][r] = cpx{g.x, g.y};
-        }
+        for (int r = 0; r < 4; ++r) w2[b][r] = cis_rev(n * (4 * wave + b + 16 * (q + 4 * r)), N);
     }
 
     auto stages23 = [&](cpx (&v)[4][4]) {
@@ -1073,11 +1066,10 @@ __device__ __forceinline__ int op_index(int form, int j, int h, int lane) {
     return ((form * 3 + (j - 1)) * 2 + h) * 64 + lane;
 }
 
-// Entry e of the table, from the positive-angle table of length 64 (forward
-// sign: the conjugate).  Row m of half h is output k (grouped: 4 (m/4) + 2 h +
+// Entry e of the table (forward).  Row m of half h is output k (grouped: 4 (m/4) + 2 h +
 // (m%4)/2; q + 4 r order: m/4 + 4 (2 h + (m%4)/2)), part (m%4)%2; column kk is
 // input i = kk/2, part kk%2.
-__device__ __forceinline__ u32x4 op_entry(int e, const float2* __restrict__ tw64) {
+__device__ __forceinline__ u32x4 op_entry(int e) {
     const int lane = e & 63, h = (e >> 6) & 1, j = (e >> 7) % 3 + 1, form = (e >> 7) / 3;
     const int m = lane & 15, kq = lane >> 4;
     const int gq = m >> 2, i2 = m & 3, o = i2 & 1;
@@ -1086,13 +1078,9 @@ __device__ __forceinline__ u32x4 op_entry(int e, const float2* __restrict__ tw64
 #pragma unroll
     for (int x = 0; x < 8; ++x) {
         const int kk = 8 * kq + x;
-        const int in = kk >> 1, p = kk & 1;
+        const int in = kk >> 1;
         const int idx = form == 0 ? k * (j + 4 * in) : in * (4 * k + j);
-        const float2 w = tw64[idx & 63];
-        const float c = w.x, sn = -w.y;
-        // out.re = c*in.re - s*in.im ; out.im = s*in.re + c*in.im
-        const float v = o == 0 ? (p == 0 ? c : -sn) : (p == 0 ? sn : c);
-        r[x] = static_cast<_Float16>(v);
+        r[x] = rotation_entry<true>(idx, 64, o, kk & 1);
     }
     return __builtin_bit_cast(u32x4, r);
 }
@@ -1151,8 +1139,7 @@ __device__ __forceinline__ void forward(const unsigned* in, unsigned* fx, const 
 template <int kPerCu = 3>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kPerCu))) void
 conv2d64_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__ h,
-                     __half2* __restrict__ y, int batch, const float2* __restrict__ tw64,
-                     int tiles_per_block) {
+                     __half2* __restrict__ y, int batch, int tiles_per_block) {
     using namespace conv2dm;
     __shared__ __align__(16) unsigned buf[2][kBuf];
     __shared__ u32x4 ops[kOps];
@@ -1165,7 +1152,7 @@ conv2d64_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__ 
     f16x8 ag[2], as[2];
     dft16_operands_grouped<true>(ag, lane);
     dft16_operands<true>(as, lane);
-    for (int e = tid; e < kOps; e += 256) ops[e] = op_entry(e, tw64);  // read after a barrier below
+    for (int e = tid; e < kOps; e += 256) ops[e] = op_entry(e);  // read after a barrier below
 
     long long img, img_end, step;
     tile_walk(batch, tiles_per_block, img, img_end, step);
@@ -1318,10 +1305,9 @@ __device__ __forceinline__ int cm_addr(int c, int kr) {
 constexpr int kOps = 7 * 2 * 64;  // u32x4 entries (14 KB)
 __device__ __forceinline__ int op_index(int j, int h, int lane) { return ((j - 1) * 2 + h) * 64 + lane; }
 
-// Entry e of the table, from the positive-angle table of length 128 (the
-// forward sign is its conjugate).  Row m of half h is output k = 4 (m / 4) +
+// Entry e of the table (forward).  Row m of half h is output k = 4 (m / 4) +
 // 2 h + (m % 4) / 2, part (m % 4) % 2; column kk is input kk / 2, part kk % 2.
-__device__ __forceinline__ u32x4 op_entry(int e, const float2* __restrict__ tw128) {
+__device__ __forceinline__ u32x4 op_entry(int e) {
     const int lane = e & 63, h = (e >> 6) & 1, j = (e >> 7) + 1;
     const int m = lane & 15, kq = lane >> 4;
     const int o = m & 1;
@@ -1330,12 +1316,7 @@ __device__ __forceinline__ u32x4 op_entry(int e, const float2* __restrict__ tw12
 #pragma unroll
     for (int x = 0; x < 8; ++x) {
         const int kk = 8 * kq + x;
-        const int in = kk >> 1, p = kk & 1;
-        const float2 w = tw128[(k * (j + 8 * in)) & 127];
-        const float c = w.x, sn = -w.y;
-        // out.re = c*in.re - s*in.im ; out.im = s*in.re + c*in.im
-        const float v = o == 0 ? (p == 0 ? c : -sn) : (p == 0 ? sn : c);
-        r[x] = static_cast<_Float16>(v);
+        r[x] = rotation_entry<true>(k * (j + 8 * (kk >> 1)), 128, o, kk & 1);
     }
     return __builtin_bit_cast(u32x4, r);
 }
@@ -1409,8 +1390,7 @@ __device__ __forceinline__ void put_rows_conj(unsigned* buf, const cpx (&v)[8][4
 template <int kPerCu = 1>  // workgroups per CU (the LDS allows one)
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * kPerCu))) void
 conv2d128_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__ h,
-                      __half2* __restrict__ y, int batch, const float2* __restrict__ tw128,
-                      int tiles_per_block) {
+                      __half2* __restrict__ y, int batch, int tiles_per_block) {
     using namespace conv2dm128;
     constexpr int kImg = 128 * 128;
     __shared__ __align__(16) unsigned buf[2][kBuf];
@@ -1420,7 +1400,7 @@ conv2d128_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__
 
     f16x8 ag[2];
     dft16_operands_grouped<true>(ag, lane);
-    for (int e = tid; e < kOps; e += 512) ops[e] = op_entry(e, tw128);  // read after a barrier below
+    for (int e = tid; e < kOps; e += 512) ops[e] = op_entry(e);  // read after a barrier below
 
     long long img, img_end, step;
     tile_walk(batch, tiles_per_block, img, img_end, step);

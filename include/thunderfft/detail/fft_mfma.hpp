@@ -52,6 +52,28 @@ __device__ __forceinline__ f32x4 mfma16x16x32(f16x8 a, f16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
+// Entry (output part o, input part p; 0 = real, 1 = imaginary) of the real 2 x 2
+// block of a rotation by num / den of a revolution (den a power of two, at
+// least 4; forward: by -num / den).  One hardware cosine, a quarter of a
+// revolution away for the sine: on MI355X its f16 rounding is that of the
+// exact value for every multiple of 1/2048 of a revolution, and the operands
+// cost no memory access.  Read from a table in memory they were 16 gathers per
+// lane and DFT16, and the twiddles (cis_rev now) 20 more in the three-stage
+// kernels, up to 64 lines each: 2 us of a CU's cache per workgroup, which
+// bounded small and ordinary batches.  Half2, in a graph of calls:
+//   C2C N = 4096, 1001 signals: 7.8 against 11.0 us; 16384: 89 against 91
+//   C2C N = 1024, 4003 signals: 7.8 against 8.4 us; 65535: 86.3 against 90
+//   conv1d N = 1024, 4097 signals, one filter: 12.4 against 15.8 us
+//   conv1d N = 4096, 257 signals and filters: 9.6 against 13.5 us
+//   real conv1d N = 4096, 16 channels of 200: 12.5 against 17.1 us
+//   conv2d 64 x 64, 1000 images: 13.7 against 17.9 us
+template <bool FWD>
+__device__ __forceinline__ _Float16 rotation_entry(int num, int den, int o, int p) {
+    const int shift = o == p ? 0 : ((o == 0) == FWD ? -den / 4 : den / 4);
+    return static_cast<_Float16>(__builtin_amdgcn_cosf(
+        static_cast<float>((num + shift) & (den - 1)) / static_cast<float>(den)));
+}
+
 // A-operand registers of the DFT16 matrix for this lane: [half].
 // Row m of half h is output k = m/4 + 4*(2h + (m%4)/2), part (m%4)%2;
 // column k' is input j = k'/2, part k'%2.
@@ -71,13 +93,7 @@ __device__ __forceinline__ void dft16_operands(f16x8 (&a)[2], int lane) {
         for (int e = 0; e < 8; ++e) {
             const int kk = 8 * q + e;
             const int j = kInterleaved ? (kk >> 3) + 4 * ((kk >> 1) & 3) : kk >> 1;
-            const int p = kk & 1;
-            const int ang = (j * k) & 15;
-            const float c = kCos16[ang];
-            const float s = FWD ? -kSin16[ang] : kSin16[ang];
-            // out.re = c*in.re - s*in.im ; out.im = s*in.re + c*in.im
-            const float v = o == 0 ? (p == 0 ? c : -s) : (p == 0 ? s : c);
-            a[h][e] = static_cast<_Float16>(v);
+            a[h][e] = rotation_entry<FWD>(j * k, 16, o, kk & 1);
         }
     }
 }
@@ -98,12 +114,7 @@ __device__ __forceinline__ void dft16_operands_grouped(f16x8 (&a)[2], int lane) 
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int kk = 8 * q + e;
-            const int j = kk >> 1, p = kk & 1;
-            const int ang = (j * k) & 15;
-            const float c = kCos16[ang];
-            const float s = FWD ? -kSin16[ang] : kSin16[ang];
-            const float v = o == 0 ? (p == 0 ? c : -s) : (p == 0 ? s : c);
-            a[h][e] = static_cast<_Float16>(v);
+            a[h][e] = rotation_entry<FWD>((kk >> 1) * k, 16, o, kk & 1);
         }
     }
 }
@@ -180,29 +191,19 @@ struct MfmaPlan {
     }
 };
 
-// Half h of this lane's DFT16 A operand built from the positive-angle table
-// tw of length N = 256 C, with input (column) j of the matrix scaled by
-// W_16C^(j m): entry (k, j) is W_16^(j k) W_16C^(j m) = W_N^(16 j (k C + m)).
-// m = 0 gives the plain DFT16 matrix (the table's values at multiples of N/16
-// are the correctly rounded cos/sin, as the constants of dft16_operands).
-// Row and column order as dft16_operands<FWD, false>.
+// Half h of this lane's DFT16 A operand with input (column) j of the matrix
+// scaled by W_16C^(j m): entry (k, j) is W_16^(j k) W_16C^(j m) =
+// W_16C^(j (k C + m)).  m = 0 gives the plain DFT16 matrix.  Row and column
+// order as dft16_operands<FWD, false>.
 template <bool FWD>
-__device__ __forceinline__ f16x8 dft16_operand_twiddled(int lane, int h, int m, int C,
-                                                        const float2* __restrict__ tw) {
-    const int N = 256 * C;
+__device__ __forceinline__ f16x8 dft16_operand_twiddled(int lane, int h, int m, int C) {
     const int mr = lane & 15, q = lane >> 4;
     const int k = (mr >> 2) + 4 * (2 * h + ((mr & 3) >> 1));
-    const int o = mr & 1;
     f16x8 r;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const int kk = 8 * q + e;
-        const int j = kk >> 1, p = kk & 1;
-        const float2 w = tw[(16 * j * (k * C + m)) & (N - 1)];
-        const float c = w.x, sn = FWD ? -w.y : w.y;
-        // out.re = c*in.re - s*in.im ; out.im = s*in.re + c*in.im
-        const float v = o == 0 ? (p == 0 ? c : -sn) : (p == 0 ? sn : c);
-        r[e] = static_cast<_Float16>(v);
+        r[e] = rotation_entry<FWD>((kk >> 1) * (k * C + m), 16 * C, mr & 1, kk & 1);
     }
     return r;
 }
@@ -251,37 +252,36 @@ struct Stage3Plain {
     }
 };
 
-// Workgroup set-up of the MFMA kernels for direction FWD, from the
-// positive-angle table: this lane's plain DFT16 operands, the step-2 twiddles
+// Workgroup set-up of the MFMA kernels for direction FWD, computed with the
+// hardware sine and cosine (cis_rev, 1e-7): this lane's plain DFT16 operands, the step-2 twiddles
 // W_N^(t*k1) (t = 16c + n, k1 = q + 4r) shared through LDS as
 // w1 = [c][r][lane], and for the stage before the last DFT16 either the
 // folded operands a3 (Stage3Folded; a3 non-null) or this lane's twiddles
 // w2[m - 1] = W_16C^(n m) (Stage3Plain; w2 non-null).  Collective over the
 // kThreads-lane workgroup (ends with a barrier).
 template <int C, bool FWD, int kThreads = 256>
-__device__ __forceinline__ void mfma_setup(f16x8 (&a)[2], cpx* w1, u32x4* a3, cpx* w2,
-                                           const float2* __restrict__ tw) {
+__device__ __forceinline__ void mfma_setup(f16x8 (&a)[2], cpx* w1, u32x4* a3, cpx* w2) {
     using P = MfmaPlan<C>;
     constexpr int N = P::N;
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15;
     dft16_operands<FWD>(a, lane);
     for (int e = tid; e < P::kTw1; e += kThreads) {
         const int l = e & 63, r = (e >> 6) & 3, c = e >> 8;
-        const float2 x = tw[((16 * c + (l & 15)) * ((l >> 4) + 4 * r)) & (N - 1)];
-        w1[e] = FWD ? cpx{x.x, -x.y} : cpx{x.x, x.y};
+        const cpx x = cis_rev((16 * c + (l & 15)) * ((l >> 4) + 4 * r), N);
+        w1[e] = FWD ? cpx{x.re, -x.im} : x;
     }
     if constexpr (C > 1) {
         if (a3) {
             for (int e = tid; e < (C - 1) * 2 * 64; e += kThreads) {
                 const int l = e & 63, h = (e >> 6) & 1, m = 1 + (e >> 7);
-                a3[e] = __builtin_bit_cast(u32x4, dft16_operand_twiddled<FWD>(l, h, m, C, tw));
+                a3[e] = __builtin_bit_cast(u32x4, dft16_operand_twiddled<FWD>(l, h, m, C));
             }
         }
         if (w2) {
 #pragma unroll
             for (int m = 1; m < C; ++m) {
-                const float2 x = tw[(16 * n * m) & (N - 1)];
-                w2[m - 1] = FWD ? cpx{x.x, -x.y} : cpx{x.x, x.y};
+                const cpx x = cis_rev(16 * n * m, N);
+                w2[m - 1] = FWD ? cpx{x.re, -x.im} : x;
             }
         }
     }
@@ -412,12 +412,8 @@ __device__ __forceinline__ f16x4 dft8_mfma_operand(int lane) {
     const int m = i >> 1, o = i & 1;
     f16x4 r;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int c = 2 * q + (e >> 1), p = e & 1;
-        const int ang = (2 * m * c) & 15;  // W_8^(m c) = W_16^(2 m c)
-        const float cs = kCos16[ang], sn = -kSin16[ang];
-        r[e] = static_cast<_Float16>(o == 0 ? (p == 0 ? cs : -sn) : (p == 0 ? sn : cs));
-    }
+    for (int e = 0; e < 4; ++e)
+        r[e] = rotation_entry<true>(m * (2 * q + (e >> 1)), 8, o, e & 1);
     return r;
 }
 
@@ -487,30 +483,6 @@ __device__ __forceinline__ void mfma_fft_staged(unsigned* region, const f16x8 (&
     mfma_steps2to6<C, FWD>(region, w1, s3, lane, y);
 }
 
-// The DFT16 operands of dft16_operands with the entries computed by cis_rev
-// instead of read from the constant table (no memory access; the f16
-// rounding of each entry dominates the transcendental's error).
-template <bool FWD, bool kInterleaved = false>
-__device__ __forceinline__ void dft16_operands_arith(f16x8 (&a)[2], int lane) {
-    const int m = lane & 15, q = lane >> 4;
-    const int gq = m >> 2, i = m & 3;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int k = gq + 4 * (2 * h + (i >> 1));
-        const int o = i & 1;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int kk = 8 * q + e;
-            const int j = kInterleaved ? (kk >> 3) + 4 * ((kk >> 1) & 3) : kk >> 1;
-            const int p = kk & 1;
-            const cpx cs = cis_rev(j * k, 16);
-            const float c = cs.re, s = FWD ? -cs.im : cs.im;
-            const float v = o == 0 ? (p == 0 ? c : -s) : (p == 0 ? s : c);
-            a[h][e] = static_cast<_Float16>(v);
-        }
-    }
-}
-
 // Per-lane coefficients of one direction of the two-stage MFMA transform
 // held in registers (mfma_fft_regs): the stage-1 operands for inputs in the
 // transform's own output layout (a_in, column-permuted), the plain operands,
@@ -557,8 +529,8 @@ struct MfmaCoeffs {
     }
     template <bool FWD>
     __device__ __forceinline__ void build(int lane) {
-        dft16_operands_arith<FWD, true>(a_in, lane);
-        dft16_operands_arith<FWD>(a, lane);
+        dft16_operands<FWD, true>(a_in, lane);
+        dft16_operands<FWD>(a, lane);
         fill<FWD>(lane, [](int k) { return cis_rev(k, N); });
     }
 };
@@ -595,110 +567,14 @@ __device__ __forceinline__ void mfma_fft_regs(unsigned* region, const float2* __
 //   2. twiddle W_N^(t*k1), k1 = q + 4r   3. DFT_C over c (in-lane)
 //   4. twiddle W_16C^(n*m)               5. LDS transpose
 //   6. DFT16 over n -> X[k1 + 16 m + 16C (q' + 4 r')]
-// A wave owns 4/C transforms (C <= 4, 16 values per lane) or one (C = 8,
-// 32 values per lane); a workgroup of 4 waves walks tiles of 4 waves' worth.
-// C <= 4 is held to <= 128 VGPRs (4 waves per SIMD) without spilling.
-template <int C>
-inline constexpr int kMfmaMinWavesPerEU = C <= 4 ? 4 : 1;
-
-template <int C, bool FWD, bool kPrefetch>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMfmaMinWavesPerEU<C>))) void
-c2c_mfma_kernel(const __half2* __restrict__ in,
-                                                       __half2* __restrict__ out, int batch,
-                                                       const float2* __restrict__ tw,
-                                                       int tiles_per_block) {
-    using P = MfmaPlan<C>;
-    constexpr int N = P::N;
-    constexpr int kB = P::kBlocks;
-    constexpr int kRaw = P::kVals / 4;  // 16-byte loads per lane
-    __shared__ unsigned lds[4 * P::kRegion];
-    __shared__ cpx w1[P::kTw1];
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int n = lane & 15, q = lane >> 4;
-    unsigned* region = lds + wave * P::kRegion;
-
-    // The twiddle before the last DFT16 stays an fp32 multiply here: folding
-    // it into LDS-held operands (as the convolutions do) measured slower for
-    // the transform alone (compute pass 29.8 vs 27.8 us at N = 1024).
-    f16x8 a[2];
-    cpx w2[C > 1 ? C - 1 : 1];
-    mfma_setup<C, FWD>(a, w1, nullptr, w2, tw);
-    const Stage3Plain<false> s3{a, w2};
-
-    const long long ntiles = (static_cast<long long>(batch) + P::kFPB - 1) / P::kFPB;
-    long long tile, tile_end, step;
-    tile_walk(ntiles, tiles_per_block, tile, tile_end, step);
-    if (tile >= tile_end) return;  // uniform over the workgroup
-
-    // Valid values (0..kWaveVals) of this wave's kFPW transforms in tile tl.
-    auto valid = [&](long long tl) {
-        const long long v = (static_cast<long long>(batch) - tl * P::kFPB - wave * P::kFPW) * N;
-        return v <= 0 ? 0 : (v >= P::kWaveVals ? P::kWaveVals : static_cast<int>(v));
-    };
-    auto load = [&](u32x4 (&r)[kRaw], long long tl) {
-        const int nv = valid(tl);
-        const __half2* src = in + (tl * P::kFPB + wave * P::kFPW) * N;
-#pragma unroll
-        for (int i = 0; i < kRaw; ++i) {
-            const int e = 4 * lane + 256 * i;
-            r[i] = e < nv ? ld_nt(reinterpret_cast<const u32x4*>(src + e)) : u32x4{};
-        }
-    };
-
-    u32x4 next[kRaw];
-    if constexpr (kPrefetch) load(next, tile);
-    for (; tile < tile_end; tile += step) {
-        u32x4 cur[kRaw];
-        if constexpr (kPrefetch) {
-#pragma unroll
-            for (int i = 0; i < kRaw; ++i) cur[i] = next[i];
-            if (tile + step < tile_end) load(next, tile + step);
-        } else {
-            load(cur, tile);
-        }
-
-        // ---- stage the wave's transforms in LDS (natural order, padded) ----
-        wave_lds_sync();
-#pragma unroll
-        for (int i = 0; i < kRaw; ++i)
-            *reinterpret_cast<u32x4*>(region + P::in_pad(4 * lane + 256 * i)) = cur[i];
-        wave_lds_sync();
-
-        cpx y[kB][4];
-        mfma_fft_staged<C, FWD>(region, a, w1, s3, lane, y);
-        // ---- store: lane (n = k1, q), block (f, m) holds X_f[k1 + 16 m + 16C (q + 4 r)] ----
-        wave_lds_sync();
-#pragma unroll
-        for (int b = 0; b < kB; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                region[P::out_pad((b / C) * N + n + 16 * (b % C) + P::kM * (q + 4 * r))] =
-                    pack_half2(y[b][r]);
-        wave_lds_sync();
-        const int nv = valid(tile);
-        __half2* dst = out + (tile * P::kFPB + wave * P::kFPW) * N;
-#pragma unroll
-        for (int i = 0; i < kRaw; ++i) {
-            const int e = 4 * lane + 256 * i;
-            if (e < nv)
-                st_nt(reinterpret_cast<u32x4*>(dst + e),
-                      *reinterpret_cast<const u32x4*>(region + P::out_pad(e)));
-        }
-    }
-}
-
-}  // namespace thff
-
-namespace thff {
-
-// One-shot form of c2c_mfma_kernel: every wave moves one tile of kFPW
-// transforms and exits, as a streaming copy does (the dispatcher then keeps
-// the CUs evenly fed), with no LDS table and no workgroup barrier: the
-// lane's DFT16 operands come from the constant table and its 16 + (C - 1)
-// twiddles are computed with the hardware sine and cosine (cis_rev, accurate
-// to far below the f16 rounding the data takes), so nothing but the data
-// touches memory.  The wave's loads are issued before the coefficients are
+// One-shot: every wave moves one tile of kFPW transforms and exits, as a
+// streaming copy does (the dispatcher then keeps the CUs evenly fed), with no
+// LDS table and no workgroup barrier: the lane's DFT16 operands and its 16 +
+// (C - 1) twiddles are computed with the hardware sine and cosine (cis_rev,
+// accurate to far below the f16 rounding the data takes), so nothing but the
+// data touches memory.  The twiddle before the last DFT16 stays an fp32
+// multiply: folded into LDS-held operands (as the convolutions do) it measured
+// slower for the transform alone (compute pass 29.8 vs 27.8 us at N = 1024).  The wave's loads are issued before the coefficients are
 // computed.  Grid: one 256-lane workgroup per four tiles.
 template <int C, bool FWD, int kWaves = 4>
 __global__ __launch_bounds__(64 * kWaves) void c2c_mfma_wave_kernel(const __half2* __restrict__ in,
@@ -853,8 +729,8 @@ struct Mfma4096Coeffs {
     }
     template <bool FWD>
     __device__ __forceinline__ void build(int tid) {
-        dft16_operands_arith<FWD>(a, tid & 63);
-        dft16_operands_arith<FWD, true>(a_in, tid & 63);
+        dft16_operands<FWD>(a, tid & 63);
+        dft16_operands<FWD, true>(a_in, tid & 63);
         fill<FWD>(tid, [](int k) { return cis_rev(k, N); });
     }
 };
@@ -928,8 +804,7 @@ __device__ __forceinline__ void mfma4096_fft_regs(unsigned* xbuf, const float2* 
 
 template <bool FWD, bool kPrefetch>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c2c_mfma4096_kernel(
-    const __half2* __restrict__ in, __half2* __restrict__ out, int batch,
-    const float2* __restrict__ tw, int tiles_per_block) {
+    const __half2* __restrict__ in, __half2* __restrict__ out, int batch, int tiles_per_block) {
     using P = Mfma4096;
     constexpr int N = P::N;
     __shared__ __align__(16) unsigned xbuf[P::kExchange];
@@ -938,23 +813,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
     const int wave = tid >> 6, lane = tid & 63;
     const int n = lane & 15, q = lane >> 4;
     unsigned* const region = xbuf + 4 * P::kMatrix * wave;  // matrices k1 = 4 wave ... + 3
-
-    f16x8 a[2];
-    dft16_operands<FWD>(a, lane);
-    // Twiddles: W_4096^(t k1), t = 64 wave + 4 n + b, k1 = q + 4 r; W_4096^(16 n k2), k2 = q + 4 r.
-    cpx w1[4][4], w2[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float2 x = tw[((64 * wave + 4 * n + b) * (q + 4 * r)) & (N - 1)];
-            w1[b][r] = FWD ? cpx{x.x, -x.y} : cpx{x.x, x.y};
-        }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float2 x = tw[(16 * n * (q + 4 * r)) & (N - 1)];
-        w2[r] = FWD ? cpx{x.x, -x.y} : cpx{x.x, x.y};
-    }
 
     // tiles_per_block = 0: the grid is sized to the device and walks the batch
     // grid-stride (tile_walk); otherwise contiguous runs of that many.
@@ -971,6 +829,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
 
     u32x4 next[4];
     if constexpr (kPrefetch) load(next, tile);
+
+    f16x8 a[2];
+    dft16_operands<FWD>(a, lane);
+    // Twiddles: W_4096^(t k1), t = 64 wave + 4 n + b, k1 = q + 4 r; W_4096^(16 n k2), k2 = q + 4 r.
+    cpx w1[4][4], w2[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const cpx x = cis_rev((64 * wave + 4 * n + b) * (q + 4 * r), N);
+            w1[b][r] = FWD ? cpx{x.re, -x.im} : x;
+        }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const cpx x = cis_rev(16 * n * (q + 4 * r), N);
+        w2[r] = FWD ? cpx{x.re, -x.im} : x;
+    }
     for (; tile < tile_end; tile += step) {
         u32x4 cur[4];
         if constexpr (kPrefetch) {
@@ -1090,9 +965,8 @@ struct Mfma2048 {
 // part K % 2); entries of the other sequence's inputs are zero.  With
 // kPermuted the columns follow the device API's N = 2048 fragment order
 // instead: lane group kq of the data operand holds sequence kq % 2's inputs
-// j = 2 c + kq / 2 in its complex slots c = 0..3.  kArith computes the
-// entries with cis_rev instead of reading the constant table.
-template <bool FWD, bool kPermuted = false, bool kArith = false>
+// j = 2 c + kq / 2 in its complex slots c = 0..3.
+template <bool FWD, bool kPermuted = false>
 __device__ __forceinline__ void dft8_pair_operands(f16x8 (&a)[2], int lane) {
     const int m = lane & 15, kq = lane >> 4;
     const int k1 = m >> 1, o = m & 1;
@@ -1103,26 +977,14 @@ __device__ __forceinline__ void dft8_pair_operands(f16x8 (&a)[2], int lane) {
             const int slot = e >> 1, p = e & 1;
             const int seq = kPermuted ? (kq & 1) : kq >> 1;
             const int j = kPermuted ? 2 * slot + (kq >> 1) : 4 * (kq & 1) + slot;
-            const int ang = (2 * j * k1) & 15;  // W_8^(j k1) = W_16^(2 j k1)
-            float c, s;
-            if constexpr (kArith) {
-                const cpx cs = cis_rev(ang, 16);
-                c = cs.re;
-                s = FWD ? -cs.im : cs.im;
-            } else {
-                c = kCos16[ang];
-                s = FWD ? -kSin16[ang] : kSin16[ang];
-            }
-            const float v = o == 0 ? (p == 0 ? c : -s) : (p == 0 ? s : c);
-            a[h][e] = static_cast<_Float16>(seq == h ? v : 0.0f);
+            a[h][e] = seq == h ? rotation_entry<FWD>(j * k1, 8, o, p) : static_cast<_Float16>(0.0f);
         }
     }
 }
 
 template <bool FWD, bool kPrefetch>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c2c_mfma2048_kernel(
-    const __half2* __restrict__ in, __half2* __restrict__ out, int batch,
-    const float2* __restrict__ tw, int tiles_per_block) {
+    const __half2* __restrict__ in, __half2* __restrict__ out, int batch, int tiles_per_block) {
     using P = Mfma2048;
     constexpr int N = P::N;
     __shared__ __align__(16) unsigned xbuf[P::kExchange];
@@ -1132,26 +994,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
     const int n = lane & 15, q = lane >> 4;
     const int f = wave >> 1;  // this wave's transform within the tile (stage 1)
     unsigned* const region = xbuf + 4 * P::kMatrix * wave;
-
-    f16x8 a8[2], a[2];
-    dft8_pair_operands<FWD>(a8, lane);
-    dft16_operands<FWD>(a, lane);
-    // Twiddles: W_2048^(t k1), t = 128 (w & 1) + 64 H + 4 n + b, k1 = 2 q + i
-    // (r = 2 H + i); W_256^(t0 k2) = W_2048^(8 n k2), k2 = q + 4 r.
-    cpx w1[4][4], w2[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int t = 128 * (wave & 1) + 64 * (r >> 1) + 4 * n + b, k1 = 2 * q + (r & 1);
-            const float2 x = tw[(t * k1) & (N - 1)];
-            w1[b][r] = FWD ? cpx{x.x, -x.y} : cpx{x.x, x.y};
-        }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float2 x = tw[(8 * n * (q + 4 * r)) & (N - 1)];
-        w2[r] = FWD ? cpx{x.x, -x.y} : cpx{x.x, x.y};
-    }
 
     const long long ntiles = (static_cast<long long>(batch) + 1) / 2;
     long long tile, tile_end, step;
@@ -1171,6 +1013,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
 
     u32x4 next[4];
     if constexpr (kPrefetch) load(next, tile);
+
+    f16x8 a8[2], a[2];
+    dft8_pair_operands<FWD>(a8, lane);
+    dft16_operands<FWD>(a, lane);
+    // Twiddles: W_2048^(t k1), t = 128 (w & 1) + 64 H + 4 n + b, k1 = 2 q + i
+    // (r = 2 H + i); W_256^(t0 k2) = W_2048^(8 n k2), k2 = q + 4 r.
+    cpx w1[4][4], w2[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = 128 * (wave & 1) + 64 * (r >> 1) + 4 * n + b, k1 = 2 * q + (r & 1);
+            const cpx x = cis_rev(t * k1, N);
+            w1[b][r] = FWD ? cpx{x.re, -x.im} : x;
+        }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const cpx x = cis_rev(8 * n * (q + 4 * r), N);
+        w2[r] = FWD ? cpx{x.re, -x.im} : x;
+    }
     for (; tile < tile_end; tile += step) {
         u32x4 cur[4];
         if constexpr (kPrefetch) {
@@ -1291,8 +1153,8 @@ struct Mfma2048Coeffs {
     }
     template <bool FWD>
     __device__ __forceinline__ void build(int tid) {
-        dft8_pair_operands<FWD, true, true>(a8, tid & 63);
-        dft16_operands_arith<FWD>(a, tid & 63);
+        dft8_pair_operands<FWD, true>(a8, tid & 63);
+        dft16_operands<FWD>(a, tid & 63);
         fill<FWD>(tid, [](int k) { return cis_rev(k, N); });
     }
 };
@@ -1406,8 +1268,7 @@ struct Mfma128 {
 
 template <bool FWD, bool kPrefetch>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c2c_mfma128_kernel(
-    const __half2* __restrict__ in, __half2* __restrict__ out, int batch,
-    const float2* __restrict__ tw, int tiles_per_block) {
+    const __half2* __restrict__ in, __half2* __restrict__ out, int batch, int tiles_per_block) {
     using P = Mfma128;
     constexpr int N = P::N;
     __shared__ __align__(16) unsigned lds[4 * P::kRegion];
@@ -1415,16 +1276,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
     const int wave = tid >> 6, lane = tid & 63;
     const int n = lane & 15, q = lane >> 4;
     unsigned* const region = lds + wave * P::kRegion;
-
-    f16x8 a[2], a8[2];
-    dft16_operands<FWD>(a, lane);
-    dft8_pair_operands<FWD>(a8, lane);
-    cpx w1[4];  // W_128^(t k1), t = n % 8, k1 = q + 4 r
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float2 x = tw[((n & 7) * (q + 4 * r)) & (N - 1)];
-        w1[r] = FWD ? cpx{x.x, -x.y} : cpx{x.x, x.y};
-    }
 
     const long long ntiles = (static_cast<long long>(batch) + P::kFPB - 1) / P::kFPB;
     long long tile, tile_end, step;
@@ -1448,6 +1299,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
 
     u32x4 next[4];
     if constexpr (kPrefetch) load(next, tile);
+
+    f16x8 a[2], a8[2];
+    dft16_operands<FWD>(a, lane);
+    dft8_pair_operands<FWD>(a8, lane);
+    cpx w1[4];  // W_128^(t k1), t = n % 8, k1 = q + 4 r
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const cpx x = cis_rev((n & 7) * (q + 4 * r), N);
+        w1[r] = FWD ? cpx{x.re, -x.im} : x;
+    }
     for (; tile < tile_end; tile += step) {
         u32x4 cur[4];
         if constexpr (kPrefetch) {

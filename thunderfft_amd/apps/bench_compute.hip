@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) void repeat_mfma(const __half2* in, __half2* o
     unsigned* region = lds + wave * P::kRegion;
     f16x8 a[2];
     cpx w2[C > 1 ? C - 1 : 1];
-    mfma_setup<C, true>(a, w1, nullptr, w2, tw);
+    mfma_setup<C, true>(a, w1, nullptr, w2);
     const Stage3Plain<false> s3{a, w2};
     const long long first = static_cast<long long>(blockIdx.x) * P::kFPB + wave * P::kFPW;
     const bool valid = first + P::kFPW <= batch;

@@ -54,14 +54,10 @@ inline Grid make_grid(long long ntiles, int per_cu, int num_cus) {
 //   fp16 N = 128 (MFMA, c2c_mfma128_kernel): 2 per CU with prefetch 87.3 us,
 //     against 90.0 at 3 per CU, 99.5 with one tile per workgroup and 90.3-91.1
 //     for the VALU kernel (one tile per workgroup; device grids 93).
-//   fp16 N = 256 ... 1024: the one-shot kernel (kHalfOneShot below), whose
-//     shape is fixed there.  Before it, with the table-based kernel: N = 256
-//     one tile per workgroup, 86.0-88.7 us wherever the output lies; the
-//     2-per-CU grid-stride walk with prefetch as fast only for some output
-//     placements (86.3-103 us over 12 offsets of y from x, one box); N = 512,
-//     1024 on the walk (one tile per workgroup took 98-114 us for them, the
-//     per-tile table set-up included).
-//   fp16 MFMA (the walk): 2 per CU with prefetch, 86-91 us.  Runs
+//   fp16 N = 256 ... 1024: the one-shot kernel (below), whose shape is fixed there.
+//   fp16 N = 4096 (the walk): 2 per CU with prefetch, 89 us; 3 per CU is
+//     ahead by up to 10% for 1000 to 2000 transforms (13.1 against 14.5 us)
+//     and 8% behind for 16384.  Runs
 //     of contiguous tiles per workgroup, which leave the balancing to the
 //     dispatcher, are slower: 2 tiles 87-98 us, 4-32 tiles 93-110 us (the
 //     grid-stride walk keeps all workgroups on neighbouring tiles).
@@ -82,8 +78,7 @@ constexpr LaunchShape launch_shape(int precision) {
         return N <= 1024 ? LaunchShape{0, false, N == 256 || N == 512}
                          : LaunchShape{16, true, true};
     if (N == 128) return {2, true};
-    if (N <= 128 || N == 256) return {0, false};
-    return {2, true};
+    return N == 64 ? LaunchShape{0, false} : LaunchShape{2, true};
 }
 
 // half2 lengths whose radix-16 stages run on MFMA (fft_mfma.hpp): N = 256*C
@@ -105,59 +100,40 @@ void enqueue(Grid g, const IO* x, IO* y, int batch, const float2* tw, hipStream_
 }
 
 // fp16 N = 256 ... 1024 run the one-shot kernel (c2c_mfma_wave_kernel: one
-// tile per wave, the wave's twiddles computed in the kernel, no LDS table,
-// no workgroup barrier) instead of the persistent 2-per-CU grid-stride
-// kernel (c2c_mfma_kernel, whose workgroups build LDS tables once and walk
-// many tiles).  2^26 values, same output buffer, alternating (MI355X):
-// N = 1024 86.6-87.0 against 88.4-89.1 us, 512 86.4-87.0 against 86.8-87.6,
-// 256 85.7-86.4 against 86.5-87.6; over 8 output placements (bench.py's
-// placement leg) 86.9-88.4 us against 90.0-102.0 us at N = 1024: the
-// dispatcher keeps the CUs evenly fed, as for a streaming copy, and the
-// time no longer depends on where the output lies.  Workgroups of 1 or 2
-// such waves: 86.4-87.0 and 87.1-87.2 us at N = 1024, slower at 256 and 512.
-// The three-stage kernels (N = 2048, 4096) as one tile per workgroup with
-// computed twiddles took 128.3-128.8 and 94.7-95.1 us against 89.3-89.9 and
-// 89.5-89.9 us, so they keep the persistent walk.
-template <int N>
-inline constexpr bool kHalfOneShot = N >= 256 && N <= 1024;
+// tile per wave, its coefficients computed, no LDS table, no workgroup
+// barrier).  Against a persistent 2-per-CU grid-stride kernel with LDS
+// tables: N = 1024 86.6-87.0 against 88.4-89.1 us for 2^26 values, and
+// 86.9-88.4 us over 8 output placements (bench.py's placement leg) against
+// 90.0-102.0: the dispatcher keeps the CUs evenly fed, as for a streaming
+// copy, and the time does not depend on where the output lies.  Workgroups
+// of 1 or 2 such waves: 86.4-87.0 and 87.1-87.2 us at N = 1024, slower at 256
+// and 512.  One tile per workgroup for the three-stage kernels (N = 2048,
+// 4096) takes 118 and 96.6 us against 91.2 and 88.9 us for the walk.
 inline constexpr int kHalfOneShotWaves = 4;  // waves (tiles) per workgroup
 
 template <int N, bool FWD>
-void enqueue_mfma(Grid g, const __half2* x, __half2* y, int batch, const float2* tw,
-                  hipStream_t stream) {
-    if constexpr (kHalfOneShot<N>) {
-        constexpr int kW = kHalfOneShotWaves;
-        constexpr long long kPerBlock = static_cast<long long>(kW) * MfmaPlan<N / 256>::kFPW;
-        const long long blocks = (static_cast<long long>(batch) + kPerBlock - 1) / kPerBlock;
-        if (blocks <= 0) return;
-        c2c_mfma_wave_kernel<N / 256, FWD, kW><<<static_cast<unsigned>(blocks), 64 * kW, 0, stream>>>(
-            x, y, batch);
-        (void)g;
-        (void)tw;
-    } else {
-        constexpr bool kPf = launch_shape<N>(1).prefetch;
-        c2c_mfma_kernel<N / 256, FWD, kPf><<<g.blocks, 256, 0, stream>>>(x, y, batch, tw,
-                                                                         g.tiles_per_block);
-    }
+void enqueue_mfma(const __half2* x, __half2* y, int batch, hipStream_t stream) {
+    constexpr int kW = kHalfOneShotWaves;
+    constexpr long long kPerBlock = static_cast<long long>(kW) * MfmaPlan<N / 256>::kFPW;
+    const long long blocks = (static_cast<long long>(batch) + kPerBlock - 1) / kPerBlock;
+    if (blocks <= 0) return;
+    c2c_mfma_wave_kernel<N / 256, FWD, kW><<<static_cast<unsigned>(blocks), 64 * kW, 0, stream>>>(
+        x, y, batch);
 }
 
 template <bool FWD>
-void enqueue_mfma128(Grid g, const __half2* x, __half2* y, int batch, const float2* tw,
-                     hipStream_t stream) {
+void enqueue_mfma128(Grid g, const __half2* x, __half2* y, int batch, hipStream_t stream) {
     constexpr bool kPf = launch_shape<128>(1).prefetch;
-    c2c_mfma128_kernel<FWD, kPf><<<g.blocks, 256, 0, stream>>>(x, y, batch, tw, g.tiles_per_block);
+    c2c_mfma128_kernel<FWD, kPf><<<g.blocks, 256, 0, stream>>>(x, y, batch, g.tiles_per_block);
 }
 
 template <int N, bool FWD>
-void enqueue_mfma3(Grid g, const __half2* x, __half2* y, int batch, const float2* tw,
-                   hipStream_t stream) {
+void enqueue_mfma3(Grid g, const __half2* x, __half2* y, int batch, hipStream_t stream) {
     constexpr bool kPf = launch_shape<N>(1).prefetch;
     if constexpr (N == 2048)
-        c2c_mfma2048_kernel<FWD, kPf><<<g.blocks, 256, 0, stream>>>(x, y, batch, tw,
-                                                                    g.tiles_per_block);
+        c2c_mfma2048_kernel<FWD, kPf><<<g.blocks, 256, 0, stream>>>(x, y, batch, g.tiles_per_block);
     else
-        c2c_mfma4096_kernel<FWD, kPf><<<g.blocks, 256, 0, stream>>>(x, y, batch, tw,
-                                                                    g.tiles_per_block);
+        c2c_mfma4096_kernel<FWD, kPf><<<g.blocks, 256, 0, stream>>>(x, y, batch, g.tiles_per_block);
 }
 
 // Buffers that are element-aligned but not 16-byte aligned (any vec2_t<T>
@@ -206,19 +182,19 @@ hipError_t launch_c2c(int precision, bool forward, bool aligned16, const void* i
         auto* y = static_cast<__half2*>(out);
         if constexpr (kHalfOnMfma<N>) {
             if (forward)
-                enqueue_mfma<N, true>(g, x, y, batch, tw, stream);
+                enqueue_mfma<N, true>(x, y, batch, stream);
             else
-                enqueue_mfma<N, false>(g, x, y, batch, tw, stream);
+                enqueue_mfma<N, false>(x, y, batch, stream);
         } else if constexpr (kHalfOnMfma3<N>) {
             if (forward)
-                enqueue_mfma3<N, true>(g, x, y, batch, tw, stream);
+                enqueue_mfma3<N, true>(g, x, y, batch, stream);
             else
-                enqueue_mfma3<N, false>(g, x, y, batch, tw, stream);
+                enqueue_mfma3<N, false>(g, x, y, batch, stream);
         } else if constexpr (kHalfOnMfma128<N>) {
             if (forward)
-                enqueue_mfma128<true>(g, x, y, batch, tw, stream);
+                enqueue_mfma128<true>(g, x, y, batch, stream);
             else
-                enqueue_mfma128<false>(g, x, y, batch, tw, stream);
+                enqueue_mfma128<false>(g, x, y, batch, stream);
         } else if (forward) {
             enqueue<__half2, N, true>(g, x, y, batch, tw, stream);
         } else {
@@ -293,10 +269,10 @@ hipError_t launch_conv1d(int precision, bool per_signal_filter, const void* x, c
             const auto* hh = static_cast<const __half2*>(h);
             auto* yy = static_cast<__half2*>(y);
             if (per_signal_filter)
-                conv1d_mfma_kernel<C, true><<<g.blocks, 256, 0, stream>>>(xx, hh, yy, batch, tw,
+                conv1d_mfma_kernel<C, true><<<g.blocks, 256, 0, stream>>>(xx, hh, yy, batch,
                                                                           g.tiles_per_block);
             else
-                conv1d_mfma_kernel<C, false><<<g.blocks, 256, 0, stream>>>(xx, hh, yy, batch, tw,
+                conv1d_mfma_kernel<C, false><<<g.blocks, 256, 0, stream>>>(xx, hh, yy, batch,
                                                                            g.tiles_per_block);
             return hipGetLastError();
         }
@@ -313,10 +289,9 @@ hipError_t launch_conv1d(int precision, bool per_signal_filter, const void* x, c
             const auto* hh = static_cast<const __half2*>(h);
             auto* yy = static_cast<__half2*>(y);
             if (per_signal_filter)
-                conv1d_mfma4096_kernel<N, true><<<g.blocks, 256, 0, stream>>>(xx, hh, yy, batch, tw);
+                conv1d_mfma4096_kernel<N, true><<<g.blocks, 256, 0, stream>>>(xx, hh, yy, batch);
             else
-                conv1d_mfma4096_kernel<N, false><<<g.blocks, 256, 0, stream>>>(xx, hh, yy, batch,
-                                                                               tw);
+                conv1d_mfma4096_kernel<N, false><<<g.blocks, 256, 0, stream>>>(xx, hh, yy, batch);
             return hipGetLastError();
         }
     }
@@ -352,22 +327,22 @@ hipError_t launch_conv1d_real(int precision, const void* x, const float2* spectr
     const long long transforms = (static_cast<long long>(batch) + 1) / 2 * channels;
     // fp16 N = 256 ... 2048: both transforms on MFMA (fft_conv_mfma.hpp);
     // measured against this VALU path at 2^26 samples: 61 vs 68 us (N=256),
-    // 60 vs 87 (512), 64 vs 87 (1024).  Grid: the occupancy (2 workgroups per
-    // CU for N = 256 and 2048, else 3); up to N = 1024 the channels' spectra
+    // 60 vs 87 (512), 64 vs 87 (1024).  Grid: the occupancy, 3 workgroups per
+    // CU (N = 256: 51.5 against 57.0 us for 2), 2 for N = 2048; up to N = 1024 the channels' spectra
     // stay in registers (5-9% over reloading them per tile).
     if constexpr (N >= 256 && N <= 2048) {
         if (precision != 0) {
             using M = MfmaPlan<N / 256>;
             const long long ntiles = (transforms + M::kFPB - 1) / M::kFPB;
-            const Grid g = make_grid(ntiles, N == 256 || N == 2048 ? 2 : 3, num_cus);
+            const Grid g = make_grid(ntiles, N == 2048 ? 2 : 3, num_cus);
             if (real_buffer_fits<N / 256>(channels))
                 conv1d_real_mfma_kernel<N / 256, true><<<g.blocks, 256, 0, stream>>>(
                     static_cast<const __half*>(x), spectrum, static_cast<__half*>(y), batch,
-                    channels, tw, g.tiles_per_block);
+                    channels, g.tiles_per_block);
             else
                 conv1d_real_mfma_kernel<N / 256, false><<<g.blocks, 256, 0, stream>>>(
                     static_cast<const __half*>(x), spectrum, static_cast<__half*>(y), batch,
-                    channels, tw, g.tiles_per_block);
+                    channels, g.tiles_per_block);
             return hipGetLastError();
         }
     }
@@ -380,11 +355,11 @@ hipError_t launch_conv1d_real(int precision, const void* x, const float2* spectr
             if (channels <= kReal4096BufferMaxChannels)
                 conv1d_real_mfma4096_kernel<N, true><<<g.blocks, 256, 0, stream>>>(
                     static_cast<const __half*>(x), spectrum, static_cast<__half*>(y), batch,
-                    channels, tw, g.tiles_per_block);
+                    channels, g.tiles_per_block);
             else
                 conv1d_real_mfma4096_kernel<N, false><<<g.blocks, 256, 0, stream>>>(
                     static_cast<const __half*>(x), spectrum, static_cast<__half*>(y), batch,
-                    channels, tw, g.tiles_per_block);
+                    channels, g.tiles_per_block);
             return hipGetLastError();
         }
     }
@@ -451,7 +426,7 @@ hipError_t launch_conv2d64(int precision, const void* x, const void* h, void* y,
         const Grid g = make_grid(batch, kConv2dMfmaPerCu, num_cus);
         conv2d64_mfma_kernel<kConv2dMfmaPerCu><<<g.blocks, 256, 0, stream>>>(
             static_cast<const __half2*>(x), static_cast<const __half2*>(h),
-            static_cast<__half2*>(y), batch, tw, g.tiles_per_block);
+            static_cast<__half2*>(y), batch, g.tiles_per_block);
     }
     return hipGetLastError();
 }
@@ -472,7 +447,7 @@ hipError_t launch_conv2d128(int precision, const void* x, const void* h, void* y
     else
         conv2d128_mfma_kernel<1><<<g.blocks, 512, 0, stream>>>(
             static_cast<const __half2*>(x), static_cast<const __half2*>(h),
-            static_cast<__half2*>(y), batch, tw, g.tiles_per_block);
+            static_cast<__half2*>(y), batch, g.tiles_per_block);
     return hipGetLastError();
 }
 #endif
