@@ -641,6 +641,9 @@ struct RealIo<__half2> {
 // (row pair p, channel d) on a tile walk whose successive tiles are `adv`
 // transforms apart: positions advance without a 64-bit division per tile,
 // and transform tau + k (k small) is located with one 32-bit division.
+// (All divisions are of 32 bits: one launch holds at most 2^24 tiles of 64
+// transforms, and a 64-bit division takes about 150 instructions, four of
+// which stood before a workgroup's first load.)
 struct ChannelPos {
     long long p;
     int d;
@@ -650,12 +653,14 @@ struct ChannelWalk {
     int adv_d;
     int channels;
     __host__ __device__ __forceinline__ ChannelWalk(long long adv, int ch) : channels(ch) {
-        adv_p = adv / ch;
-        adv_d = static_cast<int>(adv - adv_p * ch);
+        const ChannelPos a = at(adv);
+        adv_p = a.p;
+        adv_d = a.d;
     }
     __host__ __device__ __forceinline__ ChannelPos at(long long tau) const {
-        const long long p = tau / channels;
-        return {p, static_cast<int>(tau - p * channels)};
+        const unsigned t = static_cast<unsigned>(tau), c = static_cast<unsigned>(channels);
+        const unsigned p = t / c;
+        return {p, static_cast<int>(t - p * c)};
     }
     // (adv_d < channels and q.d < channels: at most one carry)
     __host__ __device__ __forceinline__ ChannelPos advance(ChannelPos q) const {
@@ -737,6 +742,12 @@ __global__ __launch_bounds__(256) void conv1d_real_kernel(
     // already): the channel's spectrum stays in registers while the channel
     // does not change, instead of being read from L2 per tile.
     constexpr bool kKeepSpectrum = N == 4096;
+    // The others load it per tile, with a prefetch (fp32, 2 waves per SIMD) in
+    // flight during the forward transform: N = 2048 112.5 against 121 us, 1024
+    // 108 against 113, 64 and 128 96-97 against 99-100 us (2^26 samples, 16
+    // channels); without one (half2 N = 64, 128, 4 waves) after it, 10.3
+    // against 11.8 us for 2^22.6 samples of N = 128.
+    constexpr bool kEarlySpectrum = !kKeepSpectrum && kPf != Prefetch::kNone;
     int spec_d = -1;
     cpx spec[kKeepSpectrum ? 16 : 1];
 
@@ -828,12 +839,23 @@ __global__ __launch_bounds__(256) void conv1d_real_kernel(
     RowsT next;
     if constexpr (kPf != Prefetch::kNone)
         if (tile < tile_end) fetch_any(tile, pos, next);
-
     for (; tile < tile_end; tile += step) {
-        // ---- both rows of each transform -> (re, im) = (row 0, row 1) ----
-        RowsT cur;
         const Pos at = pos;
         pos = advance(pos);
+        // The spectrum of the tile's channel (a channel past the last
+        // transform too: always a valid spectrum row).
+        long long pair_f;
+        int d;
+        locate(at, f, pair_f, d);
+        float2 hk[kKeepSpectrum ? 1 : 16];
+        auto load_bins = [&]() {
+            const float2* hs = spectrum + static_cast<long long>(d) * N + t;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) hk[j] = hs[j * P::kTPF];
+        };
+        if constexpr (kEarlySpectrum) load_bins();
+        // ---- both rows of each transform -> (re, im) = (row 0, row 1) ----
+        RowsT cur;
         if constexpr (kPf == Prefetch::kEarly) {
             cur = next;
             if (tile + step < tile_end) fetch_any(tile + step, pos, next);
@@ -869,30 +891,23 @@ __global__ __launch_bounds__(256) void conv1d_real_kernel(
         }
 
         // ---- FFT, product with the channel's spectrum, inverse FFT ----
-        // (a channel past the last transform too: always a valid spectrum row)
-        long long pair_f;
-        int d;
-        locate(at, f, pair_f, d);
         fft_registers<N, true>(v, slot, t, w);
         if constexpr (kKeepSpectrum) {
             if (d != spec_d) {
                 const float2* hs = spectrum + static_cast<long long>(d) * N + t;
 #pragma unroll
                 for (int j = 0; j < 16; ++j) {
-                    const float2 hk = hs[j * P::kTPF];
-                    spec[j] = cpx{hk.x, hk.y};
+                    const float2 x = hs[j * P::kTPF];
+                    spec[j] = cpx{x.x, x.y};
                 }
                 spec_d = d;
             }
 #pragma unroll
             for (int j = 0; j < 16; ++j) v[j] = cmul(v[j], spec[j]);
         } else {
-            const float2* hs = spectrum + static_cast<long long>(d) * N + t;
+            if constexpr (!kEarlySpectrum) load_bins();
 #pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const float2 hk = hs[j * P::kTPF];
-                v[j] = cmul(v[j], cpx{hk.x, hk.y});
-            }
+            for (int j = 0; j < 16; ++j) v[j] = cmul(v[j], cpx{hk[j].x, hk[j].y});
         }
         if constexpr (kPf == Prefetch::kLate)
             if (tile + step < tile_end) fetch_any(tile + step, pos, next);

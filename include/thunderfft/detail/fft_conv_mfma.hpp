@@ -204,6 +204,27 @@ conv1d_real_mfma_kernel(const __half* __restrict__ x, const float2* __restrict__
                 r1[i] = base1[i] >= 0 ? ld_nt(reinterpret_cast<const u32x4*>(x + base1[i])) : u32x4{};
             }
         }
+        // The spectra of the wave's transforms stay in registers while their
+        // channels do not change: they are chan[0] + f mod D, so chan[0]
+        // decides, and on a grid-stride walk whose stride in transforms is a
+        // multiple of D it never changes.  Loaded here, beside the rows, a
+        // workgroup's first tile waits for memory once.
+        if constexpr (kKeepSpectra) {
+            if (chan[0] != spec_d) {
+#pragma unroll
+                for (int b = 0; b < kB; ++b) {
+                    const float2* hs = spectrum + static_cast<long long>(chan[b / C]) * N + n +
+                                       16 * (b % C) + P::kM * q;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float2 hk = hs[P::kM * 4 * r];
+                        spec[b][r] = cpx{hk.x, hk.y};
+                    }
+                }
+                spec_d = chan[0];
+                wait_vmem_all();  // on this rarely taken path, not after the branch
+            }
+        }
         wave_lds_sync();  // the previous tile's output reads are done
 #pragma unroll
         for (int i = 0; i < kSteps; ++i) {
@@ -219,24 +240,7 @@ conv1d_real_mfma_kernel(const __half* __restrict__ x, const float2* __restrict__
         mfma_stage1_lds<C>(region, a, lane, v);
         mfma_steps2to6<C, true>(region, w1, s3, lane, v);
         // ---- product: block (f, m), lane (n, q): bin k = n + 16 m + 16C (q + 4 r) ----
-        // The spectra of the wave's transforms stay in registers while their
-        // channels do not change: they are chan[0] + f mod D, so chan[0]
-        // decides, and on a grid-stride walk whose stride in transforms is a
-        // multiple of D it never changes.
         if constexpr (kKeepSpectra) {
-            if (chan[0] != spec_d) {
-#pragma unroll
-                for (int b = 0; b < kB; ++b) {
-                    const float2* hs = spectrum + static_cast<long long>(chan[b / C]) * N + n +
-                                       16 * (b % C) + P::kM * q;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float2 hk = hs[P::kM * 4 * r];
-                        spec[b][r] = cpx{hk.x, hk.y};
-                    }
-                }
-                spec_d = chan[0];
-            }
 #pragma unroll
             for (int b = 0; b < kB; ++b)
 #pragma unroll
@@ -367,6 +371,14 @@ conv1d_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__ h,
         steps(v);
     };
 
+    auto offset = [&](long long tl) { return (tl * P::kFPB + wave * P::kFPW) * N; };
+    // A shared filter at C <= 4: the next tile's signal loads are issued as
+    // soon as the current one is staged (its registers are free then), the
+    // first's beside the filter's; 1-3% faster at 2^25 values
+    // (at C = 8 the registers are not there).
+    constexpr bool kPrefetchShared = !kPerSignal && C <= 4;
+    u32x4 rn[kRaw];
+
     unsigned hp[kB][4];  // FFT(h), packed half2
     auto keep = [&](const cpx (&v)[kB][4]) {
 #pragma unroll
@@ -377,20 +389,17 @@ conv1d_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__ h,
     if constexpr (!kPerSignal) {
         // Every transform of the wave is the shared filter: stage it kFPW times.
         cpx v[kB][4];
-        wave_lds_sync();
+        u32x4 rh[kRaw];
 #pragma unroll
-        for (int i = 0; i < kRaw; ++i) {
-            const int e = 4 * lane + 256 * i;
-            *reinterpret_cast<u32x4*>(region + P::in_pad(e)) =
-                ld_nt(reinterpret_cast<const u32x4*>(h + e % N));
-        }
-        wave_lds_sync();
+        for (int i = 0; i < kRaw; ++i)
+            rh[i] = ld_nt(reinterpret_cast<const u32x4*>(h + (4 * lane + 256 * i) % N));
+        if constexpr (kPrefetchShared) load(x + offset(tile), tile < tile_end ? valid(tile) : 0, rn);
+        stage(rh);
         mfma_stage1_lds<C>(region, a, lane, v);
         steps(v);
         keep(v);
     }
 
-    auto offset = [&](long long tl) { return (tl * P::kFPB + wave * P::kFPW) * N; };
     // Per-signal filters at C <= 4: the loads run a transform ahead of their
     // use, in registers that are free at that point -- the signal's while the
     // filter is transformed (its packed spectrum is not live yet), the next
@@ -400,14 +409,8 @@ conv1d_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__ h,
     // 92-94 us for 16384 x 2048, same 8-byte spill); loading the next filter
     // during the inverse as well spills 44 bytes per lane (97 us).
     constexpr bool kPipelined = kPerSignal && C <= 4;
-    // A shared filter at C <= 4: the next tile's signal loads are issued as
-    // soon as the current one is staged (its registers are free then); 1-3%
-    // faster at 2^25 values (at C = 8 the registers are not there).
-    constexpr bool kPrefetchShared = !kPerSignal && C <= 4;
     u32x4 rh[kRaw];
     if constexpr (kPipelined) load(h + offset(tile), tile < tile_end ? valid(tile) : 0, rh);
-    u32x4 rn[kRaw];
-    if constexpr (kPrefetchShared) load(x + offset(tile), tile < tile_end ? valid(tile) : 0, rn);
     // At N = 2048 a wave's issue priority falls as its workgroup gets ahead
     // (ProgressPriority): 63.5 against 66-67 us (shared filter) and 91.0
     // against 91.7-92.0 us (per-signal) at 2^25 values; neutral at N <= 1024.
@@ -680,10 +683,22 @@ conv1d_real_mfma4096_kernel(const __half* __restrict__ x, const float2* __restri
             }
         }
     };
+    auto load_spectrum = [&](long long d) {
+        const float2* hs = spectrum + d * N + 4 * wave + 16 * n + 256 * q;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float2 hk = hs[b + 1024 * r];
+                spec[b][r] = cpx{hk.x, -hk.y};  // conj(H)
+            }
+        spec_d = d;
+    };
     u32x4 next[4];
     if constexpr (kBufferIO) {
         if (tile >= tile_end) return;  // uniform over the workgroup
         load(pos, next);
+        load_spectrum(pos.d);  // in flight with the first rows
         // Four stores to a resource of no bytes (dropped by the range check):
         // the loop is then entered, like every later pass, with the pieces
         // followed by four stores in flight, so the compiler's count at the
@@ -742,19 +757,11 @@ conv1d_real_mfma4096_kernel(const __half* __restrict__ x, const float2* __restri
         stages23(v);
         // ---- product: bin k = 4 w + b + 16 n + 256 (q + 4 r) ----
         if (d != spec_d) {  // uniform: a new channel's spectrum
-            const float2* hs = spectrum + d * N + 4 * wave + 16 * n + 256 * q;
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float2 hk = hs[b + 1024 * r];
-                    spec[b][r] = cpx{hk.x, -hk.y};  // conj(H)
-                }
+            load_spectrum(d);
             // Wait here, on this rarely taken path: a wait after the branch
             // would have to count these loads as the latest ones and so
             // would also wait for the next tile's pieces on every tile.
             wait_vmem_all();
-            spec_d = d;
         }
         // ---- inverse stage 1 from the registers: the forward DFT16 over k3
         // of conj(Z H) = conj(Z conj(G)), G = conj(H) held in spec, sequences
@@ -935,9 +942,9 @@ conv1d_mfma4096_kernel(const __half2* __restrict__ x, const __half2* __restrict_
         cpx v[4][4];
         u32x4 zh[4];
         load(h, zh);
+        load(x + tile * N, zx);
         forward(zh, v);
         keep(v);
-        load(x + tile * N, zx);
     }
     // A wave's issue priority falls as its workgroup gets ahead of the others
     // (ProgressPriority): 95 against 99-101 us (per-signal) and 65 against
@@ -948,11 +955,11 @@ conv1d_mfma4096_kernel(const __half2* __restrict__ x, const __half2* __restrict_
         priority.set(left);
         cpx v[4][4];
         if constexpr (kPerSignal) {
-            u32x4 z[4];
-            load(h + tile * N, z);
-            forward(z, v);
-            keep(v);
+            u32x4 zh[4], z[4];
+            load(h + tile * N, zh);
             load(x + tile * N, z);
+            forward(zh, v);
+            keep(v);
             forward(z, v);
         } else {
             u32x4 z[4];
