@@ -204,3 +204,69 @@ def test_initialize_races_transforms_on_another_thread():
     d_y = torch.empty_like(d_x)
     thff.ThunderFFT_global("float", n, True, d_x, d_y, batch)
     assert torch.equal(d_y, d_ref)
+
+
+def test_conv2d_workspaces_on_many_streams_and_threads():
+    """The 1024 x 1024 convolution keeps a workspace for up to four streams:
+    six streams in turn, twice, with a different filter each time and nothing
+    waited for between, two threads on one stream each and on a shared one,
+    and again after Finalize gave the workspaces back.  Every result equals
+    that of the same call alone, bit for bit."""
+    import threading
+
+    import torch
+
+    import thunderfft_amd as thff
+
+    size, T = 1024, "half"
+    thff.ThunderFFTInitialize(T, size)
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    x = torch.randn(2 * size * size, device="cuda", generator=gen).half()
+    filters = [(torch.randn(2 * size * size, device="cuda", generator=gen) / size).half()
+               for _ in range(6)]
+
+    def call(h, y, stream):
+        thff.ThunderFFT_conv2d_async(T, size, size, x, h, y, 1, stream)
+
+    refs = []
+    for h in filters:
+        refs.append(torch.empty_like(x))
+        thff.ThunderFFT_conv2d(T, size, size, x, h, refs[-1], 1)
+    torch.cuda.synchronize()
+
+    def same(y, k):
+        return torch.equal(y.view(torch.int16), refs[k].view(torch.int16))
+
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    for _ in range(2):
+        out = [[torch.full_like(x, float("nan")) for _ in filters] for _ in streams]
+        torch.cuda.synchronize()
+        for k, h in enumerate(filters):
+            for i, s in enumerate(streams):
+                call(h, out[i][k], s)
+        torch.cuda.synchronize()
+        assert all(same(y, k) for ys in out for k, y in enumerate(ys))
+        del out
+        thff.ThunderFFTFinalize(T)
+        thff.ThunderFFTInitialize(T, size)
+
+    for pair in ((streams[0], streams[1]), (streams[2], streams[2])):
+        out = [[torch.full_like(x, float("nan")) for _ in filters] for _ in range(2)]
+        torch.cuda.synchronize()
+        errors = []
+
+        def work(i):
+            try:
+                for _ in range(20):
+                    for k, h in enumerate(filters):
+                        call(h, out[i][k], pair[i])
+            except Exception as e:  # reported by the main thread
+                errors.append(e)
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+        assert not errors and all(same(y, k) for ys in out for k, y in enumerate(ys))

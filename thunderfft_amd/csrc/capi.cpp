@@ -97,6 +97,99 @@ int scratch_address(int device, float2** out) {
     return THFF_OK;
 }
 
+// Workspaces of thff_conv2d's 1024 x 1024 form, kept between calls: allocating
+// and freeing one stream-ordered took 23 us of host time a call (the three
+// launches take 10), and a synchronised call 45 us more, the pool giving the
+// memory back each time.  At most kMaxWorkspaces per device (32 MiB), one for
+// each stream that calls; further streams, hipStreamPerThread (one handle for
+// many streams) and captured calls allocate for the call as before, and so
+// does a call whose stream's workspace another thread is enqueueing with.
+// The next user waits for the event that the last one recorded, so a
+// workspace is safe even if its stream was destroyed and the handle belongs to
+// another stream now.  Finalize gives them back.
+constexpr size_t kWorkspaceBytes = sizeof(float2) * kScratchValues;
+constexpr int kMaxWorkspaces = 4;
+struct Workspace {
+    void* memory = nullptr;
+    hipEvent_t done = nullptr;  // recorded behind the last call that used it
+    hipStream_t stream = nullptr;
+    bool busy = false;  // a thread is enqueueing with it
+};
+struct DeviceWorkspaces {
+    std::mutex mutex;
+    Workspace slots[kMaxWorkspaces];
+};
+DeviceWorkspaces g_workspaces[kMaxDevices];
+
+// A kept workspace ready for work on `s`, or null (allocate for the call).
+Workspace* acquire_workspace(int device, hipStream_t s) {
+    if (s == hipStreamPerThread) return nullptr;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (capture != hipStreamCaptureStatusNone) return nullptr;
+    DeviceWorkspaces& all = g_workspaces[device];
+    Workspace* found = nullptr;
+    bool fresh = false;
+    {
+        std::lock_guard<std::mutex> lock(all.mutex);
+        for (auto& w : all.slots) {
+            if (w.memory || w.busy) {
+                if (w.stream != s) continue;
+                if (w.busy) return nullptr;
+                found = &w;
+                fresh = false;
+                break;
+            }
+            if (!found) found = &w, fresh = true;
+        }
+        if (!found) return nullptr;
+        found->busy = true;
+        found->stream = s;
+    }
+    hipError_t err;
+    if (fresh) {
+        err = hipEventCreateWithFlags(&found->done, hipEventDisableTiming);
+        if (err == hipSuccess) {
+            err = hipMallocAsync(&found->memory, kWorkspaceBytes, s);
+            if (err != hipSuccess) {
+                (void)hipEventDestroy(found->done);
+                found->memory = nullptr;
+            }
+        }
+    } else {
+        err = hipStreamWaitEvent(s, found->done, 0);
+    }
+    if (err == hipSuccess) return found;
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> lock(all.mutex);
+    found->busy = false;
+    return nullptr;
+}
+
+// Behind the call's last launch on `s`.
+hipError_t release_workspace(int device, Workspace* w, hipStream_t s) {
+    const hipError_t err = hipEventRecord(w->done, s);
+    std::lock_guard<std::mutex> lock(g_workspaces[device].mutex);
+    w->busy = false;
+    return err;
+}
+
+// Frees the device's idle workspaces (the current device).
+void free_workspaces(int device) {
+    DeviceWorkspaces& all = g_workspaces[device];
+    std::lock_guard<std::mutex> lock(all.mutex);
+    for (auto& w : all.slots) {
+        if (!w.memory || w.busy) continue;
+        (void)hipEventSynchronize(w.done);
+        (void)hipEventDestroy(w.done);
+        (void)hipFreeAsync(w.memory, nullptr);
+        w = Workspace{};
+    }
+}
+
 int length_slot(int n) {
     int s = 0;
     while ((64 << s) < n) ++s;
@@ -356,7 +449,7 @@ int conv1d_valid_impl(int precision, const void* x, long long input_len, const v
 
 // 2-D convolution sizes: rows = cols = 64 and 128 run one fused kernel per
 // image (the image stays on chip); 1024 runs the three passes of
-// fft_image.hpp, with a stream-ordered workspace for the filter's row spectra.
+// fft_image.hpp, with a workspace for the filter's row spectra.
 int conv2d_impl(int precision, int rows, int cols, const void* x, const void* h, void* y,
                 int batch, void* stream, bool synchronize, bool allocate = true) {
     if (!supported_precision(precision))
@@ -389,25 +482,26 @@ int conv2d_impl(int precision, int rows, int cols, const void* x, const void* h,
     } else if (rows == 128) {
         err = thff::launch_conv2d128(precision, x, h, y, batch, table, cus, s);
     } else {
-        constexpr int kN = 1024;
-        const size_t spectrum_bytes = sizeof(float2) * kN * kN;
-        void* spectrum = nullptr;
-        if (allocate) {
-            err = hipMallocAsync(&spectrum, spectrum_bytes, s);
-            if (err != hipSuccess) return fail_hip(err, "ThunderFFT_conv2d workspace");
-        } else {
-            int device = 0;
-            err = hipGetDevice(&device);
-            if (err != hipSuccess) return fail_hip(err, "hipGetDevice (conv2d)");
+        int device = 0;
+        err = hipGetDevice(&device);
+        if (err != hipSuccess) return fail_hip(err, "hipGetDevice (conv2d)");
+        void* memory = nullptr;
+        Workspace* kept = nullptr;
+        if (!allocate) {
             float2* p = nullptr;
             const int src = scratch_address(device, &p);
             if (src != THFF_OK) return src;
-            spectrum = p;
+            memory = p;
+        } else if ((kept = acquire_workspace(device, s)) != nullptr) {
+            memory = kept->memory;
+        } else {
+            err = hipMallocAsync(&memory, kWorkspaceBytes, s);
+            if (err != hipSuccess) return fail_hip(err, "ThunderFFT_conv2d workspace");
         }
-        err = thff::launch_conv2d1024(precision, x, h, y, static_cast<float2*>(spectrum), batch,
+        err = thff::launch_conv2d1024(precision, x, h, y, static_cast<float2*>(memory), batch,
                                       table, cus, s);
         if (allocate) {
-            const hipError_t ferr = hipFreeAsync(spectrum, s);
+            const hipError_t ferr = kept ? release_workspace(device, kept, s) : hipFreeAsync(memory, s);
             if (err == hipSuccess) err = ferr;
         }
     }
@@ -505,8 +599,10 @@ int thff_finalize(int precision) {
     if (!supported_precision(precision))
         return fail(THFF_EINVAL, "ThunderFFTFinalize<T>: supported T are float and half only");
     std::lock_guard<std::mutex> lock(g_mutex[precision]);
-    DeviceTables* d = device_tables(precision, "hipGetDevice (finalize)", nullptr);
+    int device = 0;
+    DeviceTables* d = device_tables(precision, "hipGetDevice (finalize)", &device);
     if (!d) return THFF_EIO;
+    free_workspaces(device);
     d->current.store(0, std::memory_order_release);
     hipError_t first = hipSuccess;
     for (auto& slot : d->table) {
