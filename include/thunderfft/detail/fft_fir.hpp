@@ -295,12 +295,14 @@ conv1d_fir_kernel(const IO* __restrict__ x, const float2* __restrict__ taps, IO*
         }
         const long long start = at.r * P::kSpan;
         const long long left = out_len - start;
-        IO* const dst = y + at.q * out_len + start + kVec * lane;
+        IO* const span = y + at.q * out_len + start;
+        IO* const dst = span + kVec * lane;
+        const StreamOut<false> whole(span, P::kSpan * static_cast<int>(sizeof(IO)));
 #pragma unroll
         for (int g = 0; g < P::kGroups; ++g) {
             const u32x4 v = linear[16 * g];
             if (left >= P::kSpan) {
-                st_nt(reinterpret_cast<Vec*>(dst + g * P::kGroup), static_cast<Vec>(v));
+                whole.store(v, 16 * lane, 1024 * g);
             } else {
                 W1 w[kVec];
                 __builtin_memcpy(w, &v, 16);

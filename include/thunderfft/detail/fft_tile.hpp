@@ -221,6 +221,14 @@ struct TileRaw {
     W w[kCount];
 };
 
+// Bytes of tile tl that exist (the last tile of a batch may be partial).
+template <class IO, int N>
+__device__ __forceinline__ int tile_bytes(long long tl, long long batch) {
+    using P = C2CPlan<N>;
+    const long long left = batch - tl * P::kFPB;
+    return static_cast<int>(left < P::kFPB ? left : P::kFPB) * N * static_cast<int>(sizeof(IO));
+}
+
 // Moves 4096-value tiles between HBM and the pass layout (`batch` counts
 // transforms of length N).  Tile element e
 // sits at LDS position lds_pad(e) while staged, which is also where transform
@@ -278,23 +286,33 @@ struct TileIO {
         for (int j = 0; j < 16; ++j) v[j] = slot[lds_pad(t + j * P::kTPF)];
     }
 
-    // v[j] = y[t + TPF*j] -> LDS -> 16-byte non-temporal stores of tile tl.
+    // v[j] = y[t + TPF*j] -> LDS -> 16-byte streamed stores of tile tl (kThrough:
+    // see StreamOut).
+    template <bool kThrough = true>
     __device__ __forceinline__ void store(const cpx (&v)[16], IO* __restrict__ base, long long tl,
                                           long long batch) const {
         region_sync<P::kWaveLocal>();
 #pragma unroll
         for (int j = 0; j < 16; ++j) slot[lds_pad(t + j * P::kTPF)] = v[j];
         region_sync<P::kWaveLocal>();
-        const int nv = valid(tl, batch);
-        IO* dst = base + tl * P::kTile + 1024 * wave;
+        const auto piece = [&](int i) {
+            cpx q[kVec];
 #pragma unroll
-        for (int i = 0; i < Raw::kCount; ++i) {
-            const int e = kVec * lane + 64 * kVec * i;
-            if (e < nv) {
-                cpx q[kVec];
+            for (int c = 0; c < kVec; ++c) q[c] = chunk[lds_pad(kVec * lane + 64 * kVec * i + c)];
+            return I::encode4(q);
+        };
+        if constexpr (kThrough) {
+            const StreamOut<true> dst(base + tl * P::kTile, tile_bytes<IO, N>(tl, batch));
 #pragma unroll
-                for (int c = 0; c < kVec; ++c) q[c] = chunk[lds_pad(e + c)];
-                st_nt(reinterpret_cast<W*>(dst + e), I::encode4(q));
+            for (int i = 0; i < Raw::kCount; ++i)
+                dst.store(piece(i), (1024 * wave + kVec * lane) * static_cast<int>(sizeof(IO)), 1024 * i);
+        } else {
+            const int nv = valid(tl, batch);
+            IO* dst = base + tl * P::kTile + 1024 * wave;
+#pragma unroll
+            for (int i = 0; i < Raw::kCount; ++i) {
+                const int e = kVec * lane + 64 * kVec * i;
+                if (e < nv) st_nt(reinterpret_cast<W*>(dst + e), piece(i));
             }
         }
     }
@@ -327,13 +345,23 @@ struct DirectIO {
 #pragma unroll
         for (int j = 0; j < 16; ++j) v[j] = Io<IO>::decode1(r.w[j]);
     }
+    // kThrough: see StreamOut; for buffers that start on a line.
+    template <bool kThrough = false>
     __device__ __forceinline__ void store(const cpx (&v)[16], IO* __restrict__ base, long long tl,
                                           long long batch) const {
-        const long long tr = tl * P::kFPB + f;
-        if (tr >= batch) return;
-        W* p = reinterpret_cast<W*>(base + tr * N + t);
+        if constexpr (kThrough) {
+            const StreamOut<true> dst(base + tl * P::kTile, tile_bytes<IO, N>(tl, batch));
 #pragma unroll
-        for (int j = 0; j < 16; ++j) st_nt(p + j * P::kTPF, Io<IO>::encode1(v[j]));
+            for (int j = 0; j < 16; ++j)
+                dst.store(Io<IO>::encode1(v[j]), (f * N + t) * static_cast<int>(sizeof(IO)),
+                          j * P::kTPF * static_cast<int>(sizeof(IO)));
+        } else {
+            const long long tr = tl * P::kFPB + f;
+            if (tr >= batch) return;
+            W* p = reinterpret_cast<W*>(base + tr * N + t);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) st_nt(p + j * P::kTPF, Io<IO>::encode1(v[j]));
+        }
     }
 };
 
