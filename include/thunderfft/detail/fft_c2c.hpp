@@ -29,7 +29,7 @@ namespace thff {
 template <int N>
 inline constexpr int kMinWavesPerEU = N <= 1024 ? 3 : 1;
 
-// kThrough: direct movement stores through the L2 (StreamOut).
+// kThrough: stores go through the L2 (StreamOut).
 template <class IO, int N, bool FWD, bool kPrefetch, bool kDirect = false, bool kThrough = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMinWavesPerEU<N>))) void
 c2c_kernel(const IO* __restrict__ in, IO* __restrict__ out, int batch, const float2* __restrict__ tw,
@@ -79,9 +79,7 @@ c2c_kernel(const IO* __restrict__ in, IO* __restrict__ out, int batch, const flo
         cpx v[16];
         io.stage(cur, v);
         fft_registers<N, FWD>(v, io.slot, io.t, w);
-        // float2 N = 64 is the exception: 2^22 values 10.8 us left in the L2,
-        // 12.4 written through (N = 128: level there, 2.5% faster for 2^26).
-        io.template store<!(std::is_same_v<IO, float2> && N == 64)>(v, out, tile, batch);
+        io.template store<kThrough>(v, out, tile, batch);
     }
 }
 

@@ -201,12 +201,14 @@ __device__ __forceinline__ unsigned as_u32(float f) { return __builtin_bit_cast(
 template <class IO>
 struct Io;
 
-// W1 holds one complex value, W4 one 16-byte vector of kVec values.
+// W1 holds one complex value, W4 one 16-byte vector of kVec values; A4 is a W4
+// in memory at its element's alignment (16-byte global accesses need no more).
 template <>
 struct Io<float2> {
     static constexpr int kVec = 2;
     using W1 = u32x2;
     using W4 = u32x4;
+    typedef unsigned A4 __attribute__((ext_vector_type(4), aligned(8)));
     __device__ __forceinline__ static cpx decode1(W1 w) { return {as_f32(w.x), as_f32(w.y)}; }
     __device__ __forceinline__ static W1 encode1(cpx v) { return W1{as_u32(v.re), as_u32(v.im)}; }
     __device__ __forceinline__ static void decode4(W4 w, cpx* v) {
@@ -223,6 +225,7 @@ struct Io<__half2> {
     static constexpr int kVec = 4;
     using W1 = unsigned;
     using W4 = u32x4;
+    typedef unsigned A4 __attribute__((ext_vector_type(4), aligned(4)));
     __device__ __forceinline__ static cpx unpack(unsigned w) {
         const float2 f = __half22float2(__builtin_bit_cast(__half2, w));
         return {f.x, f.y};

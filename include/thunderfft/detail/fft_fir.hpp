@@ -62,18 +62,6 @@ struct FirPlan {
     static constexpr int kMaxSteps = steps(64);
 };
 
-// 16-byte vectors at the element's alignment.
-template <class IO>
-struct FirVec;
-template <>
-struct FirVec<float2> {
-    typedef unsigned type __attribute__((ext_vector_type(4), aligned(8)));
-};
-template <>
-struct FirVec<__half2> {
-    typedef unsigned type __attribute__((ext_vector_type(4), aligned(4)));
-};
-
 // The matrix of a wave's lanes, (row, k) = (lane mod 16, lane / 16), read from
 // two tables of the taps with zeros on both sides: entry d of table p is the
 // pair that multiplies a value's (real, imaginary) for output part p.  The
@@ -219,7 +207,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFirMinWave
 conv1d_fir_kernel(const IO* __restrict__ x, const float2* __restrict__ taps, IO* __restrict__ y,
                   long long len, int ntaps, int batch) {
     using P = FirPlan<IO, A>;
-    using Vec = typename FirVec<IO>::type;
+    using Vec = typename Io<IO>::A4;
     using W1 = typename Io<IO>::W1;
     constexpr int kVec = P::kVec;
     __shared__ u32x4 lds[4 * 4 * P::kPlane];

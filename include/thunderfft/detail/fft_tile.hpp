@@ -266,7 +266,7 @@ struct TileIO {
 #pragma unroll
         for (int i = 0; i < Raw::kCount; ++i) {
             const int e = kVec * lane + 64 * kVec * i;
-            r.w[i] = e < nv ? ld_nt(reinterpret_cast<const W*>(src + e)) : W{};
+            r.w[i] = e < nv ? static_cast<W>(ld_nt(reinterpret_cast<const typename I::A4*>(src + e))) : W{};
         }
     }
 
@@ -287,7 +287,7 @@ struct TileIO {
     }
 
     // v[j] = y[t + TPF*j] -> LDS -> 16-byte streamed stores of tile tl (kThrough:
-    // see StreamOut).
+    // see StreamOut; for buffers that start on a 16-byte boundary).
     template <bool kThrough = true>
     __device__ __forceinline__ void store(const cpx (&v)[16], IO* __restrict__ base, long long tl,
                                           long long batch) const {
@@ -312,7 +312,9 @@ struct TileIO {
 #pragma unroll
             for (int i = 0; i < Raw::kCount; ++i) {
                 const int e = kVec * lane + 64 * kVec * i;
-                if (e < nv) st_nt(reinterpret_cast<W*>(dst + e), piece(i));
+                if (e < nv)
+                    st_nt(reinterpret_cast<typename I::A4*>(dst + e),
+                          static_cast<typename I::A4>(piece(i)));
             }
         }
     }
@@ -345,7 +347,7 @@ struct DirectIO {
 #pragma unroll
         for (int j = 0; j < 16; ++j) v[j] = Io<IO>::decode1(r.w[j]);
     }
-    // kThrough: see StreamOut; for buffers that start on a line.
+    // kThrough: see StreamOut.
     template <bool kThrough = false>
     __device__ __forceinline__ void store(const cpx (&v)[16], IO* __restrict__ base, long long tl,
                                           long long batch) const {

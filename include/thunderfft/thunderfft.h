@@ -69,8 +69,9 @@ int thff_finalize(int precision);
  *   half2) -> THFF_EINVAL, since no kernel can read a split element.
  * Any element-aligned buffer is accepted, as in the reference: buffers on a
  * 16-byte boundary (every hipMalloc pointer, and every offset of whole
- * transforms of >= 2 values) take the vectorised kernels; others take a
- * kernel that moves single elements.
+ * transforms of >= 2 values) take the fastest kernels; others take the fp32
+ * kernel, whose 16-byte or single-element accesses need no more than the
+ * element's alignment.
  * Requires thff_initialize(precision, n) on the current device (THFF_EIO
  * otherwise).  Synchronises `stream` before returning, like the reference. */
 int thff_global(int precision, int n, int forward, const void* d_input, void* d_output,

@@ -147,6 +147,38 @@ def test_element_aligned_buffers(T, n):
 
 
 @pytest.mark.parametrize("T", ["float", "half"])
+@pytest.mark.parametrize("n", SIZES)
+def test_element_aligned_buffers_at_the_staging_threshold(T, n):
+    """2^21 values, where float (and half up to N = 256) moves 16 bytes at the
+    element's alignment, and just below, with a partial last tile: the result
+    is that of the aligned call, to the rounding of two correct transforms
+    (twice TIGHT), and nothing around the output changes."""
+    import torch
+
+    import thunderfft_amd as thff
+
+    esize = 8 if T == "float" else 4
+    dt = torch.float32 if T == "float" else torch.float16
+    thff.ThunderFFTInitialize(T, n)
+    for batch in ((1 << 21) // n + 3, (1 << 21) // n - 1):
+        count = batch * n
+        x = torch.empty(2 * count + 8, dtype=dt, device="cuda")
+        thff.fill_uniform(T, x, count + 4, 5 + n)
+        for in_off, out_off in ((1, 3), (3, 0)):
+            src = x[2 * in_off:2 * (in_off + count)]
+            ref = torch.empty(2 * count, dtype=dt, device="cuda")
+            thff.ThunderFFT_global(T, n, True, src.clone(), ref, batch)
+            out = torch.full((2 * (out_off + count) + 32,), 7.0, dtype=dt, device="cuda")
+            thff.ThunderFFT_global(T, n, True, x.data_ptr() + in_off * esize,
+                                   out.data_ptr() + out_off * esize, batch)
+            got = out[2 * out_off:2 * (out_off + count)]
+            rel = float(torch.linalg.vector_norm(got.float() - ref.float()) /
+                        torch.linalg.vector_norm(ref.float()))
+            assert rel <= 2 * TIGHT[T], (T, n, batch, in_off, out_off, rel)
+            assert bool((out[:2 * out_off] == 7).all()) and bool((out[2 * (out_off + count):] == 7).all())
+
+
+@pytest.mark.parametrize("T", ["float", "half"])
 def test_fft_convenience(T):
     """thunderfft_amd.fft: complex64 / float16[..., N, 2] tensors, with and
     without a caller's out, against the oracle; the length that was current

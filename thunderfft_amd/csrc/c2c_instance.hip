@@ -95,9 +95,11 @@ inline constexpr bool kHalfOnMfma128 = N == 128;
 template <class IO, int N, bool FWD>
 void enqueue(Grid g, const IO* x, IO* y, int batch, const float2* tw, hipStream_t stream) {
     constexpr LaunchShape kShape = launch_shape<N>(std::is_same_v<IO, float2> ? 0 : 1);
-    // Whole lines, written through (N = 256 172.4 against 174.7 us, 2048 178.5
-    // against 180.9); N = 4096 is 5% slower with it for 1025 signals.
-    constexpr bool kThrough = kShape.direct && N < 4096;
+    // Whole lines, written through (fp32 N = 256 172.4 against 174.7 us, 2048
+    // 178.5 against 180.9, 1024 171.2 against 173.6; half2 N = 64 84.9 against
+    // 86.6), but for fp32 N = 64 (2^22 values 12.4 against 10.8 us) and 4096
+    // (1025 signals 5% slower).
+    constexpr bool kThrough = !std::is_same_v<IO, float2> || (N > 64 && N < 4096);
     c2c_kernel<IO, N, FWD, kShape.prefetch, kShape.direct, kThrough><<<g.blocks, 256, 0, stream>>>(
         x, y, batch, tw, g.tiles_per_block);
 }
@@ -140,19 +142,37 @@ void enqueue_mfma3(Grid g, const __half2* x, __half2* y, int batch, hipStream_t 
 }
 
 // Buffers that are element-aligned but not 16-byte aligned (any vec2_t<T>
-// pointer, the reference's contract): the VALU kernel with direct movement
-// (DirectIO, fft_tile.hpp), whose accesses are one element each, one tile
-// per workgroup.
-template <class IO, int N>
+// pointer, the reference's contract): the VALU kernel, one tile per workgroup,
+// either staged, with 16-byte accesses at the element's alignment, or with
+// direct movement, one element per lane and access.  Direct movement covers
+// 64 N / 1024 consecutive values at a time, so short transforms are staged
+// (2^26 values, half2 N = 64 91.8 against 525 us, 128 94.6 against 225; fp32
+// N = 64 188 against 313 us); it saves the staging's latency in small calls
+// (fp32 N = 1024, 1023 signals: 5.8 against 6.2 us), and for half2 from
+// N = 512 on the staging costs more than the accesses (N = 1024, 2^26 values:
+// 111 against 125 us).  The rest is staged from 2^21 values on (fp32 N = 1024,
+// 2895 signals: 9.7 against 12.1 us; half2 N = 256, 16383: 8.1 against 11.1).
+template <class IO, int N, bool kDirect>
 void enqueue_unaligned(bool forward, const IO* x, IO* y, int batch, const float2* tw,
                        hipStream_t stream) {
     const unsigned blocks =
         static_cast<unsigned>((static_cast<long long>(batch) + C2CPlan<N>::kFPB - 1) /
                               C2CPlan<N>::kFPB);
     if (forward)
-        c2c_kernel<IO, N, true, false, true><<<blocks, 256, 0, stream>>>(x, y, batch, tw, 1);
+        c2c_kernel<IO, N, true, false, kDirect><<<blocks, 256, 0, stream>>>(x, y, batch, tw, 1);
     else
-        c2c_kernel<IO, N, false, false, true><<<blocks, 256, 0, stream>>>(x, y, batch, tw, 1);
+        c2c_kernel<IO, N, false, false, kDirect><<<blocks, 256, 0, stream>>>(x, y, batch, tw, 1);
+}
+
+template <class IO, int N>
+void enqueue_unaligned(bool forward, const IO* x, IO* y, int batch, const float2* tw,
+                       hipStream_t stream) {
+    constexpr bool kAlwaysStaged = N <= 128;
+    constexpr bool kAlwaysDirect = std::is_same_v<IO, __half2> && N >= 512;
+    if (kAlwaysStaged || (!kAlwaysDirect && static_cast<long long>(batch) * N >= (1LL << 21)))
+        enqueue_unaligned<IO, N, kAlwaysDirect>(forward, x, y, batch, tw, stream);
+    else
+        enqueue_unaligned<IO, N, !kAlwaysStaged>(forward, x, y, batch, tw, stream);
 }
 
 template <int N>

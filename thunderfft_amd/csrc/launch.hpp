@@ -8,7 +8,7 @@ namespace thff {
 
 // Enqueue the batched C2C kernel for length N.  precision: 0 float2, 1 half2.
 // aligned16: both buffers start on a 16-byte boundary (otherwise they need
-// only the element's alignment, and tiles move value by value).  tw: the
+// only the element's alignment).  tw: the
 // device's fp32 table of N values (cos, sin)(2*pi*m/N); num_cus: the
 // device's compute-unit count (sizes the grid).
 template <int N>
