@@ -224,6 +224,40 @@ def test_conv1d_grid_stride_walks(T, n, per_signal):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("n", [64, 128, 256, 512, 1024, 2048])
+@pytest.mark.parametrize("tiles_per_cu", [4, 16])
+def test_conv1d_grids_for_few_tiles(n, tiles_per_cu):
+    """fp32, a shared filter up to N = 256 and per-signal filters above, takes
+    its grid by the tiles per CU: one tile fewer than the line (one signal
+    short, so partial) and one signal past it.  Every signal through the
+    impulse roll, at the tolerance of the grid-stride walks above."""
+    import torch
+
+    import thunderfft_amd as thff
+
+    per_signal = n > 256
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    whole = tiles_per_cu * cus * thff.transforms_per_block(n)
+    thff.ThunderFFTInitialize("float", n)
+    for batch in (whole - thff.transforms_per_block(n), whole - 1, whole + 1):
+        x = torch.empty(2 * n * batch, device="cuda")
+        thff.fill_uniform("float", x, n * batch, oracle.BENCH_SEED_BASE + n + batch)
+        y = torch.full_like(x, float("nan"))
+        shifts = (7 * np.arange(batch if per_signal else 1) + 3) % n
+        imp = torch.zeros(len(shifts), n, 2, device="cuda")
+        imp[torch.arange(len(shifts), device="cuda"), torch.from_numpy(shifts).cuda(), 0] = 1
+        print(f"float conv1d N={n} batch={batch}", flush=True)
+        thff.ThunderFFT_conv1d("float", n, x, imp, y, batch, per_signal)
+        s = torch.from_numpy(np.broadcast_to(shifts, (batch,)).copy()).cuda()
+        idx = (torch.arange(n, device="cuda")[None, :] - s[:, None]) % n
+        want = torch.gather(x.view(batch, n, 2), 1, idx[:, :, None].expand(batch, n, 2))
+        got = y.view(batch, n, 2)
+        err = float(torch.linalg.vector_norm(got - want) / torch.linalg.vector_norm(want))
+        assert err <= TIGHT["float"] and float((got - want).abs().max()) <= 1e-5
+        del x, y, imp, idx, want, got
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("T", ["half", "float"])
 def test_conv1d_beyond_2e31_values(T):
     """The benchmarked conv1d's length (2048) over 2^31 + 3 * 2048 complex

@@ -39,8 +39,9 @@ inline Grid make_grid(long long ntiles, int per_cu, int num_cus) {
 // whether the next tile's loads are issued before the current tile is
 // transformed.  Measured at batch = 2^26/N:
 //   fp32 N <= 1024: one tile per workgroup, 172-177 us (device grids: 181+).
-//   fp32 N = 2048, 4096: 16 per CU with prefetch, 184 us (one or two tiles
-//     per workgroup: 188-194 us); with direct movement, same box: 178 / 180 us
+//   fp32 N = 2048, 4096: 16 per CU (fewer for few tiles: launch_c2c) with
+//     prefetch, 184 us (one or two tiles per workgroup: 188-194 us); with
+//     direct movement, same box: 178 / 180 us
 //     against 12 per CU 181 / 179, 8 per CU 184 / 180, 4 per CU 189 / 181,
 //     8 per CU without prefetch 186 / 186, one tile per workgroup 181 / 186.
 //     fp32 N = 2048 as one transform per 128-lane workgroup (each pass
@@ -192,7 +193,21 @@ hipError_t launch_c2c(int precision, bool forward, bool aligned16, const void* i
     if constexpr (kHalfOnMfma<N>)
         if (mfma) fpb = MfmaPlan<N / 256>::kFPB;
     const long long ntiles = (static_cast<long long>(batch) + fpb - 1) / fpb;
-    const Grid g = make_grid(ntiles, launch_shape<N>(precision).per_cu, num_cus);
+    int per_cu = launch_shape<N>(precision).per_cu;
+    if (precision == 0 && N >= 2048) {
+        // Beyond 16 tiles per CU the 16 per CU of launch_shape; below, fewer
+        // workgroups that each prefetch what 16 per CU would start afresh:
+        // up to 5 tiles per CU 2 (N = 2048: 1448 signals 10.0 against 12.2
+        // us, 2048 13.2 against 15.6; N = 4096: 1024 signals 14.4 against
+        // 16.6), then 4 (N = 2048: 4096 signals 26.5 against 27.5; N = 4096:
+        // 2048 27.4 against 29.3, 3821 47.1 against 48.5; at 2^26 values
+        // 4 per CU takes 183-185 us, 16 per CU 179-181).
+        if (ntiles <= 5LL * num_cus)
+            per_cu = 2;
+        else if (ntiles <= 16LL * num_cus)
+            per_cu = 4;
+    }
+    const Grid g = make_grid(ntiles, per_cu, num_cus);
     if (precision == 0) {
         const auto* x = static_cast<const float2*>(in);
         auto* y = static_cast<float2*>(out);
@@ -231,12 +246,19 @@ hipError_t launch_c2c(int precision, bool forward, bool aligned16, const void* i
 // workgroups per CU (make_grid; 0 = one tile per workgroup) and next-tile
 // prefetch.  Measured on MI355X (complex: 2^25 values per array; real: 2^26
 // samples, 64 channels):
-//   complex fp32, per-signal filters: one tile per workgroup up to N = 1024
-//     (127-144 us against 134-181 us for device grids, prefetch 138-152);
-//     N = 2048 3 per CU (160 us; 2 tiles per workgroup 172, prefetch 163);
+//   complex fp32, per-signal filters: one tile per workgroup up to N = 256
+//     (130-133 us against 135-152 us for device grids); N = 512 ... 2048 3 per
+//     CU up to 16 tiles per CU (N = 1024: 4097 signals 22.0, 10086 46.3 us; one
+//     tile per workgroup 23.7, 49.7; N = 2048: 6 per CU 2-4% behind), beyond
+//     that 6 per CU, so that a finished workgroup's place is taken at once
+//     (N = 512 136.9, 1024 140.0 us, one tile per workgroup 140.0, 145.6;
+//     N = 2048 146.3, 3 per CU 149.3);
 //     N = 4096 2 per CU (167 us; prefetch 192).
-//   complex fp32, shared filter (transformed once per workgroup): one tile
-//     per workgroup up to N = 256 (92-96 us, equal to prefetch); N = 512 2
+//   complex fp32, shared filter (transformed once per workgroup): up to N =
+//     256 one tile per workgroup (93-97 us, 3 per CU the same), except
+//     between 4 and 16 tiles per CU, where 3 per CU is ahead (2^22.7 values
+//     22.7-23.7 against 24.3-25.0 us; at 600 tiles N = 128 is behind, 13.0
+//     against 9.9); N = 512 2
 //     per CU with early prefetch (101 us, one tile per workgroup 122);
 //     N = 1024, 2048 3 per CU (102 and 107 us; one tile per workgroup 127);
 //     N = 4096 2 per CU with early prefetch (113 us against 121).
@@ -251,11 +273,13 @@ struct ConvShape {
 };
 
 template <int N>
-constexpr ConvShape valu_conv_shape(int precision, bool real, bool per_signal) {
+constexpr ConvShape valu_conv_shape(int precision, bool real, bool per_signal,
+                                    long long tiles_per_cu) {
     if (precision != 0) return {real ? 4 : 16, Prefetch::kNone};
     if (real) return {2, N <= 512 ? Prefetch::kLate : Prefetch::kEarly};
-    if (per_signal) return {N <= 1024 ? 0 : N == 2048 ? 3 : 2, Prefetch::kNone};
-    if (N <= 256) return {0, Prefetch::kNone};
+    if (per_signal) return {N <= 256 ? 0 : N == 4096 ? 2 : tiles_per_cu >= 16 ? 6 : 3,
+                             Prefetch::kNone};
+    if (N <= 256) return {tiles_per_cu >= 4 && tiles_per_cu < 16 ? 3 : 0, Prefetch::kNone};
     if (N == 512 || N == 4096) return {2, Prefetch::kEarly};
     return {3, Prefetch::kNone};
 }
@@ -320,7 +344,8 @@ hipError_t launch_conv1d(int precision, bool per_signal_filter, const void* x, c
     }
     using P = C2CPlan<N>;
     const long long ntiles = (static_cast<long long>(batch) + P::kFPB - 1) / P::kFPB;
-    const ConvShape shape = valu_conv_shape<N>(precision, false, per_signal_filter);
+    const ConvShape shape =
+        valu_conv_shape<N>(precision, false, per_signal_filter, ntiles / (num_cus > 0 ? num_cus : 256));
     const Grid g = make_grid(ntiles, shape.per_cu, num_cus);
     if (precision == 0)
         enqueue_conv1d<float2, N>(per_signal_filter, g, shape.prefetch,
@@ -387,9 +412,9 @@ hipError_t launch_conv1d_real(int precision, const void* x, const float2* spectr
         }
     }
     const long long ntiles = (transforms + P::kFPB - 1) / P::kFPB;
-    const ConvShape shape = valu_conv_shape<N>(precision, true, false);
+    const ConvShape shape = valu_conv_shape<N>(precision, true, false, 0);
     const Grid g = make_grid(ntiles, shape.per_cu, num_cus);
-    constexpr Prefetch kF32 = valu_conv_shape<N>(0, true, false).prefetch;
+    constexpr Prefetch kF32 = valu_conv_shape<N>(0, true, false, 0).prefetch;
     // fp32 N >= 2048 moves samples straight between HBM and registers
     // (conv1d_real_kernel's kDirect): N = 4096 108-114 us against 115-117,
     // 2048 115-119 against 120-123; at N = 1024 it measured slower (125 vs 113).
