@@ -327,17 +327,18 @@ def test_grid_stride_walks(T, n):
     _large_case(T, n, 514 * tile + max(1, tile // 2), directions=(True,))
 
 
-@pytest.mark.parametrize("n", [2048, 4096])
-@pytest.mark.parametrize("tiles_per_cu", [5, 16])
-def test_grids_for_few_tiles(n, tiles_per_cu):
-    """fp32 N >= 2048 takes 2, 4 or 16 workgroups per CU by the tiles per CU:
-    either side of both lines, a whole number of tiles and one partial tile more."""
+@pytest.mark.parametrize("T,n,tiles_per_cu", [("float", n, t) for n in (2048, 4096) for t in (5, 16)]
+                         + [("half", n, t) for n in (128, 2048, 4096) for t in (5, 10)])
+def test_grids_for_few_tiles(T, n, tiles_per_cu):
+    """fp32 N >= 2048 takes 2, 4 or 16 workgroups per CU by the tiles per CU,
+    fp16 N = 128, 2048 and 4096 2 or 3: either side of both lines, a whole
+    number of tiles and one partial tile more."""
     import torch
 
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     whole = tiles_per_cu * cus * (4096 // n)
     for batch in (whole, whole + 1):
-        _large_case("float", n, batch, directions=(True,))
+        _large_case(T, n, batch, directions=(True,))
 
 
 @pytest.mark.parametrize("T,n", [("float", 1024), ("half", 1024), ("half", 4096), ("float", 4096),

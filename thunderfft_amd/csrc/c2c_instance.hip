@@ -207,6 +207,14 @@ hipError_t launch_c2c(int precision, bool forward, bool aligned16, const void* i
         else if (ntiles <= 16LL * num_cus)
             per_cu = 4;
     }
+    // The half2 walks take a third workgroup per CU between 5 and 10 tiles per
+    // CU: N = 128, 46341 signals 9.8 against 10.6 us, 65537 13.2 against 13.9;
+    // N = 2048, 2897 signals 11.9 against 12.5; N = 4096, 2049 signals 13.3
+    // against 14.0.  Outside it the third is even or behind (N = 4096, 1025
+    // signals 7.9 against 7.6; N = 2048, 1449 8.8 against 7.9, 32769 99
+    // against 91).
+    if (precision != 0 && per_cu == 2 && ntiles > 5LL * num_cus && ntiles <= 10LL * num_cus)
+        per_cu = 3;
     const Grid g = make_grid(ntiles, per_cu, num_cus);
     if (precision == 0) {
         const auto* x = static_cast<const float2*>(in);
@@ -265,8 +273,10 @@ hipError_t launch_c2c(int precision, bool forward, bool aligned16, const void* i
 //   real fp32: 2 per CU with prefetch, late up to N = 512 and early above:
 //     97-116 us for N = 64 ... 512 (one tile per workgroup 110-153) and
 //     112/121/115 us for N = 1024/2048/4096 (168-176 without prefetch).
-//   fp16 on VALU (N = 64, 128 only): real 4 per CU (62-64 us; prefetch
-//     62-74), complex 16 per CU (conv1d 78-87 us against 85-91).
+//   fp16 on VALU (N = 64, 128 only): 4 per CU, the occupancy: real 62-64 us
+//     (prefetch 62-74); complex shared filter 56.8 / 61.2 us for N = 64 / 128
+//     (16 per CU 62.9 / 68.9, 5 69 / 74, 3 61 / 65; 2^24 values 30.8 / 33.7
+//     against 38.1 / 41.7), per-signal 78.4 / 83.0 us (16 per CU 83.0 / 87.7).
 struct ConvShape {
     int per_cu;
     Prefetch prefetch;
@@ -275,7 +285,7 @@ struct ConvShape {
 template <int N>
 constexpr ConvShape valu_conv_shape(int precision, bool real, bool per_signal,
                                     long long tiles_per_cu) {
-    if (precision != 0) return {real ? 4 : 16, Prefetch::kNone};
+    if (precision != 0) return {4, Prefetch::kNone};
     if (real) return {2, N <= 512 ? Prefetch::kLate : Prefetch::kEarly};
     if (per_signal) return {N <= 256 ? 0 : N == 4096 ? 2 : tiles_per_cu >= 16 ? 6 : 3,
                              Prefetch::kNone};
