@@ -711,7 +711,8 @@ __global__ __launch_bounds__(256) void conv1d_real_filter_kernel(const float* __
 // accesses, 64 consecutive samples per wave instruction) and stores the
 // real and imaginary parts of its last-pass registers the same way, with no
 // LDS staging.
-template <class IO, int N, Prefetch kPf = Prefetch::kNone, bool kDirect = false>
+template <class IO, int N, Prefetch kPf = Prefetch::kNone, bool kDirect = false,
+          bool kEarly = kPf != Prefetch::kNone>
 __global__ __launch_bounds__(256) void conv1d_real_kernel(
     const typename RealIo<IO>::S* __restrict__ x, const float2* __restrict__ spectrum,
     typename RealIo<IO>::S* __restrict__ y, int batch, int channels,
@@ -742,12 +743,12 @@ __global__ __launch_bounds__(256) void conv1d_real_kernel(
     // already): the channel's spectrum stays in registers while the channel
     // does not change, instead of being read from L2 per tile.
     constexpr bool kKeepSpectrum = N == 4096;
-    // The others load it per tile, with a prefetch (fp32, 2 waves per SIMD) in
+    // The others load it per tile, kEarly (with a prefetch: fp32, 2 waves per SIMD) in
     // flight during the forward transform: N = 2048 112.5 against 121 us, 1024
     // 108 against 113, 64 and 128 96-97 against 99-100 us (2^26 samples, 16
     // channels); without one (half2 N = 64, 128, 4 waves) after it, 10.3
     // against 11.8 us for 2^22.6 samples of N = 128.
-    constexpr bool kEarlySpectrum = !kKeepSpectrum && kPf != Prefetch::kNone;
+    constexpr bool kEarlySpectrum = !kKeepSpectrum && kEarly;
     int spec_d = -1;
     cpx spec[kKeepSpectrum ? 16 : 1];
 

@@ -235,6 +235,37 @@ def test_full_size_impulse_rolls(T, n, batch, channels):
         assert rel <= 1e-3 and err.max() <= 5e-3, label
 
 
+@pytest.mark.parametrize("n", [512, 1024, 2048])
+def test_second_tile_for_some_workgroups(n):
+    """float, a grid of two workgroups per CU: one tile each (the spectrum in
+    flight during the forward transform), one tile more and one less than two
+    each (the spectrum after it), two each.  Channel d's filter is a unit
+    impulse at tap (17 d + 1) mod N, so its output is its input rolled, to the
+    rounding of the transforms (TIGHT)."""
+    import torch
+
+    import thunderfft_amd as thff
+
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    fpb = thff.transforms_per_block(n)
+    for tiles in (2 * cus, 2 * cus + 1, 4 * cus - 1, 4 * cus):
+        channels, batch = tiles, 2 * fpb  # tiles * fpb transforms of two rows
+        taps = [(17 * d + 1) % n for d in range(channels)]
+        h = np.zeros((channels, n), dtype=np.float32)
+        h[np.arange(channels), taps] = 1
+        d_spec = spectra("float", n, h, 1.0 / n)
+        x = torch.empty(batch * channels * n, dtype=torch.float32, device="cuda")
+        thff.fill_uniform("float", x, batch * channels * n // 2, n + tiles)
+        y = torch.empty_like(x)
+        thff.ThunderFFT_conv1d_real("float", n, x, d_spec, y, batch, channels)
+        x, y = x.view(batch, channels, n), y.view(batch, channels, n)
+        shift = (torch.arange(n, device="cuda")[None, :] -
+                 torch.tensor(taps, device="cuda")[:, None]) % n
+        ref = torch.gather(x, 2, shift.expand(batch, channels, n))
+        rel = float(torch.linalg.vector_norm(y - ref) / torch.linalg.vector_norm(ref))
+        assert rel <= TIGHT["float"], (n, tiles, rel)
+
+
 @pytest.mark.parametrize("T", ["half", "float"])
 def test_beyond_2e31_samples(T):
     """[8194][64][4096] real samples, 2^31 + 2^19 per array (4.3 GB fp16,

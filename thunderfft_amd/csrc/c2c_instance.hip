@@ -428,14 +428,31 @@ hipError_t launch_conv1d_real(int precision, const void* x, const float2* spectr
     // fp32 N >= 2048 moves samples straight between HBM and registers
     // (conv1d_real_kernel's kDirect): N = 4096 108-114 us against 115-117,
     // 2048 115-119 against 120-123; at N = 1024 it measured slower (125 vs 113).
-    if (precision == 0)
-        conv1d_real_kernel<float2, N, kF32, (N >= 2048)><<<g.blocks, 256, 0, stream>>>(
-            static_cast<const float*>(x), spectrum, static_cast<float*>(y), batch, channels, tw,
-            g.tiles_per_block);
-    else if constexpr (N < 256)  // fp16 N >= 256 returned above (MFMA)
+    if (precision == 0) {
+        const auto launch = [&](auto early) {
+            conv1d_real_kernel<float2, N, kF32, (N >= 2048), decltype(early)::value>
+                <<<g.blocks, 256, 0, stream>>>(static_cast<const float*>(x), spectrum,
+                                               static_cast<float*>(y), batch, channels, tw,
+                                               g.tiles_per_block);
+        };
+        // Where only some workgroups have a second tile, its spectrum is loaded
+        // after the forward transform (N = 2048, 50 channels: 57 rows 14.7
+        // against 15.7 us for the early load, 66 rows 15.7 against 16.6; N =
+        // 1024, 115 rows 13.5 against 13.8; N = 512, 231 rows 14.7 against
+        // 14.9); from two full rounds on early (N = 2048, 115 rows 24.1 against
+        // 25.2).
+        if constexpr (N >= 512 && N <= 2048) {
+            if (ntiles > g.blocks && ntiles < 2LL * g.blocks) {
+                launch(std::false_type{});
+                return hipGetLastError();
+            }
+        }
+        launch(std::true_type{});
+    } else if constexpr (N < 256) {  // fp16 N >= 256 returned above (MFMA)
         conv1d_real_kernel<__half2, N><<<g.blocks, 256, 0, stream>>>(
             static_cast<const __half*>(x), spectrum, static_cast<__half*>(y), batch, channels, tw,
             g.tiles_per_block);
+    }
     return hipGetLastError();
 }
 
