@@ -341,6 +341,15 @@ def test_grids_for_few_tiles(T, n, tiles_per_cu):
         _large_case(T, n, batch, directions=(True,))
 
 
+@pytest.mark.parametrize("n,line", [(n, v) for n, end in ((128, 3 << 22), (512, 3 << 22), (1024, 3 << 20))
+                                    for v in (1 << 21, end)])
+def test_store_forms_at_their_lines(n, line):
+    """fp32 N = 128, 512 and 1024 store through the L2 up to 2^21 values and from
+    3 * 2^22 (N = 1024: 3 * 2^20) on: both sides of both lines."""
+    for batch in (line // n - 1, line // n, line // n + 1):
+        _large_case("float", n, batch, directions=(True, False))
+
+
 @pytest.mark.parametrize("T,n", [("float", 1024), ("half", 1024), ("half", 4096), ("float", 4096),
                                  ("half", 128), ("half", 2048)])
 def test_beyond_2e31_values(T, n):

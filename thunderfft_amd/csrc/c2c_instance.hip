@@ -101,6 +101,23 @@ void enqueue(Grid g, const IO* x, IO* y, int batch, const float2* tw, hipStream_
     // 86.6), but for fp32 N = 64 (2^22 values 12.4 against 10.8 us) and 4096
     // (1025 signals 5% slower).
     constexpr bool kThrough = !std::is_same_v<IO, float2> || (N > 64 && N < 4096);
+    // fp32 N = 128, 512 and 1024 leave the lines in the L2 where both arrays
+    // fit the memory-side cache and are more than 2^21 values: N = 128 up to
+    // 3 * 2^22 (18820 signals 7.6 us, written through 8.0; 32768 12.8, 13.1;
+    // 65536 24.5, 24.8), N = 512 likewise (5042 signals 8.7, 9.9; 8192 13.8,
+    // 14.1; 16384 25.3, 25.5), N = 1024 as long as every tile runs at once, 3
+    // per CU (2702 signals 8.4, 8.6; 3104 12.1, 11.5).  N = 256 gains from the
+    // write-through there (10809 signals 10.1, 9.6), and so do all outside
+    // (N = 128: 16384 signals 6.3, 6.1, 131072 45.5, 44.9).
+    if constexpr (std::is_same_v<IO, float2> && (N == 128 || N == 512 || N == 1024)) {
+        constexpr long long kEnd = N == 1024 ? 3LL << 20 : 3LL << 22;
+        const long long values = static_cast<long long>(batch) * N;
+        if (values > 1LL << 21 && values < kEnd) {
+            c2c_kernel<IO, N, FWD, kShape.prefetch, kShape.direct><<<g.blocks, 256, 0, stream>>>(
+                x, y, batch, tw, g.tiles_per_block);
+            return;
+        }
+    }
     c2c_kernel<IO, N, FWD, kShape.prefetch, kShape.direct, kThrough><<<g.blocks, 256, 0, stream>>>(
         x, y, batch, tw, g.tiles_per_block);
 }
