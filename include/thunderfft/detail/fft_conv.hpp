@@ -555,7 +555,7 @@ __global__ __launch_bounds__(1024) void conv2d128_lanes_kernel(const float2* __r
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < 16; ++j)
-            __builtin_amdgcn_raw_buffer_store_b64(u32x2{}, none, 0, 64 * kN * j, 2);
+            __builtin_amdgcn_raw_buffer_store_b64(u32x2{}, none, 8 * j, 0, 2);
     }
     forward(hs, L, u, c, t);
     constexpr float kScale = 1.0f / kImg;

@@ -355,8 +355,9 @@ conv1d_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__ h,
     auto load = [&](const __half2* src, int nv, u32x4 (&raw)[kRaw]) {
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<__half2*>(src), 0, 4 * nv, 0x00020000);
+        const int at = step_base(16 * lane);
 #pragma unroll
-        for (int i = 0; i < kRaw; ++i) raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * lane, 1024 * i, 2);
+        for (int i = 0; i < kRaw; ++i) raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, at + 1024 * i, 0, 2);
     };
     // Stage loaded values in the wave's region; transform what is staged.
     auto stage = [&](const u32x4 (&raw)[kRaw]) {
@@ -477,10 +478,11 @@ conv1d_mfma_kernel(const __half2* __restrict__ x, const __half2* __restrict__ h,
         const __amdgpu_buffer_rsrc_t ys =
             __builtin_amdgcn_make_buffer_rsrc(y + off, 0, 4 * nv, 0x00020000);
         const unsigned* const obase = region + P::out_pad(4 * lane);
+        const int at = step_base(16 * lane);
 #pragma unroll
         for (int i = 0; i < kRaw; ++i)
             __builtin_amdgcn_raw_buffer_store_b128(
-                *reinterpret_cast<const u32x4*>(obase + P::kOutStep * i), ys, 16 * lane, 1024 * i, 2);
+                *reinterpret_cast<const u32x4*>(obase + P::kOutStep * i), ys, at + 1024 * i, 0, 2);
         if constexpr (C == 8) priority.set(--left);
     }
 }
@@ -669,9 +671,10 @@ conv1d_real_mfma4096_kernel(const __half* __restrict__ x, const float2* __restri
             const RealRowPair rp = RealRowPair::at(ps.p, ps.d, channels, batch, N);
             const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
                 const_cast<__half*>(x + rp.row0), 0, live ? rp.bytes : 0, 0x00020000);
+            const int at = step_base(load_off);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                raw[e] = __builtin_amdgcn_raw_buffer_load_b128(rs, load_off, 512 * e, 2);
+                raw[e] = __builtin_amdgcn_raw_buffer_load_b128(rs, at + 512 * e, 0, 2);
         } else {
             long long r0, r1;
             rows(ps, r0, r1);

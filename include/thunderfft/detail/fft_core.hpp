@@ -167,8 +167,11 @@ __device__ __forceinline__ void st_nt(W* p, W w) {
 }
 
 // The `bytes` bytes at `base` (both uniform over the wave) as a buffer for
-// streamed stores: offset v (per lane) + s (constant); accesses past the end
-// are dropped by the hardware's range check.  kThrough also writes through the
+// streamed stores; stores at offset v (per lane) past the end are dropped by
+// the hardware's range check.  A constant step s goes into the scalar offset,
+// which the check may leave out or take off the size first: for steps below
+// `bytes` of lanes whose v is past the end whenever v + s is.  Other steps are
+// part of v, based on step_base().  kThrough also writes through the
 // XCD's L2 (agent scope) instead of leaving lines for the write-back at the
 // kernel's end.  For whole lines from workgroups that each store once it is
 // mostly the faster form: a copy of 512 MiB takes 162.4 against 165.0 us, the fp32
@@ -184,13 +187,21 @@ struct StreamOut {
     __amdgpu_buffer_rsrc_t rs;
     __device__ __forceinline__ StreamOut(void* base, int bytes)
         : rs(__builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000)) {}
-    __device__ __forceinline__ void store(u32x4 w, int v, int s) const {
+    __device__ __forceinline__ void store(u32x4 w, int v, int s = 0) const {
         __builtin_amdgcn_raw_buffer_store_b128(w, rs, v, s, kPolicy);
     }
-    __device__ __forceinline__ void store(u32x2 w, int v, int s) const {
+    __device__ __forceinline__ void store(u32x2 w, int v, int s = 0) const {
         __builtin_amdgcn_raw_buffer_store_b64(w, rs, v, s, kPolicy);
     }
 };
+
+// v as the base of a buffer access's constant steps: opaque here, so that the
+// steps (up to 4095) become the instructions' immediate offsets; sums known
+// outside a loop are computed there and kept, a register for each step.
+__device__ __forceinline__ int step_base(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
 
 // Bit casts taken on plain scalars: clang mis-evaluates __builtin_bit_cast
 // applied directly to an ext-vector element (w.y read as w.x), so elements

@@ -303,9 +303,9 @@ struct TileIO {
         };
         if constexpr (kThrough) {
             const StreamOut<true> dst(base + tl * P::kTile, tile_bytes<IO, N>(tl, batch));
+            const int at = step_base((1024 * wave + kVec * lane) * static_cast<int>(sizeof(IO)));
 #pragma unroll
-            for (int i = 0; i < Raw::kCount; ++i)
-                dst.store(piece(i), (1024 * wave + kVec * lane) * static_cast<int>(sizeof(IO)), 1024 * i);
+            for (int i = 0; i < Raw::kCount; ++i) dst.store(piece(i), at + 1024 * i);
         } else {
             const int nv = valid(tl, batch);
             IO* dst = base + tl * P::kTile + 1024 * wave;

@@ -17,7 +17,8 @@ import numpy as np
 import pytest
 
 import oracle
-from thff_testlib import GATE, SIZES, TIGHT, from_device, run_case, to_device
+from thff_testlib import (GATE, SIZES, TIGHT, from_device, run_case, tile_guarded_output,
+                          to_device)
 
 pytestmark = pytest.mark.gpu
 
@@ -144,6 +145,27 @@ def test_element_aligned_buffers(T, n):
             assert m["nonfinite"] == 0 and m["rel_l2"] <= GATE and m["rel_l2"] <= TIGHT[T], label
             around = np.concatenate([out[:out_off], out[out_off + count:]])
             assert np.all(around == guard), label
+
+
+@pytest.mark.parametrize("T", ["float", "half"])
+@pytest.mark.parametrize("n", SIZES)
+def test_partial_tiles_keep_to_the_output(T, n):
+    """One signal, and one more than a whole tile: nothing within a tile of the
+    output changes, and every signal is transformed."""
+    import thunderfft_amd as thff
+
+    fpb = thff.transforms_per_block(n)
+    thff.ThunderFFTInitialize(T, n)
+    for batch in (1, fpb + 1):
+        x = oracle.represent(oracle.uniform(n, batch, seed=n + batch), T)
+        d_x = to_device(x, T)
+        for forward in (True, False):
+            y, intact = tile_guarded_output(batch * n, T)
+            thff.ThunderFFT_global(T, n, forward, d_x, y, batch)
+            m = oracle.metrics(from_device(y, T), oracle.fft(x, forward=forward).reshape(-1))
+            label = (T, n, batch, forward, m["rel_l2"])
+            assert intact(), label
+            assert m["nonfinite"] == 0 and m["rel_l2"] <= TIGHT[T], label
 
 
 @pytest.mark.parametrize("T", ["float", "half"])

@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 import oracle
-from thff_testlib import GATE, SIZES, from_device, to_device
+from thff_testlib import GATE, SIZES, from_device, tile_guarded_output, to_device
 
 pytestmark = pytest.mark.gpu
 
@@ -75,6 +75,28 @@ def test_conv1d_matches_direct_convolution(T, n):
             print(label, flush=True)
             assert m["nonfinite"] == 0, label
             assert m["rel_l2"] <= GATE and m["rel_l2"] <= TIGHT[T], label
+
+
+@pytest.mark.parametrize("T", ["float", "half"])
+@pytest.mark.parametrize("n", SIZES)
+def test_conv1d_partial_tiles_keep_to_the_output(T, n):
+    """One signal, and one more than a whole tile: nothing within a tile of the
+    output changes, and every signal is convolved."""
+    import thunderfft_amd as thff
+
+    fpb = thff.transforms_per_block(n)
+    thff.ThunderFFTInitialize(T, n)
+    for per_signal in (True, False):
+        for batch in (1, fpb + 1):
+            x = oracle.represent(oracle.uniform(n, batch, seed=n + batch), T)
+            h = oracle.represent(_filters(n, batch if per_signal else 1, seed=n + batch), T)
+            y, intact = tile_guarded_output(batch * n, T)
+            thff.ThunderFFT_conv1d(T, n, to_device(x, T), to_device(h, T), y, batch, per_signal)
+            m = oracle.metrics(from_device(y, T).reshape(batch, n),
+                               oracle.circconv1d(x, h, per_signal))
+            label = (T, n, per_signal, batch, m["rel_l2"])
+            assert intact(), label
+            assert m["nonfinite"] == 0 and m["rel_l2"] <= TIGHT[T], label
 
 
 @pytest.mark.parametrize("T", ["float", "half"])

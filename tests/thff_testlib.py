@@ -44,6 +44,26 @@ def guarded_output(count: int, T: str):
     return to_device(host, T)
 
 
+def tile_guarded_output(count: int, T: str):
+    """NaN-filled output of `count` complex values and whether a tile and a half
+    of sentinels (6144 values) on either side of it still hold: a kernel moves
+    tiles of 4096 values, so a piece of a partial tile that is stored although
+    it should be dropped lands there."""
+    import torch
+
+    guard = 6144
+    dt = torch.float32 if T == "float" else torch.float16
+    buf = torch.full((2 * (count + 2 * guard),), GUARD_VALUE[0], dtype=dt, device="cuda")
+    out = buf[2 * guard:2 * (guard + count)]
+    out.fill_(float("nan"))
+
+    def intact() -> bool:
+        return bool((buf[:2 * guard] == GUARD_VALUE[0]).all()
+                    and (buf[2 * (guard + count):] == GUARD_VALUE[0]).all())
+
+    return out, intact
+
+
 def guards_changed(out_host: np.ndarray, count: int) -> int:
     g = out_host[count:]
     return int(np.sum((g.real != GUARD_VALUE[0]) | (g.imag != GUARD_VALUE[1])))
