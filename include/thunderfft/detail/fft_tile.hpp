@@ -288,7 +288,7 @@ struct TileIO {
 
     // v[j] = y[t + TPF*j] -> LDS -> 16-byte streamed stores of tile tl (kThrough:
     // see StreamOut; for buffers that start on a 16-byte boundary).
-    template <bool kThrough = true>
+    template <bool kThrough = false>
     __device__ __forceinline__ void store(const cpx (&v)[16], IO* __restrict__ base, long long tl,
                                           long long batch) const {
         region_sync<P::kWaveLocal>();

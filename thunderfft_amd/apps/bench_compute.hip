@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256) void repeat_valu(const IO* in, IO* out, int ba
     io.stage(r, v);
 #pragma unroll 1
     for (int i = 0; i < repeats; ++i) fft_registers<N, true>(v, io.slot, io.t, w);
-    io.store(v, out, blockIdx.x, batch);
+    io.template store<true>(v, out, blockIdx.x, batch);
 }
 
 // half2 on MFMA (the kernel the library runs for half, N = 256*C): steps 1-6
