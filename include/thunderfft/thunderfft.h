@@ -175,7 +175,7 @@ int thff_conv1d_valid_async(int precision, const void* d_x, long long input_len,
  * computed as IFFT2(FFT2(x[b]) * FFT2(h)) / (rows*cols).  rows = cols = 64 or
  * 128: one fused kernel (forward 2-D FFT, product, inverse) per image, the
  * image on chip.  rows = cols = 1024 (the reference's sample shape): row FFTs
- * x -> y, and of the filter into an 8 MiB workspace (kept for up to 4 streams
+ * x -> y, and of the filter into an 8.25 MiB workspace (kept for up to 4 streams
  * per device until thff_finalize; further streams and captured calls allocate
  * and free one stream-ordered, hipMallocAsync), a column pass (FFT, product,
  * inverse FFT) and inverse row FFTs in place in y.  Other shapes -> THFF_EINVAL; requires thff_initialize(precision, rows).
@@ -193,7 +193,7 @@ int thff_conv2d_async(int precision, int rows, int cols, const void* d_x, const 
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments, checks, results and return codes as thff_conv2d_async
  * (enqueued on `stream`, no synchronisation); the 1024 x 1024 form keeps the
- * filter's row spectra in a device array of the library (8 MiB per GPU, held
+ * filter's row spectra in a device array of the library (8.25 MiB per GPU, held
  * until the process ends) instead of a stream-ordered allocation, so images
  * larger than 1024 x 1024 are THFF_EINVAL.  Every call on one GPU shares
  * that array: calls that overlap on one GPU (other streams, other threads)

@@ -545,3 +545,65 @@ def test_conv2d_1024_image_counts_and_range(T, batch):
         err = (y.view(batch, size, size, 2).float() - want).flatten(1)
         rel = torch.linalg.vector_norm(err, dim=1) / torch.linalg.vector_norm(want.flatten(1), dim=1)
         assert bool(torch.isfinite(rel).all()) and float(rel.max()) <= TIGHT[T], (T, batch, rel)
+
+
+def test_conv2d_1024_half_keeps_small_and_large_outputs():
+    """half images of rms 1e-2 ... 3e-5 and tones of 60000 out (50 in, a tap of
+    1200: rows sum to 51200), each with the others in one call.  Three values on
+    the way are rounded to half (the spectra after each pass and the result):
+    TIGHT, and the spacing of the f16 subnormals in the result, 2^-24 / sqrt(6)
+    in rms over a value's two components, and in the first spectra, which are
+    11 times as large as the images."""
+    import torch
+
+    import thunderfft_amd as thff
+
+    size, T = 1024, "half"
+    thff.ThunderFFTInitialize(T, size)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    r = torch.arange(size, device="cuda", dtype=torch.float64)
+    shift, dr, dc = 5, 129, 31
+
+    def tone(kr, kc):
+        a = 2 * np.pi / size * ((kr * r)[:, None] + (kc * r)[None, :])
+        return torch.stack((torch.cos(a), torch.sin(a)), dim=-1)
+
+    quiet = [float(v) for v in (1e-2, 1e-3, 3e-4, 3e-5)]
+    images = [torch.randn(size, size, 2, device="cuda", generator=gen, dtype=torch.float64)
+              * (v / np.sqrt(2)) for v in quiet]
+    for tap, stack in ((1.0, images + [50.0 * tone(3, 8 * 11 + shift)]),
+                       (1200.0, [50.0 * tone(8 * k + k % 8, 77 * k) for k in range(9)] + images[:2])):
+        x = torch.stack(stack).half()
+        h = torch.zeros(size, size, 2, dtype=torch.float16, device="cuda")
+        h[dr, dc, 0] = tap
+        y = torch.full_like(x, float("nan"))
+        thff.ThunderFFT_conv2d(T, size, size, x, h, y, len(stack))
+        want = tap * torch.roll(x.double(), shifts=(dr, dc), dims=(1, 2))
+        err = torch.linalg.vector_norm((y.double() - want).flatten(1), dim=1)
+        norm = torch.linalg.vector_norm(want.flatten(1), dim=1)
+        rms = norm / size
+        bound = TIGHT[T] + 2.0 ** -24 / np.sqrt(6) * (1 + tap / 11) / rms
+        assert bool((err / norm <= bound).all()), (tap, err / norm, bound)
+
+
+def test_conv2d_1024_half_rounds_of_images():
+    """One image more than a round of passes takes (256), the filter in the
+    first round's launch only: every image rolled, small ones among them."""
+    import torch
+
+    import thunderfft_amd as thff
+
+    size, T, batch = 1024, "half", 257
+    thff.ThunderFFTInitialize(T, size)
+    x = torch.empty(2 * size * size * batch, dtype=torch.float16, device="cuda")
+    thff.fill_uniform(T, x, size * size * batch, 91)
+    x = x.view(batch, size, size, 2)
+    x[1::3] *= 1e-3
+    imp = np.zeros((size, size), dtype=np.complex64)
+    imp[3, 1000] = 1
+    y = torch.full_like(x, float("nan"))
+    thff.ThunderFFT_conv2d(T, size, size, x, to_device(imp, T), y, batch)
+    for b in range(batch):
+        want = torch.roll(x[b].float(), shifts=(3, 1000), dims=(0, 1))
+        rel = float(torch.linalg.vector_norm(y[b].float() - want) / torch.linalg.vector_norm(want))
+        assert rel <= TIGHT[T], (b, rel)

@@ -550,15 +550,23 @@ template <class IO>
 void enqueue_conv2d1024(const IO* x, const IO* h, IO* y, float2* workspace, int batch,
                         const float2* tw, int num_cus, hipStream_t stream) {
     using P = ImagePlan<IO>;
-    const unsigned groups = static_cast<unsigned>(batch) * P::kLen;
-    image_rows_kernel<IO, true><<<groups + P::kLen, P::kRowLanes, 0, stream>>>(
-        x, y, h, workspace, groups, tw);
+    static_assert(sizeof(float2) * P::kImage + P::kMarkImages * P::kMarks == kConv2d1024WorkspaceBytes,
+                  "workspace: the filter and the marks");
+    auto* const marks = reinterpret_cast<unsigned char*>(workspace + P::kImage);
     const int wanted = kImageColsPerCu * num_cus / P::kBlocks;  // images in flight
-    const int images = wanted < 1 ? 1 : wanted < batch ? wanted : batch;
-    image_cols_kernel<IO><<<P::kBlocks * images, 256, 0, stream>>>(
-        y, workspace, batch, P::kScale / (1024.0f * 1024.0f), tw);
-    image_rows_kernel<IO, false><<<groups, P::kRowLanes, 0, stream>>>(y, y, nullptr, nullptr, groups,
-                                                                      tw);
+    const int round = P::kMarked ? P::kMarkImages : batch;
+    for (int first = 0; first < batch; first += round) {  // first < 2^16
+        const int n = batch - first < round ? batch - first : round;
+        const unsigned groups = static_cast<unsigned>(n) * P::kLen;
+        const int images = wanted < 1 ? 1 : wanted < n ? wanted : n;
+        IO* const out = y + first * P::kImage;
+        image_rows_kernel<IO, true><<<groups + (first == 0 ? P::kLen : 0), P::kRowLanes, 0, stream>>>(
+            x + first * P::kImage, out, h, workspace, groups, nullptr, tw);
+        image_cols_kernel<IO><<<P::kBlocks * images, 256, 0, stream>>>(
+            out, workspace, marks, n, P::kScale * P::kQuiet / (1024.0f * 1024.0f), tw);
+        image_rows_kernel<IO, false><<<groups, P::kRowLanes, 0, stream>>>(out, out, nullptr, nullptr,
+                                                                          groups, marks, tw);
+    }
 }
 }  // namespace
 

@@ -63,19 +63,18 @@ struct DeviceTables {
 DeviceTables g_tables[2][kMaxDevices];
 std::mutex g_mutex[2];
 
-// Workspace of the allocation-free 2-D convolution (thff_conv2d_noalloc):
-// one fp32 spectrum of the largest image the multi-pass form takes,
-// 1024 x 1024 (8 MiB), in a device array of this library's code object, so
+// Workspace of the allocation-free 2-D convolution (thff_conv2d_noalloc) of the
+// largest image, 1024 x 1024 (8.25 MiB), in a device array of this library's code object, so
 // that each GPU the library runs on holds its own copy until the process
 // ends.  In host code `scratch` names the symbol, not a device address: the
 // address of the current device's copy is resolved once per device with
 // hipGetSymbolAddress (in ThunderFFTInitialize, which every convolution
 // requires first, or at the first call) and kept in g_scratch.  Every
 // allocation-free call on a GPU shares that GPU's copy: calls that overlap on
-// one GPU race.  Nothing in it needs clearing: the filter pass writes every
-// value before the column pass reads it.
-constexpr long long kScratchValues = 1024LL * 1024LL;
-__device__ __align__(256) float2 scratch[kScratchValues];
+// one GPU race.  Nothing in it needs clearing: the passes write every value
+// and mark before a later one reads it.
+constexpr long long kScratchImage = 1024LL * 1024LL;
+__device__ __align__(256) float2 scratch[thff::kConv2d1024WorkspaceBytes / sizeof(float2)];
 std::atomic<float2*> g_scratch[kMaxDevices] = {};
 std::mutex g_scratch_mutex;
 
@@ -100,7 +99,7 @@ int scratch_address(int device, float2** out) {
 // Workspaces of thff_conv2d's 1024 x 1024 form, kept between calls: allocating
 // and freeing one stream-ordered took 23 us of host time a call (the three
 // launches take 10), and a synchronised call 45 us more, the pool giving the
-// memory back each time.  At most kMaxWorkspaces per device (32 MiB), one for
+// memory back each time.  At most kMaxWorkspaces per device (33 MiB), one for
 // each stream that calls; further streams, hipStreamPerThread (one handle for
 // many streams) and captured calls allocate for the call as before, and so
 // does a call whose stream's workspace another thread is enqueueing with.
@@ -109,7 +108,7 @@ int scratch_address(int device, float2** out) {
 // another stream now.  The null stream, which is never another, orders its
 // calls by itself: no event there (3 us of its time).  Finalize gives them
 // back.
-constexpr size_t kWorkspaceBytes = sizeof(float2) * kScratchValues;
+constexpr size_t kWorkspaceBytes = thff::kConv2d1024WorkspaceBytes;
 constexpr int kMaxWorkspaces = 4;
 struct Workspace {
     void* memory = nullptr;
@@ -472,7 +471,7 @@ int conv2d_impl(int precision, int rows, int cols, const void* x, const void* h,
         return fail(THFF_EINVAL, "ThunderFFT_conv2d requires 16-byte aligned buffers");
     if (batch > (rows == 1024 ? (1 << 16) : (1 << 24)))
         return fail(THFF_EINVAL, "ThunderFFT batch exceeds one launch");
-    if (!allocate && static_cast<long long>(rows) * cols > kScratchValues)
+    if (!allocate && static_cast<long long>(rows) * cols > kScratchImage)
         return fail(THFF_EINVAL,
                     "ThunderFFT_conv2d_noalloc: the image exceeds the allocation-free workspace "
                     "(one 1024 x 1024 spectrum)");

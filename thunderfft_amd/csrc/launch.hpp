@@ -50,8 +50,10 @@ hipError_t launch_conv2d128(int precision, const void* x, const void* h, void* y
                             const float2* tw, int num_cus, hipStream_t stream);
 
 // Enqueue the fused 2-D circular convolution of `batch` 1024 x 1024 images
-// with one shared 1024 x 1024 filter h (tw: the N = 1024 table); workspace: one
-// image of fp32 complex values.
+// with one shared 1024 x 1024 filter h (tw: the N = 1024 table); workspace:
+// kConv2d1024WorkspaceBytes (one image of fp32 complex values and the half2
+// column pass's marks, fft_image.hpp), 16-byte aligned.
+inline constexpr long long kConv2d1024WorkspaceBytes = 8LL * 1024 * 1024 + 256 * 1024;
 hipError_t launch_conv2d1024(int precision, const void* x, const void* h, void* y,
                              float2* workspace, int batch, const float2* tw, int num_cus,
                              hipStream_t stream);
