@@ -175,10 +175,11 @@ int thff_conv1d_valid_async(int precision, const void* d_x, long long input_len,
  * computed as IFFT2(FFT2(x[b]) * FFT2(h)) / (rows*cols).  rows = cols = 64 or
  * 128: one fused kernel (forward 2-D FFT, product, inverse) per image, the
  * image on chip.  rows = cols = 1024 (the reference's sample shape): row FFTs
- * x -> y, and of the filter into an 8.25 MiB workspace (kept for up to 4 streams
- * per device until thff_finalize; further streams and captured calls allocate
- * and free one stream-ordered, hipMallocAsync), a column pass (FFT, product,
- * inverse FFT) and inverse row FFTs in place in y.  Other shapes -> THFF_EINVAL; requires thff_initialize(precision, rows).
+ * x -> y, and of the filter into an 8.25 MiB workspace (up to 4 per device are
+ * kept until thff_finalize, for the streams that call; a further stream takes
+ * over one that is not in use; if there is none, and for captured calls, one is
+ * allocated and freed stream-ordered, hipMallocAsync), a column pass (FFT,
+ * product, inverse FFT) and inverse row FFTs in place in y.  Other shapes -> THFF_EINVAL; requires thff_initialize(precision, rows).
  * x and y hold batch*rows*cols complex values, h rows*cols.  Same checks,
  * return codes and synchronisation as thff_conv1d. */
 int thff_conv2d(int precision, int rows, int cols, const void* d_x, const void* d_h, void* d_y,

@@ -270,3 +270,116 @@ def test_conv2d_workspaces_on_many_streams_and_threads():
             t.join()
         torch.cuda.synchronize()
         assert not errors and all(same(y, k) for ys in out for k, y in enumerate(ys))
+
+
+class _Hip:
+    """The few runtime calls that torch has no counterpart for."""
+
+    def __init__(self):
+        import ctypes
+
+        self.c = ctypes
+        self.lib = ctypes.CDLL("libamdhip64.so")
+
+    def call(self, name, *args):
+        err = getattr(self.lib, name)(*args)
+        assert err == 0, (name, err)
+
+    def stream(self):
+        s = self.c.c_void_p()
+        self.call("hipStreamCreate", self.c.byref(s))
+        return s
+
+    def destroy(self, s):
+        self.call("hipStreamDestroy", s)
+
+    def pool_used(self, high):
+        """Bytes in use of the device's default pool: now, or the most since the
+        last call with `high`."""
+        pool, value = self.c.c_void_p(), self.c.c_uint64()
+        self.call("hipDeviceGetDefaultMemPool", self.c.byref(pool), 0)
+        self.call("hipMemPoolGetAttribute", pool, 8 if high else 7, self.c.byref(value))
+        if high:
+            self.call("hipMemPoolSetAttribute", pool, 8, self.c.byref(self.c.c_uint64(0)))
+        return value.value
+
+
+def test_conv2d_workspaces_outlive_their_streams():
+    """Twelve streams (created beforehand, so that no handle comes back) used and
+    destroyed in turn, each with a filter of its own: the first four calls keep
+    a workspace each, the others take over one of those and allocate nothing,
+    and every result equals that of the call alone."""
+    import torch
+
+    import thunderfft_amd as thff
+
+    size, T = 1024, "half"
+    hip = _Hip()
+    thff.ThunderFFTFinalize(T)
+    thff.ThunderFFTInitialize(T, size)
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    x = torch.randn(2 * size * size, device="cuda", generator=gen).half()
+    before = None
+    kept = []
+    streams = [hip.stream() for _ in range(12)]
+    for i, s in enumerate(streams):
+        h = (torch.randn(2 * size * size, device="cuda", generator=gen) / size).half()
+        y = torch.full_like(x, float("nan"))
+        torch.cuda.synchronize()
+        if before is None:
+            before = hip.pool_used(False)
+        hip.pool_used(True)
+        thff.ThunderFFT_conv2d_async(T, size, size, x, h, y, 1, s.value)
+        hip.call("hipStreamSynchronize", s)
+        kept.append((hip.pool_used(True) - before, hip.pool_used(False) - before))
+        hip.destroy(s)
+        ref = torch.empty_like(x)
+        thff.ThunderFFT_conv2d_noalloc(T, size, size, x, h, ref, 1)
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), ref.view(torch.int16)), i
+    one = kept[0][1]
+    assert one >= 8 << 20, kept
+    assert [k[1] for k in kept] == [one * min(i + 1, 4) for i in range(12)], kept
+    assert all(k[0] <= 4 * one for k in kept), kept
+    thff.ThunderFFTFinalize(T)
+    assert hip.pool_used(False) == before
+
+
+def test_conv2d_workspace_taken_over_during_a_capture():
+    """Six streams in turn while another is being captured: the captured call and
+    the others give the results of the calls alone, replay after replay."""
+    import torch
+
+    import thunderfft_amd as thff
+
+    size, T = 1024, "half"
+    thff.ThunderFFTInitialize(T, size)
+    gen = torch.Generator(device="cuda").manual_seed(13)
+    x = torch.randn(2 * size * size, device="cuda", generator=gen).half()
+    filters = [(torch.randn(2 * size * size, device="cuda", generator=gen) / size).half()
+               for _ in range(7)]
+    refs = [torch.empty_like(x) for _ in filters]
+    for h, r in zip(filters, refs):
+        thff.ThunderFFT_conv2d_noalloc(T, size, size, x, h, r, 1)
+    outs = [torch.full_like(x, float("nan")) for _ in filters]
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    for k, s in enumerate(streams):  # the workspaces, before the capture
+        thff.ThunderFFT_conv2d_async(T, size, size, x, filters[k], outs[k], 1, s)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        thff.ThunderFFT_conv2d_noalloc(T, size, size, x, filters[6], outs[6], 1, side)
+        for k, s in enumerate(streams):
+            thff.ThunderFFT_conv2d_async(T, size, size, x, filters[k], outs[k], 1, s)
+    torch.cuda.synchronize()
+
+    def check(which):
+        for k in which:
+            assert torch.equal(outs[k].view(torch.int16), refs[k].view(torch.int16)), k
+
+    check(range(6))
+    for _ in range(3):
+        outs[6].fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        check(range(7))

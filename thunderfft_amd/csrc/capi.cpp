@@ -100,14 +100,16 @@ int scratch_address(int device, float2** out) {
 // and freeing one stream-ordered took 23 us of host time a call (the three
 // launches take 10), and a synchronised call 45 us more, the pool giving the
 // memory back each time.  At most kMaxWorkspaces per device (33 MiB), one for
-// each stream that calls; further streams, hipStreamPerThread (one handle for
-// many streams) and captured calls allocate for the call as before, and so
-// does a call whose stream's workspace another thread is enqueueing with.
+// each stream that calls; a further stream takes over an idle one whose last
+// use has finished, so that streams that come and go do not use them up.  While
+// all are in use, a further stream allocates for the call, and so do
+// hipStreamPerThread (one handle for many streams), captured calls and a call
+// whose stream's workspace another thread is enqueueing with.
 // The next user waits for the event that the last one recorded, so a
 // workspace is safe even if its stream was destroyed and the handle belongs to
 // another stream now.  The null stream, which is never another, orders its
-// calls by itself: no event there (3 us of its time).  Finalize gives them
-// back.
+// calls by itself: no event there (3 us of its time), so its workspace is not
+// taken over.  Finalize gives them back.
 constexpr size_t kWorkspaceBytes = thff::kConv2d1024WorkspaceBytes;
 constexpr int kMaxWorkspaces = 4;
 struct Workspace {
@@ -121,6 +123,20 @@ struct DeviceWorkspaces {
     Workspace slots[kMaxWorkspaces];
 };
 DeviceWorkspaces g_workspaces[kMaxDevices];
+
+// Whether the last use of a workspace that is not the null stream's has
+// finished.  (The query would end another thread's capture in progress.)
+bool finished(const Workspace& w) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const hipError_t err = hipEventQuery(w.done);
+    if (err != hipSuccess) (void)hipGetLastError();  // hipErrorNotReady among others
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return err == hipSuccess;
+}
 
 // A kept workspace ready for work on `s`, or null (allocate for the call).
 Workspace* acquire_workspace(int device, hipStream_t s) {
@@ -146,6 +162,12 @@ Workspace* acquire_workspace(int device, hipStream_t s) {
             }
             if (!found) found = &w, fresh = true;
         }
+        if (!found)
+            for (auto& w : all.slots)
+                if (!w.busy && w.stream && finished(w)) {
+                    found = &w;
+                    break;
+                }
         if (!found) return nullptr;
         found->busy = true;
         found->stream = s;
@@ -173,6 +195,7 @@ Workspace* acquire_workspace(int device, hipStream_t s) {
 // Behind the call's last launch on `s`.
 hipError_t release_workspace(int device, Workspace* w, hipStream_t s) {
     const hipError_t err = s ? hipEventRecord(w->done, s) : hipSuccess;
+    if (err != hipSuccess) (void)hipStreamSynchronize(s);  // the event says nothing of this use
     std::lock_guard<std::mutex> lock(g_workspaces[device].mutex);
     w->busy = false;
     return err;
