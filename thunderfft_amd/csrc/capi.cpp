@@ -113,8 +113,11 @@ int scratch_address(int device, float2** out) {
 constexpr size_t kWorkspaceBytes = thff::kConv2d1024WorkspaceBytes;
 constexpr int kMaxWorkspaces = 4;
 struct Workspace {
+    // Written by the thread that made the slot busy, outside the lock: others
+    // look at them only after they saw, under the lock, that it is not.
     void* memory = nullptr;
     hipEvent_t done = nullptr;  // recorded behind the last call that used it
+    // Under the lock.
     hipStream_t stream = nullptr;
     bool busy = false;  // a thread is enqueueing with it
 };
@@ -153,7 +156,7 @@ Workspace* acquire_workspace(int device, hipStream_t s) {
     {
         std::lock_guard<std::mutex> lock(all.mutex);
         for (auto& w : all.slots) {
-            if (w.memory || w.busy) {
+            if (w.busy || w.memory) {
                 if (w.stream != s) continue;
                 if (w.busy) return nullptr;
                 found = &w;
@@ -206,7 +209,7 @@ void free_workspaces(int device) {
     DeviceWorkspaces& all = g_workspaces[device];
     std::lock_guard<std::mutex> lock(all.mutex);
     for (auto& w : all.slots) {
-        if (!w.memory || w.busy) continue;
+        if (w.busy || !w.memory) continue;
         if (w.stream)
             (void)hipEventSynchronize(w.done);
         else
