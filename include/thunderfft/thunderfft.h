@@ -176,7 +176,8 @@ int thff_conv1d_valid_async(int precision, const void* d_x, long long input_len,
  * 128: one fused kernel (forward 2-D FFT, product, inverse) per image, the
  * image on chip.  rows = cols = 1024 (the reference's sample shape): row FFTs
  * x -> y, and of the filter into an 8.25 MiB workspace (up to 4 per device are
- * kept until thff_finalize, for the streams that call; a further stream takes
+ * kept for the streams that call, until thff_finalize leaves neither precision
+ * initialised on the device; a further stream takes
  * over one that is not in use; if there is none, and for captured calls, one is
  * allocated and freed stream-ordered, hipMallocAsync), a column pass (FFT,
  * product, inverse FFT) and inverse row FFTs in place in y.  Other shapes -> THFF_EINVAL; requires thff_initialize(precision, rows).

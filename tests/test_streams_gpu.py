@@ -315,6 +315,7 @@ def test_conv2d_workspaces_outlive_their_streams():
 
     size, T = 1024, "half"
     hip = _Hip()
+    thff.ThunderFFTFinalize("float")
     thff.ThunderFFTFinalize(T)
     thff.ThunderFFTInitialize(T, size)
     gen = torch.Generator(device="cuda").manual_seed(12)
@@ -342,6 +343,37 @@ def test_conv2d_workspaces_outlive_their_streams():
     assert [k[1] for k in kept] == [one * min(i + 1, 4) for i in range(12)], kept
     assert all(k[0] <= 4 * one for k in kept), kept
     thff.ThunderFFTFinalize(T)
+    assert hip.pool_used(False) == before
+
+
+def test_conv2d_workspaces_last_as_long_as_a_precision_that_uses_them():
+    """Finalize of one precision leaves the workspaces to the other, with work
+    on them in flight; the last one gives them back."""
+    import torch
+
+    import thunderfft_amd as thff
+
+    size = 1024
+    hip = _Hip()
+    for T in ("float", "half"):
+        thff.ThunderFFTFinalize(T)
+    before = hip.pool_used(False)
+    x = torch.randn(2 * size * size, device="cuda")
+    h = torch.randn(2 * size * size, device="cuda") / size
+    y, ref = torch.empty_like(x), torch.empty_like(x)
+    for T in ("float", "half"):
+        thff.ThunderFFTInitialize(T, size)
+    thff.ThunderFFT_conv2d_noalloc("float", size, size, x, h, ref, 1)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(20):
+        thff.ThunderFFT_conv2d_async("float", size, size, x, h, y, 1, s)
+    kept = hip.pool_used(False) - before
+    thff.ThunderFFTFinalize("half")
+    assert kept >= 8 << 20 and hip.pool_used(False) - before == kept
+    thff.ThunderFFT_conv2d("float", size, size, x, h, y, 1, s)
+    assert torch.equal(y, ref)
+    thff.ThunderFFTFinalize("float")
     assert hip.pool_used(False) == before
 
 

@@ -109,7 +109,8 @@ int scratch_address(int device, float2** out) {
 // workspace is safe even if its stream was destroyed and the handle belongs to
 // another stream now.  The null stream, which is never another, orders its
 // calls by itself: no event there (3 us of its time), so its workspace is not
-// taken over.  Finalize gives them back.
+// taken over.  The Finalize after which neither precision is initialised on the
+// device gives them back (both precisions use them).
 constexpr size_t kWorkspaceBytes = thff::kConv2d1024WorkspaceBytes;
 constexpr int kMaxWorkspaces = 4;
 struct Workspace {
@@ -204,7 +205,7 @@ hipError_t release_workspace(int device, Workspace* w, hipStream_t s) {
     return err;
 }
 
-// Frees the device's idle workspaces (the current device).
+// Waits for and frees the device's idle workspaces (the current device).
 void free_workspaces(int device) {
     DeviceWorkspaces& all = g_workspaces[device];
     std::lock_guard<std::mutex> lock(all.mutex);
@@ -632,8 +633,10 @@ int thff_finalize(int precision) {
     int device = 0;
     DeviceTables* d = device_tables(precision, "hipGetDevice (finalize)", &device);
     if (!d) return THFF_EIO;
-    free_workspaces(device);
-    d->current.store(0, std::memory_order_release);
+    // Sequentially consistent: of two Finalize calls at once, at least one
+    // sees both precisions released.
+    d->current.store(0);
+    if (g_tables[1 - precision][device].current.load() == 0) free_workspaces(device);
     hipError_t first = hipSuccess;
     for (auto& slot : d->table) {
         float2* table = slot.exchange(nullptr, std::memory_order_acq_rel);
