@@ -363,11 +363,15 @@ def test_grids_for_few_tiles(T, n, tiles_per_cu):
         _large_case(T, n, batch, directions=(True,))
 
 
-@pytest.mark.parametrize("n,line", [(n, v) for n, end in ((128, 3 << 22), (512, 3 << 22), (1024, 3 << 20))
+@pytest.mark.parametrize("n,line", [(n, v) for n, end in ((128, 3 << 22), (512, 3 << 22), (1024, "3 tiles per CU"))
                                     for v in (1 << 21, end)])
 def test_store_forms_at_their_lines(n, line):
     """fp32 N = 128, 512 and 1024 store through the L2 up to 2^21 values and from
-    3 * 2^22 (N = 1024: 3 * 2^20) on: both sides of both lines."""
+    3 * 2^22 (N = 1024: 3 tiles of 4096 per CU) on: both sides of both lines."""
+    import torch
+
+    if not isinstance(line, int):
+        line = 3 * torch.cuda.get_device_properties(0).multi_processor_count * 4096
     for batch in (line // n - 1, line // n, line // n + 1):
         _large_case("float", n, batch, directions=(True, False))
 

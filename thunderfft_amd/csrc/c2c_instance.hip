@@ -94,25 +94,28 @@ inline constexpr bool kHalfOnMfma128 = N == 128;
 
 // Only the launch shape in use is instantiated.
 template <class IO, int N, bool FWD>
-void enqueue(Grid g, const IO* x, IO* y, int batch, const float2* tw, hipStream_t stream) {
+void enqueue(Grid g, const IO* x, IO* y, int batch, const float2* tw, int num_cus,
+             hipStream_t stream) {
     constexpr LaunchShape kShape = launch_shape<N>(std::is_same_v<IO, float2> ? 0 : 1);
     // Whole lines, written through (fp32 N = 256 172.4 against 174.7 us, 2048
     // 178.5 against 180.9, 1024 171.2 against 173.6; half2 N = 64 84.9 against
     // 86.6), but for fp32 N = 64 (2^22 values 12.4 against 10.8 us) and 4096
     // (1025 signals 5% slower).
     constexpr bool kThrough = !std::is_same_v<IO, float2> || (N > 64 && N < 4096);
-    // fp32 N = 128, 512 and 1024 leave the lines in the L2 where both arrays
-    // fit the memory-side cache and are more than 2^21 values: N = 128 up to
-    // 3 * 2^22 (18820 signals 7.6 us, written through 8.0; 32768 12.8, 13.1;
-    // 65536 24.5, 24.8), N = 512 likewise (5042 signals 8.7, 9.9; 8192 13.8,
-    // 14.1; 16384 25.3, 25.5), N = 1024 as long as every tile runs at once, 3
-    // per CU (2702 signals 8.4, 8.6; 3104 12.1, 11.5).  N = 256 gains from the
-    // write-through there (10809 signals 10.1, 9.6), and so do all outside
-    // (N = 128: 16384 signals 6.3, 6.1, 131072 45.5, 44.9).
+    // fp32 N = 128, 512 and 1024 leave the lines in the L2 for mid-size batches.
+    // Above 2^21 values, where the two arrays are more than the 32 MiB of the
+    // eight L2s (N = 128: 16384 signals 6.3 us, written through 6.1).  N = 128
+    // and 512 below 3 * 2^22 values, 192 of the memory-side cache's 256 MiB
+    // (N = 128: 18820 signals 7.6, 8.0; 32768 12.8, 13.1; 65536 24.5, 24.8;
+    // 131072 45.5, 44.9; N = 512: 5042 signals 8.7, 9.9; 8192 13.8, 14.1; 16384
+    // 25.3, 25.5).  N = 1024 as long as every tile runs at once, 3 per CU (2702
+    // signals 8.4, 8.6; 3104, with a second round, 12.1, 11.5).  N = 256 gains
+    // from the write-through there too (10809 signals 10.1, 9.6; the cause is
+    // not known: N = 512 stores the same way).
     if constexpr (std::is_same_v<IO, float2> && (N == 128 || N == 512 || N == 1024)) {
-        constexpr long long kEnd = N == 1024 ? 3LL << 20 : 3LL << 22;
+        const long long end = N == 1024 ? 3LL * num_cus * C2CPlan<N>::kTile : 3LL << 22;
         const long long values = static_cast<long long>(batch) * N;
-        if (values > 1LL << 21 && values < kEnd) {
+        if (values > 1LL << 21 && values < end) {
             c2c_kernel<IO, N, FWD, kShape.prefetch, kShape.direct><<<g.blocks, 256, 0, stream>>>(
                 x, y, batch, tw, g.tiles_per_block);
             return;
@@ -237,9 +240,9 @@ hipError_t launch_c2c(int precision, bool forward, bool aligned16, const void* i
         const auto* x = static_cast<const float2*>(in);
         auto* y = static_cast<float2*>(out);
         if (forward)
-            enqueue<float2, N, true>(g, x, y, batch, tw, stream);
+            enqueue<float2, N, true>(g, x, y, batch, tw, num_cus, stream);
         else
-            enqueue<float2, N, false>(g, x, y, batch, tw, stream);
+            enqueue<float2, N, false>(g, x, y, batch, tw, num_cus, stream);
     } else {
         const auto* x = static_cast<const __half2*>(in);
         auto* y = static_cast<__half2*>(out);
@@ -259,9 +262,9 @@ hipError_t launch_c2c(int precision, bool forward, bool aligned16, const void* i
             else
                 enqueue_mfma128<false>(g, x, y, batch, stream);
         } else if (forward) {
-            enqueue<__half2, N, true>(g, x, y, batch, tw, stream);
+            enqueue<__half2, N, true>(g, x, y, batch, tw, num_cus, stream);
         } else {
-            enqueue<__half2, N, false>(g, x, y, batch, tw, stream);
+            enqueue<__half2, N, false>(g, x, y, batch, tw, num_cus, stream);
         }
     }
     return hipGetLastError();
