@@ -24,8 +24,9 @@ namespace thff {
 //     both operands use it), and receives the 16 bytes q of output chunk n.
 //   half2: v_mfma_f32_16x16x32_f16, one instruction per chunk and output
 //     half.  A tap enters as the sum of two f16 values (scaled by a power of
-//     two so that the largest has exponent 10: about 22 bits of every tap),
-//     the sums are fp32, and outputs are rounded once.
+//     two so that the largest has exponent 10: within 2^-23 of itself or 2^-35
+//     of the largest, whichever is more), the sums are fp32, and outputs are
+//     rounded once.
 // What bounds it: HBM up to F of about 30 (float2) and for every F in half2;
 // beyond that the fp32 matrix rate, 4 A instructions of 32 cycles per 128
 // outputs.  Against overlap-save transforms (float2 64-point windows, of which

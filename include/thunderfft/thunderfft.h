@@ -147,7 +147,10 @@ int thff_conv1d_real_async(int precision, int n, const void* d_x, const void* d_
 /* Valid 1-D correlation with a short filter, the result of the reference's
  * conv1d_direct_fft_kernel (sample/conv1d/main.cu:38-128, driven by main
  * :207-336 with the definition of :156-174), which tiles it in 64-point FFT
- * windows; here the sum itself, on the matrix cores:
+ * windows; here the sum itself, on the matrix cores (a non-finite input value
+ * makes NaN of some neighbouring outputs that do not depend on it, up to two
+ * 64-byte chunks of values before those that do and the rest of its own chunk
+ * after them; the reference's windows spread it over their 64 points):
  *   y[b][i] = sum_{k < filter_len} x[b][i + k] * taps[k],  i < input_len - filter_len + 1,
  * complex, no conjugation.  x holds batch signals of input_len values and y
  * batch outputs of input_len - filter_len + 1 values, both in `precision`

@@ -14,9 +14,9 @@ y[i] = sum_k x[i + k] f[k] (:156-174).  Here:
 * batches of odd-length signals, input_len == filter_len, every filter
   length 1..64 on a short signal, with output sentinels;
 * at 2^24 samples the property that a unit impulse at tap k0 shifts the
-  signal, y[i] = x[i + k0]: per output for float (fp32 arithmetic), against
-  the signal scale for half (its 256-point windows run on MFMA with f16
-  data at each DFT16 stage).
+  signal, y[i] = x[i + k0]: per output;
+* the edges of the kernel's spans and of its matrix's steps, taps and signals
+  of very different size, per output against a derived bound.
 """
 import numpy as np
 import pytest
@@ -27,8 +27,8 @@ from thff_testlib import GATE, from_device, to_device
 pytestmark = pytest.mark.gpu
 
 TIGHT = {"float": 2e-6, "half": 1e-3}
-# The half path runs its 256-point windows on MFMA with f16 data at each
-# DFT16 stage: per-output errors are bounded against the signal scale.
+# Per-output errors of the half path, whose outputs are rounded once, against
+# the signal scale; test_span_edges_and_tap_scales holds each to its own bound.
 HALF_MAX_ABS = 5e-3
 GUARD = 16
 GUARD_VALUE = -271.0 + 137.0j
@@ -193,19 +193,22 @@ def test_signal_beyond_2e31_values(T):
 def test_span_edges_and_tap_scales(T):
     """Outputs one below, at and above whole spans (512 float, 1024 half, four
     waves each) and filters one below, at and above a step of the matrix, with
-    taps of any size.  Per output, S = sum |x||taps|:
+    taps of any size (spread over 2^20 in one filter), and signals of f16
+    subnormals.  Per output, S = sum |x||taps|:
       float: 4 chains of F/2 products and their sum, (F/2 + 4) 2^-23 S;
-      half: taps to 2^-21 of the largest, the same sums, one rounding to f16
-      (2^-11 of the result, 2^-24 at least)."""
+      half: taps to 2^-23 of themselves or 2^-35 of the largest, the same sums,
+      one rounding to f16 (2^-11 of the result, 2^-24 at least)."""
     rng = np.random.default_rng(512)
     span = 512 if T == "float" else 1024
     for ntaps in (1, 2, 8, 9, 10, 17, 18, 41, 42, 49, 50, 57, 58, 64):
         for out, batch in ((1, 5), (span - 1, 2), (span, 1), (span + 1, 3), (4 * span + 1, 1)):
-            for scale in (1.0, 2.0 ** -12, 2.0 ** 9):
+            for scale, spread, level in ((1.0, 6, 0), (2.0 ** -12, 20, 0), (2.0 ** 9, 6, 0), (1.0, 20, 0),
+                                         (2.0 ** 9, 6, -15)):
                 length = out + ntaps - 1
                 x = rng.uniform(-1, 1, (batch, length)) + 1j * rng.uniform(-1, 1, (batch, length))
+                x *= 2.0 ** level
                 f = rng.normal(size=ntaps) + 1j * rng.normal(size=ntaps)
-                f = (f * scale * 2.0 ** rng.integers(-6, 1, ntaps)).astype(np.complex64)
+                f = (f * scale * 2.0 ** rng.integers(-spread, 1, ntaps)).astype(np.complex64)
                 xr = oracle.represent(x.astype(np.complex64), T)
                 y, guards = run(T, xr, f, batch)
                 want = np.asarray(oracle.conv1d_valid(xr, f)).reshape(batch, out)
@@ -214,7 +217,7 @@ def test_span_edges_and_tap_scales(T):
                 if T == "float":
                     bound = (ntaps / 2 + 4) * 2.0 ** -23 * size
                 else:
-                    bound = ((ntaps / 2 + 4) * 2.0 ** -23 * size + 2.0 ** -11 * np.abs(want) + 2.0 ** -24
-                             + 2.0 ** -21 * np.abs(f).max() * np.abs(xr).max() * ntaps)
+                    bound = ((ntaps / 2 + 5) * 2.0 ** -23 * size + 2.0 ** -11 * np.abs(want) + 2.0 ** -24
+                             + 2.0 ** -35 * np.abs(f).max() * np.abs(xr).max() * ntaps)
                 worst = float(np.max(np.abs(y - want) / bound))
-                assert guards == 0 and worst <= 1.0, (T, ntaps, out, batch, scale, worst)
+                assert guards == 0 and worst <= 1.0, (T, ntaps, out, batch, scale, spread, level, worst)
