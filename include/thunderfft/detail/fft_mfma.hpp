@@ -253,7 +253,7 @@ struct Stage3Plain {
 };
 
 // Workgroup set-up of the MFMA kernels for direction FWD, computed with the
-// hardware sine and cosine (cis_rev, 1e-7): this lane's plain DFT16 operands, the step-2 twiddles
+// hardware sine and cosine (cis_rev): this lane's plain DFT16 operands, the step-2 twiddles
 // W_N^(t*k1) (t = 16c + n, k1 = q + 4r) shared through LDS as
 // w1 = [c][r][lane], and for the stage before the last DFT16 either the
 // folded operands a3 (Stage3Folded; a3 non-null) or this lane's twiddles

@@ -283,8 +283,33 @@ __global__ __launch_bounds__(256) void repeat_mfma_split(const float2* in, float
     }
 }
 
+// The computed coefficients of a denominator: entries[num][inverse][o][p] and
+// cis[num], num < den, one num per lane.
+__global__ __launch_bounds__(256) void coefficients(_Float16* entries, float2* cis, int den) {
+    const int num = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    if (num >= den) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        entries[8 * num + e] = rotation_entry<true>(num, den, e / 2, e % 2);
+        entries[8 * num + 4 + e] = rotation_entry<false>(num, den, e / 2, e % 2);
+    }
+    const cpx w = cis_rev(num, den);
+    cis[num] = make_float2(w.re, w.im);
+}
+
 }  // namespace
 }  // namespace thff
+
+// What the fp16 kernels compute instead of reading tables: for every num < den
+// (den a power of two from 4 to 4096) the eight f16 entries of a rotation by
+// num / den of a revolution ([forward, inverse][output part][input part]) and
+// its (cos, sin).  Returns 0, -22 or -5 as below.  Asynchronous on `stream`.
+extern "C" int thffx_coefficients(int den, void* entries, void* cis, void* stream) {
+    if (den < 4 || den > 4096 || (den & (den - 1)) || !entries || !cis) return -22;
+    thff::coefficients<<<(den + 255) / 256, 256, 0, static_cast<hipStream_t>(stream)>>>(
+        static_cast<_Float16*>(entries), static_cast<float2*>(cis), den);
+    return hipGetLastError() == hipSuccess ? 0 : -5;
+}
 
 // One launch of the repeat kernel for N = 1024 over `batch` transforms
 // (a multiple of the tile size); precision 0 float (VALU), 1 half (MFMA),
