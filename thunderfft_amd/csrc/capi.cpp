@@ -458,8 +458,11 @@ int conv1d_valid_impl(int precision, const void* x, long long input_len, const v
     if ((reinterpret_cast<std::uintptr_t>(x) | reinterpret_cast<std::uintptr_t>(y)) % elem ||
         reinterpret_cast<std::uintptr_t>(taps) % 8)
         return fail(THFF_EINVAL, "ThunderFFT_conv1d_valid: misaligned pointer");
-    // The most that one call takes, counted in groups of 64 windows of 64
-    // points (fp32) or 16 of 256 (fp16): at least 2^30 outputs.
+    // The most that one call takes: what fitted one launch of groups of 64
+    // windows of 64 points (fp32) or 16 of 256 (fp16), the overlap-save form of
+    // this call.  The matrix product's kernel counts in 64 bits and its grid is
+    // the device's; the limit stays where callers know it.  At F = 64 (one
+    // valid output per fp32 window) it is 2^30 outputs, else more.
     const long long window = precision == THFF_FLOAT ? 64 : 256;
     const long long per_group = precision == THFF_FLOAT ? 64 : 16;
     const long long valid = window + 1 - filter_len;
