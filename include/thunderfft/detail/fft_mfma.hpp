@@ -81,21 +81,23 @@ __device__ __forceinline__ _Float16 rotation_entry(int num, int den, int o, int 
 // j = q + 4 e (e = 0..3) instead of 4 q + e: the columns are permuted to match,
 // so a transform can consume another transform's output registers (whose
 // lane group q holds outputs q + 4 r) without moving them.
+// Half 1's outputs are half 0's plus 8, so its entries are half 0's, negated
+// at odd j: half the cosines.
 template <bool FWD, bool kInterleaved = false>
 __device__ __forceinline__ void dft16_operands(f16x8 (&a)[2], int lane) {
     const int m = lane & 15, q = lane >> 4;
-    const int gq = m >> 2, i = m & 3;
+    const int k = (m >> 2) + 4 * ((m & 3) >> 1);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int k = gq + 4 * (2 * h + (i >> 1));
-        const int o = i & 1;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int kk = 8 * q + e;
-            const int j = kInterleaved ? (kk >> 3) + 4 * ((kk >> 1) & 3) : kk >> 1;
-            a[h][e] = rotation_entry<FWD>(j * k, 16, o, kk & 1);
-        }
+    for (int e = 0; e < 8; ++e) {
+        const int j = kInterleaved ? q + 4 * (e >> 1) : 4 * q + (e >> 1);
+        a[0][e] = rotation_entry<FWD>(j * k, 16, m & 1, e & 1);
     }
+    u32x4 w = __builtin_bit_cast(u32x4, a[0]);
+    if constexpr (kInterleaved)
+        w ^= (q & 1) * 0x80008000u;
+    else
+        w ^= u32x4{0, 0x80008000u, 0, 0x80008000u};
+    a[1] = __builtin_bit_cast(f16x8, w);
 }
 
 // The DFT16 operands of dft16_operands<FWD> (plain input order) with the
@@ -970,16 +972,18 @@ template <bool FWD, bool kPermuted = false>
 __device__ __forceinline__ void dft8_pair_operands(f16x8 (&a)[2], int lane) {
     const int m = lane & 15, kq = lane >> 4;
     const int k1 = m >> 1, o = m & 1;
+    const int seq = kPermuted ? (kq & 1) : kq >> 1;
+    f16x8 v;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int slot = e >> 1, p = e & 1;
-            const int seq = kPermuted ? (kq & 1) : kq >> 1;
-            const int j = kPermuted ? 2 * slot + (kq >> 1) : 4 * (kq & 1) + slot;
-            a[h][e] = seq == h ? rotation_entry<FWD>(j * k1, 8, o, p) : static_cast<_Float16>(0.0f);
-        }
+    for (int e = 0; e < 8; ++e) {
+        const int slot = e >> 1, p = e & 1;
+        const int j = kPermuted ? 2 * slot + (kq >> 1) : 4 * (kq & 1) + slot;
+        v[e] = rotation_entry<FWD>(j * k1, 8, o, p);
     }
+    const u32x4 w = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        a[h] = __builtin_bit_cast(f16x8, seq == h ? w : u32x4{});
 }
 
 template <bool FWD, bool kPrefetch>
