@@ -171,10 +171,11 @@ def test_partial_tiles_keep_to_the_output(T, n):
 @pytest.mark.parametrize("T", ["float", "half"])
 @pytest.mark.parametrize("n", SIZES)
 def test_element_aligned_buffers_at_the_staging_threshold(T, n):
-    """2^21 values, where float (and half up to N = 256) moves 16 bytes at the
-    element's alignment, and just below, with a partial last tile: the result
-    is that of the aligned call, to the rounding of two correct transforms
-    (twice TIGHT), and nothing around the output changes."""
+    """The values from which float (and half up to N = 256) moves 16 bytes at the
+    element's alignment (a tile at N = 64, 2^19 at 128, 2^21), and just below,
+    with a partial last tile: the result is that of the aligned call, to the
+    rounding of two correct transforms (twice TIGHT), and nothing around the
+    output changes."""
     import torch
 
     import thunderfft_amd as thff
@@ -182,7 +183,8 @@ def test_element_aligned_buffers_at_the_staging_threshold(T, n):
     esize = 8 if T == "float" else 4
     dt = torch.float32 if T == "float" else torch.float16
     thff.ThunderFFTInitialize(T, n)
-    for batch in ((1 << 21) // n + 3, (1 << 21) // n - 1):
+    line = {64: 4096, 128: 1 << 19}.get(n, 1 << 21) // n
+    for batch in sorted({(1 << 21) // n + 3, (1 << 21) // n - 1, line - 1, line, line + 1}):
         count = batch * n
         x = torch.empty(2 * count + 8, dtype=dt, device="cuda")
         thff.fill_uniform(T, x, count + 4, 5 + n)
@@ -190,7 +192,7 @@ def test_element_aligned_buffers_at_the_staging_threshold(T, n):
             src = x[2 * in_off:2 * (in_off + count)]
             ref = torch.empty(2 * count, dtype=dt, device="cuda")
             thff.ThunderFFT_global(T, n, True, src.clone(), ref, batch)
-            out = torch.full((2 * (out_off + count) + 32,), 7.0, dtype=dt, device="cuda")
+            out = torch.full((2 * (out_off + count) + 12288,), 7.0, dtype=dt, device="cuda")
             thff.ThunderFFT_global(T, n, True, x.data_ptr() + in_off * esize,
                                    out.data_ptr() + out_off * esize, batch)
             got = out[2 * out_off:2 * (out_off + count)]

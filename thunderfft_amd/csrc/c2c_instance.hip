@@ -171,8 +171,13 @@ void enqueue_mfma3(Grid g, const __half2* x, __half2* y, int batch, hipStream_t 
 // N = 64 188 against 313 us); it saves the staging's latency in small calls
 // (fp32 N = 1024, 1023 signals: 5.8 against 6.2 us), and for half2 from
 // N = 512 on the staging costs more than the accesses (N = 1024, 2^26 values:
-// 111 against 125 us).  The rest is staged from 2^21 values on (fp32 N = 1024,
-// 2895 signals: 9.7 against 12.1 us; half2 N = 256, 16383: 8.1 against 11.1).
+// 111 against 125 us).  Staged are
+//   N = 64 from a whole tile on (64 signals: fp32 3.64 against 3.69 us, half2
+//     3.54, 3.64; 16 signals 3.41, 2.85 and 3.28, 2.80);
+//   N = 128 from 2^19 values (fp32: 2048 signals 4.34, 4.10, 4096 4.64, 4.64,
+//     8192 5.52, 5.77; half2: 4.08, 3.90, 4.18, 4.18, 4.48, 4.85);
+//   the rest from 2^21 values (fp32 N = 1024, 2895 signals: 9.7, 12.1; half2
+//     N = 256, 16383: 8.1, 11.1).
 template <class IO, int N, bool kDirect>
 void enqueue_unaligned(bool forward, const IO* x, IO* y, int batch, const float2* tw,
                        hipStream_t stream) {
@@ -188,12 +193,14 @@ void enqueue_unaligned(bool forward, const IO* x, IO* y, int batch, const float2
 template <class IO, int N>
 void enqueue_unaligned(bool forward, const IO* x, IO* y, int batch, const float2* tw,
                        hipStream_t stream) {
-    constexpr bool kAlwaysStaged = N <= 128;
-    constexpr bool kAlwaysDirect = std::is_same_v<IO, __half2> && N >= 512;
-    if (kAlwaysStaged || (!kAlwaysDirect && static_cast<long long>(batch) * N >= (1LL << 21)))
-        enqueue_unaligned<IO, N, kAlwaysDirect>(forward, x, y, batch, tw, stream);
-    else
-        enqueue_unaligned<IO, N, !kAlwaysStaged>(forward, x, y, batch, tw, stream);
+    if constexpr (std::is_same_v<IO, float2> || N <= 256) {
+        constexpr long long kStaged = N == 64 ? C2CPlan<N>::kTile : N == 128 ? 1LL << 19 : 1LL << 21;
+        if (static_cast<long long>(batch) * N >= kStaged) {
+            enqueue_unaligned<IO, N, false>(forward, x, y, batch, tw, stream);
+            return;
+        }
+    }
+    enqueue_unaligned<IO, N, true>(forward, x, y, batch, tw, stream);
 }
 
 template <int N>
