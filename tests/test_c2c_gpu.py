@@ -365,6 +365,25 @@ def test_grids_for_few_tiles(T, n, tiles_per_cu):
         _large_case(T, n, batch, directions=(True,))
 
 
+@pytest.mark.parametrize("n,line", [(256, 4096), (512, 1 << 16), (1024, 1 << 19), (2048, 4096)])
+def test_store_forms_of_small_calls(n, line):
+    """fp32 N = 256 ... 2048 store through the L2 from a whole tile, 2^16 or 2^19
+    values on: both sides of each line, with sentinels on both sides."""
+    import thunderfft_amd as thff
+
+    thff.ThunderFFTInitialize("float", n)
+    for batch in (line // n - 1, line // n, line // n + 1):
+        x = oracle.uniform(n, batch, seed=n + batch)
+        d_x = to_device(x, "float")
+        for forward in (True, False):
+            y, intact = tile_guarded_output(batch * n, "float")
+            thff.ThunderFFT_global("float", n, forward, d_x, y, batch)
+            m = oracle.metrics(from_device(y, "float"), oracle.fft(x, forward=forward).reshape(-1))
+            label = (n, batch, forward, m["rel_l2"])
+            assert intact(), label
+            assert m["nonfinite"] == 0 and m["rel_l2"] <= TIGHT["float"], label
+
+
 @pytest.mark.parametrize("n,line", [(n, v) for n, end in ((128, 3 << 22), (512, 3 << 22), (1024, "3 tiles per CU"))
                                     for v in (1 << 21, end)])
 def test_store_forms_at_their_lines(n, line):

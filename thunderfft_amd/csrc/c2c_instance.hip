@@ -112,10 +112,20 @@ void enqueue(Grid g, const IO* x, IO* y, int batch, const float2* tw, int num_cu
     // signals 8.4, 8.6; 3104, with a second round, 12.1, 11.5).  N = 256 gains
     // from the write-through there too (10809 signals 10.1, 9.6; the cause is
     // not known: N = 512 stores the same way).
-    if constexpr (std::is_same_v<IO, float2> && (N == 128 || N == 512 || N == 1024)) {
+    // Small fp32 calls leave them too: N = 256 and 2048 below a whole tile (4
+    // signals of 256 2.93 us, written through 3.23; 16 3.57, 3.54; 1 of 2048
+    // 4.54, 4.73, 2 4.98, 4.94), N = 512 up to 2^16 values (2 signals 3.57,
+    // 3.74; 128 4.28, 4.30; 512 4.43, 4.33), N = 1024 up to 2^19 (8 signals
+    // 4.55, 4.66; 128 4.81, 4.93; 512 5.07, 5.10; 768 5.47, 5.33).
+    if constexpr (std::is_same_v<IO, float2> && N >= 128 && N <= 2048) {
+        constexpr long long kSmall = N == 1024  ? 1LL << 19
+                                     : N == 512 ? 1LL << 16
+                                     : N == 128 ? 0
+                                                : C2CPlan<N>::kTile - 1;
+        constexpr bool kBand = N == 128 || N == 512 || N == 1024;
         const long long end = N == 1024 ? 3LL * num_cus * C2CPlan<N>::kTile : 3LL << 22;
         const long long values = static_cast<long long>(batch) * N;
-        if (values > 1LL << 21 && values < end) {
+        if (values <= kSmall || (kBand && values > 1LL << 21 && values < end)) {
             c2c_kernel<IO, N, FWD, kShape.prefetch, kShape.direct><<<g.blocks, 256, 0, stream>>>(
                 x, y, batch, tw, g.tiles_per_block);
             return;
