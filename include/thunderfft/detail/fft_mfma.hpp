@@ -60,7 +60,9 @@ __device__ __forceinline__ f32x4 mfma16x16x32(f16x8 a, f16x8 b, f32x4 c) {
 // cost no memory access.  Read from a table in memory they were 16 gathers per
 // lane and DFT16, and the twiddles (cis_rev now) 20 more in the three-stage
 // kernels, up to 64 lines each: 2 us of a CU's cache per workgroup, which
-// bounded small and ordinary batches.  Half2, in a graph of calls:
+// bounded small and ordinary batches.  Half2, in a graph of calls (with every
+// entry computed; the halves of a matrix from one set of cosines take 1-5% off
+// the first figures, 95.7 against 95.5 us to 9.0 against 8.6):
 //   C2C N = 4096, 1001 signals: 7.8 against 11.0 us; 16384: 89 against 91
 //   C2C N = 1024, 4003 signals: 7.8 against 8.4 us; 65535: 86.3 against 90
 //   conv1d N = 1024, 4097 signals, one filter: 12.4 against 15.8 us
@@ -74,6 +76,22 @@ __device__ __forceinline__ _Float16 rotation_entry(int num, int den, int o, int 
         static_cast<float>((num + shift) & (den - 1)) / static_cast<float>(den)));
 }
 
+// The same entries of one output part o, for a rotation by `rev` revolutions (a
+// multiple of 1/2048, exact in fp32): three operations and the cosine each,
+// where the integers above take five.  A half2 C2C of 8 signals of 128, most of
+// whose time is its two matrices, takes 2.99 us with these, 3.03 with
+// rotation_entry and 3.07 with the matrices from a table in memory; 512 signals
+// 3.38, 3.42 and 3.36.
+template <bool FWD>
+struct RotationRow {
+    float shift[2];  // by the input part
+    __device__ __forceinline__ explicit RotationRow(int o)
+        : shift{o == 0 ? 0.0f : (FWD ? 0.25f : -0.25f), o == 0 ? (FWD ? -0.25f : 0.25f) : 0.0f} {}
+    __device__ __forceinline__ _Float16 entry(float rev, int p) const {
+        return static_cast<_Float16>(__builtin_amdgcn_cosf(__builtin_amdgcn_fractf(rev + shift[p])));
+    }
+};
+
 // A-operand registers of the DFT16 matrix for this lane: [half].
 // Row m of half h is output k = m/4 + 4*(2h + (m%4)/2), part (m%4)%2;
 // column k' is input j = k'/2, part k'%2.
@@ -86,12 +104,12 @@ __device__ __forceinline__ _Float16 rotation_entry(int num, int den, int o, int 
 template <bool FWD, bool kInterleaved = false>
 __device__ __forceinline__ void dft16_operands(f16x8 (&a)[2], int lane) {
     const int m = lane & 15, q = lane >> 4;
-    const int k = (m >> 2) + 4 * ((m & 3) >> 1);
+    const float step = static_cast<float>((m >> 2) + 4 * ((m & 3) >> 1)) / 16.0f;  // k / 16
+    const float first = step * static_cast<float>(kInterleaved ? q : 4 * q);      // input j = first + ...
+    const RotationRow<FWD> row(m & 1);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int j = kInterleaved ? q + 4 * (e >> 1) : 4 * q + (e >> 1);
-        a[0][e] = rotation_entry<FWD>(j * k, 16, m & 1, e & 1);
-    }
+    for (int e = 0; e < 8; ++e)
+        a[0][e] = row.entry(first + step * static_cast<float>(kInterleaved ? 4 * (e >> 1) : e >> 1), e & 1);
     u32x4 w = __builtin_bit_cast(u32x4, a[0]);
     if constexpr (kInterleaved)
         w ^= (q & 1) * 0x80008000u;
@@ -971,15 +989,14 @@ struct Mfma2048 {
 template <bool FWD, bool kPermuted = false>
 __device__ __forceinline__ void dft8_pair_operands(f16x8 (&a)[2], int lane) {
     const int m = lane & 15, kq = lane >> 4;
-    const int k1 = m >> 1, o = m & 1;
     const int seq = kPermuted ? (kq & 1) : kq >> 1;
+    const float step = static_cast<float>(m >> 1) / 8.0f;  // k1 / 8
+    const float first = step * static_cast<float>(kPermuted ? kq >> 1 : 4 * (kq & 1));
+    const RotationRow<FWD> row(m & 1);
     f16x8 v;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int slot = e >> 1, p = e & 1;
-        const int j = kPermuted ? 2 * slot + (kq >> 1) : 4 * (kq & 1) + slot;
-        v[e] = rotation_entry<FWD>(j * k1, 8, o, p);
-    }
+    for (int e = 0; e < 8; ++e)
+        v[e] = row.entry(first + step * static_cast<float>(kPermuted ? 2 * (e >> 1) : e >> 1), e & 1);
     const u32x4 w = __builtin_bit_cast(u32x4, v);
 #pragma unroll
     for (int h = 0; h < 2; ++h)

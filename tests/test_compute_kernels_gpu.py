@@ -58,7 +58,7 @@ def test_computed_coefficients(den):
 
     L = ctypes.CDLL(LIB)
     L.thffx_coefficients.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
-    entries = torch.full((den, 2, 2, 2), float("nan"), dtype=torch.float16, device="cuda")
+    entries = torch.full((den, 2, 2, 2, 2), float("nan"), dtype=torch.float16, device="cuda")
     cis = torch.full((den, 2), float("nan"), device="cuda")
     assert L.thffx_coefficients(den, entries.data_ptr(), cis.data_ptr(), None) == 0
     torch.cuda.synchronize()
@@ -70,6 +70,7 @@ def test_computed_coefficients(den):
     # out.re = c in.re - s in.im, out.im = s in.re + c in.im; forward: s -> -s
     want = np.stack([np.stack([np.stack([c, -i * s], -1), np.stack([i * s, c], -1)], -2)
                      for i in (-1, 1)], 1)
+    want = np.stack([want, want], 1)  # both forms of an entry
     got = entries.cpu().numpy()
     if den <= 2048:
         assert np.array_equal(got, want.astype(np.float16))

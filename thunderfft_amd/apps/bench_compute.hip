@@ -283,15 +283,20 @@ __global__ __launch_bounds__(256) void repeat_mfma_split(const float2* in, float
     }
 }
 
-// The computed coefficients of a denominator: entries[num][inverse][o][p] and
-// cis[num], num < den, one num per lane.
+// The computed coefficients of a denominator: entries[num][form][inverse][o][p]
+// (form 0 rotation_entry, 1 RotationRow) and cis[num], num < den, one num per
+// lane.
 __global__ __launch_bounds__(256) void coefficients(_Float16* entries, float2* cis, int den) {
     const int num = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
     if (num >= den) return;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        entries[8 * num + e] = rotation_entry<true>(num, den, e / 2, e % 2);
-        entries[8 * num + 4 + e] = rotation_entry<false>(num, den, e / 2, e % 2);
+        const int o = e / 2, p = e % 2;
+        const float rev = static_cast<float>(num) / static_cast<float>(den);
+        entries[16 * num + e] = rotation_entry<true>(num, den, o, p);
+        entries[16 * num + 4 + e] = rotation_entry<false>(num, den, o, p);
+        entries[16 * num + 8 + e] = RotationRow<true>(o).entry(rev, p);
+        entries[16 * num + 12 + e] = RotationRow<false>(o).entry(rev, p);
     }
     const cpx w = cis_rev(num, den);
     cis[num] = make_float2(w.re, w.im);
@@ -301,9 +306,8 @@ __global__ __launch_bounds__(256) void coefficients(_Float16* entries, float2* c
 }  // namespace thff
 
 // What the fp16 kernels compute instead of reading tables: for every num < den
-// (den a power of two from 4 to 4096) the eight f16 entries of a rotation by
-// num / den of a revolution ([forward, inverse][output part][input part]) and
-// its (cos, sin).  Returns 0, -22 or -5 as below.  Asynchronous on `stream`.
+// (den a power of two from 4 to 4096) the f16 entries of a rotation by num / den
+// of a revolution ([form][forward, inverse][output part][input part]) and its (cos, sin).  Returns 0, -22 or -5 as below.  Asynchronous on `stream`.
 extern "C" int thffx_coefficients(int den, void* entries, void* cis, void* stream) {
     if (den < 4 || den > 4096 || (den & (den - 1)) || !entries || !cis) return -22;
     thff::coefficients<<<(den + 255) / 256, 256, 0, static_cast<hipStream_t>(stream)>>>(
