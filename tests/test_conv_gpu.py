@@ -247,7 +247,7 @@ def test_conv1d_grid_stride_walks(T, n, per_signal):
 
 
 @pytest.mark.parametrize("n", [64, 128, 256, 512, 1024, 2048])
-@pytest.mark.parametrize("tiles_per_cu", [4, 16])
+@pytest.mark.parametrize("tiles_per_cu", [4, 16, 20])
 def test_conv1d_grids_for_few_tiles(n, tiles_per_cu):
     """fp32, a shared filter up to N = 256 and per-signal filters above, takes
     its grid by the tiles per CU: one tile fewer than the line (one signal

@@ -293,9 +293,11 @@ hipError_t launch_c2c(int precision, bool forward, bool aligned16, const void* i
 // samples, 64 channels):
 //   complex fp32, per-signal filters: one tile per workgroup up to N = 256
 //     (130-133 us against 135-152 us for device grids); N = 512 ... 2048 3 per
-//     CU up to 16 tiles per CU (N = 1024: 4097 signals 22.0, 10086 46.3 us; one
-//     tile per workgroup 23.7, 49.7; N = 2048: 6 per CU 2-4% behind), beyond
-//     that 6 per CU, so that a finished workgroup's place is taken at once
+//     CU below 20 tiles per CU (N = 1024: 4097 signals 22.0, 10086 46.3 us; one
+//     tile per workgroup 23.7, 49.7; N = 2048: 6 per CU 2-4% behind, at 8192
+//     signals 78.8 against 74.6, at 9410 89.0 against 87.6), from there on
+//     (N = 2048: 11585 signals 106.2 against 106.9, 14263 126.4 against 135.1)
+//     6 per CU, so that a finished workgroup's place is taken at once
 //     (N = 512 136.9, 1024 140.0 us, one tile per workgroup 140.0, 145.6;
 //     N = 2048 146.3, 3 per CU 149.3);
 //     N = 4096 2 per CU (167 us; prefetch 192).
@@ -324,7 +326,7 @@ constexpr ConvShape valu_conv_shape(int precision, bool real, bool per_signal,
                                     long long tiles_per_cu) {
     if (precision != 0) return {4, Prefetch::kNone};
     if (real) return {2, N <= 512 ? Prefetch::kLate : Prefetch::kEarly};
-    if (per_signal) return {N <= 256 ? 0 : N == 4096 ? 2 : tiles_per_cu >= 16 ? 6 : 3,
+    if (per_signal) return {N <= 256 ? 0 : N == 4096 ? 2 : tiles_per_cu >= 20 ? 6 : 3,
                              Prefetch::kNone};
     if (N <= 256) return {tiles_per_cu >= 4 && tiles_per_cu < 16 ? 3 : 0, Prefetch::kNone};
     if (N == 512 || N == 4096) return {2, Prefetch::kEarly};
