@@ -35,7 +35,8 @@ inline constexpr int kConvMinWavesPerEU = N <= 2048 ? 3 : 1;
 // kDirect (per-signal filters, no prefetch): signal and filter load straight
 // into the first pass's registers and the output is stored from the last
 // pass's, with no LDS staging (DirectIO): 16384 x 2048 fp32 158 vs 164 us.
-template <class IO, int N, bool kPerSignal, Prefetch kPf = Prefetch::kNone, bool kDirect = false>
+// kThrough (not with kDirect): stores go through the L2 (StreamOut).
+template <class IO, int N, bool kPerSignal, Prefetch kPf, bool kDirect, bool kThrough>
 __global__ __launch_bounds__(256) __attribute__((
     amdgpu_waves_per_eu(kPf != Prefetch::kNone ? 2 : kConvMinWavesPerEU<N>))) void
 conv1d_kernel(const IO* __restrict__ x, const IO* __restrict__ h, IO* __restrict__ y, int batch,
@@ -132,8 +133,8 @@ conv1d_kernel(const IO* __restrict__ x, const IO* __restrict__ h, IO* __restrict
         fft_registers<N, false>(v, io.slot, io.t, w);
         if constexpr (kDirect)
             DirectIO<IO, N>(threadIdx.x).store(v, y, tile, batch);
-        else  // (float2 with per-signal filters, N = 64, 128: 2% slower written through)
-            io.template store<!(kPerSignal && std::is_same_v<IO, float2>)>(v, y, tile, batch);
+        else
+            io.template store<kThrough>(v, y, tile, batch);
     }
 }
 

@@ -179,14 +179,13 @@ __device__ __forceinline__ void st_nt(W* p, W w) {
 // C2C of 2^26 values 171.2 against 173.6 (N = 1024) and 174.8 against 177.0
 // (N = 128), 2^20 values at N = 128 ... 1024 4.3-5.5 against 4.8-5.9; around
 // 2^23 values, where the arrays just fit the memory-side cache, it is level to
-// 2% slower (N = 1024: 26.0 against 25.6 us).  For the VALU kernels that walk
-// their tiles it is level to 3% faster at 2^25 values and more (C2C N = 2048
-// 178.3 against 180.1, shared-filter conv1d N = 512 101.8 against 105.1, 1024
-// 99.6 against 101.3, 2048 and 4096 level), and from 6% faster to 4% slower at
-// 2^23 (conv1d N = 128 26.2 against 27.8, 2048 32.3 against 31.0); the half2
+// 2% slower (N = 1024: 26.0 against 25.6 us).  VALU kernels that walk their
+// tiles gain too (C2C N = 2048 178.3 against 180.1, shared-filter conv1d N =
+// 512 100.3 against 104.4 at 2^25 values), but not at every size; the half2
 // walks on the matrix cores and the real convolutions measured 1-6% slower
-// with it and do without.  Partial lines each cost a write to memory (an
-// unaligned half2 C2C: 12.1 against 6.5 us).
+// with it and do without.  Which calls use it, and what both forms take around
+// each line, stands at the launches (c2c_instance.hip).  Partial lines each
+// cost a write to memory (an unaligned half2 C2C: 12.1 against 6.5 us).
 template <bool kThrough>
 struct StreamOut {
     static constexpr int kPolicy = kThrough ? 18 : 2;  // nt, sc1

@@ -280,6 +280,35 @@ def test_conv1d_grids_for_few_tiles(n, tiles_per_cu):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("n,tiles", [(1024, 512), (1024, 1024), (2048, 512), (2048, "3 per CU"), (2048, 2048),
+                                     (4096, "3 per CU")])
+def test_conv1d_store_forms_at_their_lines(n, tiles):
+    """fp32, one filter for all, N >= 1024: stores go through the L2 or not by the
+    tiles of 4096 values; a whole number of them at each line, one signal less
+    (partial at N < 4096) and one more.  Every signal through the impulse roll, at the
+    tolerance of the grid-stride walks above, with sentinels on both sides."""
+    import torch
+
+    import thunderfft_amd as thff
+
+    if not isinstance(tiles, int):
+        tiles = 3 * torch.cuda.get_device_properties(0).multi_processor_count
+    thff.ThunderFFTInitialize("float", n)
+    whole = tiles * thff.transforms_per_block(n)
+    shift = 77
+    imp = torch.zeros(n, 2, device="cuda")
+    imp[shift, 0] = 1
+    for batch in (whole - 1, whole, whole + 1):
+        x = torch.empty(2 * n * batch, device="cuda")
+        thff.fill_uniform("float", x, n * batch, n + batch)
+        y, intact = tile_guarded_output(batch * n, "float")
+        thff.ThunderFFT_conv1d("float", n, x, imp, y, batch, False)
+        want = torch.roll(x.view(batch, n, 2), shift, dims=1)
+        got = y.view(batch, n, 2)
+        err = float(torch.linalg.vector_norm(got - want) / torch.linalg.vector_norm(want))
+        assert intact() and err <= TIGHT["float"] and float((got - want).abs().max()) <= 1e-5, (n, batch)
+
+
 @pytest.mark.parametrize("T", ["half", "float"])
 def test_conv1d_beyond_2e31_values(T):
     """The benchmarked conv1d's length (2048) over 2^31 + 3 * 2048 complex

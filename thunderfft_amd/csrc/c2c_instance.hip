@@ -333,18 +333,52 @@ constexpr ConvShape valu_conv_shape(int precision, bool real, bool per_signal,
     return {3, Prefetch::kNone};
 }
 
+// Whether a shared-filter fp32 conv1d of `tiles` tiles stores through the L2:
+// always up to N = 512 (2^14 values 6.08 us, without 6.45; 2^23 26.8, 28.0 at N =
+// 128; 2^25 100.3, 104.4 at 512). N = 1024 and 2048 do not just above 2^21 values,
+// where input and output are more than the L2s' 32 MiB together (N = 1024 up to
+// 2^22: 2194 signals 14.5, 13.9; 3565 18.6, 17.6; outside 2048 11.0, 11.3, 4705
+// 20.7, 21.5; N = 2048 while every tile runs at once, 3 per CU: 1260 16.6, 15.7;
+// outside 1024 13.1, 13.2, 1782 17.9, 18.7), nor N = 2048 from 2^23 values on
+// (5792 42.9, 41.9; 16384 107.7, 106.0), nor N = 4096 from 3 tiles per CU on (724
+// 17.2, 17.4; 1663 30.5, 29.4; 5792 84.7, 83.7).
+template <int N>
+bool shared_conv_through(long long tiles, int num_cus) {
+    constexpr long long kLine = (1LL << 21) / C2CPlan<N>::kTile;
+    if (N == 1024) return tiles <= kLine || tiles > 2 * kLine;
+    if (N == 2048) return tiles <= kLine || (tiles > 3LL * num_cus && tiles < 4 * kLine);
+    return N < 1024 || tiles < 3LL * num_cus;
+}
+
+// half2 (N = 64, 128) always stores through the L2; float2 with per-signal
+// filters never does (N = 64, 128: 2% slower).
 template <class IO, int N>
 void enqueue_conv1d(bool per_signal, Grid g, Prefetch pf, const IO* x, const IO* h, IO* y,
-                    int batch, const float2* tw, hipStream_t stream) {
-    if (per_signal)
-        conv1d_kernel<IO, N, true, Prefetch::kNone, (N >= 256)><<<g.blocks, 256, 0, stream>>>(
-            x, h, y, batch, tw, g.tiles_per_block);
-    else if (pf == Prefetch::kEarly)
-        conv1d_kernel<IO, N, false, Prefetch::kEarly><<<g.blocks, 256, 0, stream>>>(
-            x, h, y, batch, tw, g.tiles_per_block);
-    else
-        conv1d_kernel<IO, N, false><<<g.blocks, 256, 0, stream>>>(x, h, y, batch, tw,
-                                                                  g.tiles_per_block);
+                    int batch, const float2* tw, int num_cus, hipStream_t stream) {
+    constexpr bool kHalf = std::is_same_v<IO, __half2>;
+    const auto shared = [&](auto through) {
+        constexpr bool kThrough = decltype(through)::value;
+        if (pf == Prefetch::kEarly)
+            conv1d_kernel<IO, N, false, Prefetch::kEarly, false, kThrough>
+                <<<g.blocks, 256, 0, stream>>>(x, h, y, batch, tw, g.tiles_per_block);
+        else
+            conv1d_kernel<IO, N, false, Prefetch::kNone, false, kThrough>
+                <<<g.blocks, 256, 0, stream>>>(x, h, y, batch, tw, g.tiles_per_block);
+    };
+    if (per_signal) {
+        conv1d_kernel<IO, N, true, Prefetch::kNone, (N >= 256), kHalf>
+            <<<g.blocks, 256, 0, stream>>>(x, h, y, batch, tw, g.tiles_per_block);
+        return;
+    }
+    if constexpr (!kHalf && N >= 1024) {
+        const long long tiles =
+            (static_cast<long long>(batch) + C2CPlan<N>::kFPB - 1) / C2CPlan<N>::kFPB;
+        if (!shared_conv_through<N>(tiles, num_cus)) {
+            shared(std::false_type{});
+            return;
+        }
+    }
+    shared(std::true_type{});
 }
 
 template <int N>
@@ -399,11 +433,11 @@ hipError_t launch_conv1d(int precision, bool per_signal_filter, const void* x, c
     if (precision == 0)
         enqueue_conv1d<float2, N>(per_signal_filter, g, shape.prefetch,
                                   static_cast<const float2*>(x), static_cast<const float2*>(h),
-                                  static_cast<float2*>(y), batch, tw, stream);
+                                  static_cast<float2*>(y), batch, tw, num_cus, stream);
     else if constexpr (N < 256)  // fp16 N >= 256 returned above (MFMA)
         enqueue_conv1d<__half2, N>(per_signal_filter, g, Prefetch::kNone,
                                    static_cast<const __half2*>(x), static_cast<const __half2*>(h),
-                                   static_cast<__half2*>(y), batch, tw, stream);
+                                   static_cast<__half2*>(y), batch, tw, num_cus, stream);
     return hipGetLastError();
 }
 
