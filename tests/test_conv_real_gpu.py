@@ -235,11 +235,11 @@ def test_full_size_impulse_rolls(T, n, batch, channels):
         assert rel <= 1e-3 and err.max() <= 5e-3, label
 
 
-@pytest.mark.parametrize("n", [512, 1024, 2048])
+@pytest.mark.parametrize("n", [64, 128, 256, 512, 1024, 2048])
 def test_second_tile_for_some_workgroups(n):
-    """float, a grid of two workgroups per CU: one tile each (the spectrum in
-    flight during the forward transform), one tile more and one less than two
-    each (the spectrum after it), two each.  Channel d's filter is a unit
+    """float, a grid of two workgroups per CU, either side of the tiles where the
+    spectrum's loads move before or after the forward transform: one tile per CU,
+    one per workgroup, two and two and a half.  Channel d's filter is a unit
     impulse at tap (17 d + 1) mod N, so its output is its input rolled, to the
     rounding of the transforms (TIGHT)."""
     import torch
@@ -248,7 +248,7 @@ def test_second_tile_for_some_workgroups(n):
 
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     fpb = thff.transforms_per_block(n)
-    for tiles in (2 * cus, 2 * cus + 1, 4 * cus - 1, 4 * cus):
+    for tiles in (cus - 1, cus, 2 * cus, 2 * cus + 1, 4 * cus - 1, 4 * cus, 5 * cus - 1, 5 * cus):
         channels, batch = tiles, 2 * fpb  # tiles * fpb transforms of two rows
         taps = [(17 * d + 1) % n for d in range(channels)]
         h = np.zeros((channels, n), dtype=np.float32)

@@ -508,14 +508,22 @@ hipError_t launch_conv1d_real(int precision, const void* x, const float2* spectr
                                                static_cast<float*>(y), batch, channels, tw,
                                                g.tiles_per_block);
         };
-        // Where only some workgroups have a second tile, its spectrum is loaded
-        // after the forward transform (N = 2048, 50 channels: 57 rows 14.7
-        // against 15.7 us for the early load, 66 rows 15.7 against 16.6; N =
-        // 1024, 115 rows 13.5 against 13.8; N = 512, 231 rows 14.7 against
-        // 14.9); from two full rounds on early (N = 2048, 115 rows 24.1 against
-        // 25.2).
-        if constexpr (N >= 512 && N <= 2048) {
-            if (ntiles > g.blocks && ntiles < 2LL * g.blocks) {
+        // The channel's spectrum, early (in flight during the forward
+        // transform) or after it; 16 channels, tiles in rounds of 2 per CU:
+        //   N <= 256: after it while every workgroup has one tile (N = 128, 0.7
+        //     rounds 7.45 against 7.58 us, 1.0 8.02 against 8.14), early from the
+        //     second on (1.1 rounds 11.4 against 12.2, 4.0 28.5 against 29.2);
+        //   above: early while a CU has one tile (0.25 rounds, N = 512 7.82 against
+        //     7.88, 2048 7.88 against 7.96) and from 2 rounds on (2.2, N = 512 21.6
+        //     against 22.8; 4.0, N = 1024 32.3 against 34.0), N = 2048 from 2.5 (2.2
+        //     rounds 22.0 late, 22.3 early; 2.8 26.2, 25.7), after it between
+        //     (0.7 rounds, N = 512 9.98 against 10.16, 1024 9.51 against 9.73).
+        if constexpr (N <= 2048) {
+            const long long round = 2LL * num_cus;
+            const bool early = N <= 256 ? ntiles > round
+                                        : 2 * ntiles < round ||
+                                              2 * ntiles >= (N == 2048 ? 5 : 4) * round;
+            if (!early) {
                 launch(std::false_type{});
                 return hipGetLastError();
             }
