@@ -351,10 +351,11 @@ def test_grid_stride_walks(T, n):
     _large_case(T, n, 514 * tile + max(1, tile // 2), directions=(True,))
 
 
-@pytest.mark.parametrize("T,n,tiles_per_cu", [("float", n, t) for n in (2048, 4096) for t in (5, 16)]
+@pytest.mark.parametrize("T,n,tiles_per_cu", [("float", n, t) for n in (2048, 4096) for t in (5, 8, 16)]
                          + [("half", n, t) for n in (128, 2048, 4096) for t in (5, 10)])
 def test_grids_for_few_tiles(T, n, tiles_per_cu):
-    """fp32 N >= 2048 takes 2, 4 or 16 workgroups per CU by the tiles per CU,
+    """fp32 N >= 2048 takes 2, 4 or 16 workgroups per CU by the tiles per CU (lines at
+    5 and 8 or 16),
     fp16 N = 128, 2048 and 4096 2 or 3: either side of both lines, a whole
     number of tiles and one partial tile more."""
     import torch

@@ -186,8 +186,8 @@ void enqueue_mfma3(Grid g, const __half2* x, __half2* y, int batch, hipStream_t 
 //     3.54, 3.64; 16 signals 3.41, 2.85 and 3.28, 2.80);
 //   N = 128 from 2^19 values (fp32: 2048 signals 4.34, 4.10, 4096 4.64, 4.64,
 //     8192 5.52, 5.77; half2: 4.08, 3.90, 4.18, 4.18, 4.48, 4.85);
-//   the rest from 2^21 values (fp32 N = 1024, 2895 signals: 9.7, 12.1; half2
-//     N = 256, 16383: 8.1, 11.1).
+//   the rest above 2^21 values (fp32 N = 1024, 2895 signals: 9.7, 12.1; 2048
+//     7.90, 7.57; half2 N = 256, 16383: 8.1, 11.1; 8192 5.96, 5.73).
 template <class IO, int N, bool kDirect>
 void enqueue_unaligned(bool forward, const IO* x, IO* y, int batch, const float2* tw,
                        hipStream_t stream) {
@@ -204,7 +204,7 @@ template <class IO, int N>
 void enqueue_unaligned(bool forward, const IO* x, IO* y, int batch, const float2* tw,
                        hipStream_t stream) {
     if constexpr (std::is_same_v<IO, float2> || N <= 256) {
-        constexpr long long kStaged = N == 64 ? C2CPlan<N>::kTile : N == 128 ? 1LL << 19 : 1LL << 21;
+        constexpr long long kStaged = N == 64 ? C2CPlan<N>::kTile : N == 128 ? 1LL << 19 : (1LL << 21) + 1;
         if (static_cast<long long>(batch) * N >= kStaged) {
             enqueue_unaligned<IO, N, false>(forward, x, y, batch, tw, stream);
             return;
@@ -232,16 +232,17 @@ hipError_t launch_c2c(int precision, bool forward, bool aligned16, const void* i
     const long long ntiles = (static_cast<long long>(batch) + fpb - 1) / fpb;
     int per_cu = launch_shape<N>(precision).per_cu;
     if (precision == 0 && N >= 2048) {
-        // Beyond 16 tiles per CU the 16 per CU of launch_shape; below, fewer
-        // workgroups that each prefetch what 16 per CU would start afresh:
-        // up to 5 tiles per CU 2 (N = 2048: 1448 signals 10.0 against 12.2
-        // us, 2048 13.2 against 15.6; N = 4096: 1024 signals 14.4 against
-        // 16.6), then 4 (N = 2048: 4096 signals 26.5 against 27.5; N = 4096:
-        // 2048 27.4 against 29.3, 3821 47.1 against 48.5; at 2^26 values
-        // 4 per CU takes 183-185 us, 16 per CU 179-181).
+        // Many tiles: the 16 per CU of launch_shape; below, fewer workgroups
+        // that each prefetch what 16 per CU would start afresh: up to 5 tiles
+        // per CU 2 (N = 2048: 1448 signals 10.0 against 12.2 us, 2048 13.2
+        // against 15.6; N = 4096: 1024 signals 14.4 against 16.6), then 4, N =
+        // 2048 up to 8 (4096 signals 26.5 against 27.5; beyond, a third and
+        // fourth round are uneven: 5042 33.8, 32.1; 6653 43.6, 40.7), N = 4096
+        // up to 16 (2048 27.4, 29.3; 3821 47.1, 48.5; at 2^26 values 4 per CU
+        // takes 183-185 us, 16 per CU 179-181).
         if (ntiles <= 5LL * num_cus)
             per_cu = 2;
-        else if (ntiles <= 16LL * num_cus)
+        else if (ntiles <= (N == 2048 ? 8LL : 16LL) * num_cus)
             per_cu = 4;
     }
     // The half2 walks take a third workgroup per CU between 5 and 10 tiles per
