@@ -594,12 +594,14 @@ __device__ __forceinline__ void mfma_fft_regs(unsigned* region, const float2* __
 // accurate to far below the f16 rounding the data takes), so nothing but the
 // data touches memory.  The twiddle before the last DFT16 stays an fp32
 // multiply: folded into LDS-held operands (as the convolutions do) it measured
-// slower for the transform alone (compute pass 29.8 vs 27.8 us at N = 1024).  The wave's loads are issued before the coefficients are
-// computed.  Grid: one 256-lane workgroup per four tiles.
-template <int C, bool FWD, int kWaves = 4>
-__global__ __launch_bounds__(64 * kWaves) void c2c_mfma_wave_kernel(const __half2* __restrict__ in,
-                                                                    __half2* __restrict__ out,
-                                                                    int batch) {
+// slower for the transform alone (compute pass 29.8 vs 27.8 us at N = 1024).
+// The wave's loads are issued before the coefficients are computed.  Grid: one
+// workgroup of kWaves waves per kWaves tiles.  kPerSimd: at most that many waves
+// per SIMD (0: what the registers allow, 8 at N = 256, else 6).
+template <int C, bool FWD, int kWaves, int kPerSimd>
+__global__ __launch_bounds__(64 * kWaves)
+    __attribute__((amdgpu_waves_per_eu(kPerSimd ? kPerSimd : 1, kPerSimd ? kPerSimd : 8))) void
+c2c_mfma_wave_kernel(const __half2* __restrict__ in, __half2* __restrict__ out, int batch) {
     using P = MfmaPlan<C>;
     constexpr int N = P::N;
     constexpr int kB = P::kBlocks;

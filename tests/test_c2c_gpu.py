@@ -351,6 +351,18 @@ def test_grid_stride_walks(T, n):
     _large_case(T, n, 514 * tile + max(1, tile // 2), directions=(True,))
 
 
+@pytest.mark.parametrize("n", [256, 512, 1024])
+def test_half_waves_per_simd(n):
+    """fp16 N = 256 ... 1024 runs 4 waves per SIMD from more than 6 tiles of 1024
+    values per SIMD on: a whole number of tiles on the line, one signal less and
+    one more."""
+    import torch
+
+    line = 24 * torch.cuda.get_device_properties(0).multi_processor_count * (1024 // n)
+    for batch in (line - 1, line, line + 1):
+        _large_case("half", n, batch)
+
+
 @pytest.mark.parametrize("T,n,tiles_per_cu", [("float", n, t) for n in (2048, 4096) for t in (5, 8, 16)]
                          + [("half", n, t) for n in (128, 2048, 4096) for t in (5, 10)])
 def test_grids_for_few_tiles(T, n, tiles_per_cu):

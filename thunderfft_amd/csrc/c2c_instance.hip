@@ -145,16 +145,26 @@ void enqueue(Grid g, const IO* x, IO* y, int batch, const float2* tw, int num_cu
 // of 1 or 2 such waves: 86.4-87.0 and 87.1-87.2 us at N = 1024, slower at 256
 // and 512.  One tile per workgroup for the three-stage kernels (N = 2048,
 // 4096) takes 118 and 96.6 us against 91.2 and 88.9 us for the walk.
+// Waves per SIMD: more than fit at once, 6, and HBM serves fewer of them
+// faster, the more so the shorter a wave's computing is (us at 4 per SIMD and
+// uncapped, means over 8 layouts of three pairs of buffers: N = 256 16.1, 19.7
+// for 40342 signals, 34.2, 43.8 for 99334, 83.5, 95.1 for 262144; N = 1024 35.1,
+// 41.7 for 24833, 83.8, 89.4 for 65536; 3 per SIMD 86.1 and 84.9 for 2^26 values);
+// below that one round of all the waves is ahead (N = 256 9.1 against 9.9 for
+// 21618; N = 512 9.3 against 10.7 for 10809).
 inline constexpr int kHalfOneShotWaves = 4;  // waves (tiles) per workgroup
 
 template <int N, bool FWD>
-void enqueue_mfma(const __half2* x, __half2* y, int batch, hipStream_t stream) {
-    constexpr int kW = kHalfOneShotWaves;
-    constexpr long long kPerBlock = static_cast<long long>(kW) * MfmaPlan<N / 256>::kFPW;
+void enqueue_mfma(const __half2* x, __half2* y, int batch, int num_cus, hipStream_t stream) {
+    constexpr int kW = kHalfOneShotWaves, C = N / 256;
+    constexpr long long kPerBlock = static_cast<long long>(kW) * MfmaPlan<C>::kFPW;
     const long long blocks = (static_cast<long long>(batch) + kPerBlock - 1) / kPerBlock;
     if (blocks <= 0) return;
-    c2c_mfma_wave_kernel<N / 256, FWD, kW><<<static_cast<unsigned>(blocks), 64 * kW, 0, stream>>>(
-        x, y, batch);
+    const unsigned grid = static_cast<unsigned>(blocks);
+    if (blocks * kW > 4 * 6LL * num_cus)
+        c2c_mfma_wave_kernel<C, FWD, kW, 4><<<grid, 64 * kW, 0, stream>>>(x, y, batch);
+    else
+        c2c_mfma_wave_kernel<C, FWD, kW, 0><<<grid, 64 * kW, 0, stream>>>(x, y, batch);
 }
 
 template <bool FWD>
@@ -266,9 +276,9 @@ hipError_t launch_c2c(int precision, bool forward, bool aligned16, const void* i
         auto* y = static_cast<__half2*>(out);
         if constexpr (kHalfOnMfma<N>) {
             if (forward)
-                enqueue_mfma<N, true>(x, y, batch, stream);
+                enqueue_mfma<N, true>(x, y, batch, num_cus, stream);
             else
-                enqueue_mfma<N, false>(x, y, batch, stream);
+                enqueue_mfma<N, false>(x, y, batch, num_cus, stream);
         } else if constexpr (kHalfOnMfma3<N>) {
             if (forward)
                 enqueue_mfma3<N, true>(g, x, y, batch, stream);
