@@ -26,8 +26,8 @@
 // filter's two passes in launches of their own:
 //   float2: 32 images 278 us against 362, 9 images 89 against 136, 1 image 29
 //     (24 on the GPU) against 49
-//   half2:  32 images 182 us against 215 (a column pass on MFMA), 8 images 60
-//     against 84, 1 image 26 to 29 against 41; rel L2 3.6e-4 against 5.3e-4
+//   half2:  32 images 182 us against 215 (a column pass on MFMA), 8 images 57
+//     against 84, 1 image 25 to 29 against 41; rel L2 3.6e-4 against 5.3e-4
 //     (7.0e-4 from 8 images on): the values are rounded when stored, not
 //     between the stages of a transform
 // Tried: groups of 4 (8) rows stored column by column instead of the radix
