@@ -814,7 +814,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBPS, 4),
                      "traffic": load_traffic("float_fwd"),
-                     "kernel": "thff::c2c_kernel<float2, 1024, true, false, false>",
+                     "kernel": "thff::c2c_kernel<float2, 1024, true, false, false, true>",
                      "algorithmic_bytes": main_run["bytes_per_call"],
                      "traffic_profile": "profiles/pmc_c2c_n1024_b65536.md"},
         # traffic and mfma_util_pct are read from the rocprofv3 summaries in
